@@ -218,3 +218,59 @@ def tolerance(case):
     # against float64: at most 7e-7 for fp32 results (contractions up to 12288), 1.7e-3 for ones rounded to bf16; four times that
     fp32_out = case["kind"] == "gemm" and case["out"] == "fp32" or case["kind"] == "device" and (case["dtype"] == "fp32" or (case["flow"] != "os"))
     return {"rel": 3e-6 if fp32_out else 7e-3}
+
+
+def _cut(t, S, axis):
+    """The S block-cyclic slices of a matrix: slice s holds its blocks b with b % S == s"""
+    shape = t.shape
+    if axis == 1:
+        return [s.reshape(shape[0], -1) for s in t.reshape(shape[0], -1, S, BLOCK).unbind(2)]
+    return [s.reshape(-1, shape[1]) for s in t.reshape(-1, S, BLOCK, shape[1]).unbind(1)]
+
+
+def _exact_device(case, x, w):
+    """The last device's output block, or its partial chunks, in the order that its algorithm hands them out"""
+    flow, R, C, S = (case[v] for v in ("flow", "rows", "cols", "S"))
+    m, n, k = case["m"], case["n"], case["k"]
+    i, j = R - 1, C - 1
+    x, w = x.double(), w.double()
+    if flow == "os":
+        return x[i * (m // R):] @ w[:, j * (n // C):]
+    if flow == "ls":
+        own, axis, peers = x[i * (m // R):, j * (k // C):], 0, w[:, j * (k // C):].chunk(R, 0)
+    else:
+        own, axis, peers = w[i * (k // R):, j * (n // C):], 1, x[i * (k // R):].chunk(C, 1)
+    parts = [_cut(p, S, axis) for p in peers] if case["algorithm"] == "meshflow" else [[p] for p in peers]
+    gathered = [torch.cat([p[s] for p in parts], axis) for s in range(len(parts[0]))]
+    return [own @ g.t() if flow == "ls" else g.t() @ own for g in gathered]
+
+
+def exact(case, seed):
+    st = prepare(case, seed)
+    if case["kind"] == "gemm":
+        if case["flow"] == "os":
+            c = sum(a.double() @ b.double() for a, b in zip(st["a"], st["b"]))
+            if case["gelu"]:
+                c = torch.nn.functional.gelu(c, approximate="tanh")
+            return c if st["res"] is None else c + st["res"].double()
+        if case["flow"] == "ls":
+            a = st["a"].double()
+            return [a @ w.double().t() for w in st["b"]]
+        b = st["b"].double()
+        return [x.double().t() @ b for x in st["a"]]
+    if case["kind"] == "device":
+        return _exact_device(case, st["x"], st["w"])
+    if case["kind"] == "layer":
+        x, w, dy = st["x"].detach().double(), st["layer"].weight.detach().double(), st["dy"].double()
+        if case["flow"] == "os":
+            return x @ w, dy @ w.t(), x.t() @ dy
+        if case["flow"] == "ls":
+            return x @ w.t(), dy @ w, dy.t() @ x
+        return x.t() @ w, w @ dy.t(), x @ dy
+    S, axis, peers = (case[v] for v in ("S", "axis", "peers"))
+    mine = [sum(c[s].double().chunk(peers, axis)[peers - 1] for c in st["chunks"]) for s in range(S)]
+    if axis == 1:
+        shard = torch.stack([c.reshape(c.shape[0], -1, BLOCK) for c in mine], 2).reshape(case["rows"], -1)
+    else:
+        shard = torch.stack([c.reshape(-1, BLOCK, c.shape[1]) for c in mine], 1).reshape(-1, case["cols"])
+    return [s.double() for s in _cut(st["x"], S, axis)], shard
