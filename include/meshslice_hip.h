@@ -55,7 +55,7 @@ extern "C" {
                                    would leave much of the last round of compute units idle is done in two launches) */
 #define MS_QUERY_LAST_SPLITS 7   /* ways in which that launch split the contraction (1: not split) */
 #define MS_QUERY_LAST_VARIANT 6  /* kernel variant (tile shape, see ms_set_variant) of the first of those launches: 1..14 for
-                                   the bf16 kernels, 21..25 for the fp32 kernel.  Lets a measurement name the kernel it timed. */
+                                   the bf16 kernels, 21..27 for the fp32 kernel.  Lets a measurement name the kernel it timed. */
 #define MS_QUERY_LAST_GRID 8     /* workgroups of the first of those launches: the compute units it ran on (at most the
                                    device's, less the reserved ones; fewer when that fills every round of the launch) */
 

@@ -72,6 +72,8 @@ MS_INSTANTIATE_F32(4, 2, 1, 3)
 MS_INSTANTIATE_F32(2, 2, 2, 2)
 MS_INSTANTIATE_F32(2, 2, 1, 1)
 MS_INSTANTIATE_F32(2, 2, 3, 3)
+MS_INSTANTIATE_F32(2, 2, 1, 3)
+MS_INSTANTIATE_F32(2, 2, 1, 2)
 #undef MS_INSTANTIATE_F32
 
 namespace {
@@ -317,6 +319,7 @@ struct Pick { int v, splits; double cost; };
 
 constexpr int VARIANTS = 14;
 constexpr int F32_FIRST = 21, F32_LAST = 25;      // ids of the fp32 kernel's tiles (ms_set_variant, MS_QUERY_LAST_VARIANT)
+constexpr int F32_NARROW = 26;                    // and of the two that only the chooser takes (64 x 192, 64 x 128)
 struct TileShape { int bm, bn; };
 constexpr TileShape TILE_OF[VARIANTS + 1] = {{0, 0},     {256, 256}, {256, 256}, {128, 128}, {256, 256}, {256, 192},
                                              {192, 256}, {256, 256}, {256, 192}, {192, 256}, {256, 384}, {384, 192},
@@ -476,8 +479,9 @@ int launch_bf16(const Problem &p, const DevFacts &dev, hipStream_t stream) {
   return launch_variant(single.v, single.splits, p, dev, stream);
 }
 
-// fp32 operands: gemm_f32_tile_kernel on one of its five tiles (ids F32_FIRST ..: 256 x 128 and 128 x 192 on eight
-// waves, 128 x 128, 64 x 64 and 192 x 192 on four); `share`: two workgroups of the 128 x 128 or 64 x 64 tile per compute unit
+// fp32 operands: gemm_f32_tile_kernel on one of its seven tiles (ids F32_FIRST ..: 256 x 128 and 128 x 192 on eight
+// waves, 128 x 128, 64 x 64 and 192 x 192 on four; F32_NARROW ..: 64 x 192 and 64 x 128 on four); `share`: two workgroups
+// of the 128 x 128 tile or of one of the 64-row tiles per compute unit
 int f32_split_refused(const Problem &p, const DevFacts &dev, int bm, int bn, int splits);
 
 template <int WGM, int WGN, int TM, int TN>
@@ -551,10 +555,16 @@ int f32_split_refused(const Problem &p, const DevFacts &dev, int bm, int bn, int
 // shared 133 us, alone in two rounds 150 us; 1024 tiles of 128 x 128 shared 957 us; one round of 256 tiles of 192 x 192,
 // four waves of 3 x 3 tiles each, 567 us).  Unlike the bf16 kernels this one
 // does not sit on the power limit: a partly filled round costs a whole one.
+// The two 64-row tiles with more columns than rows are for outputs whose rows fill a 128-row tile badly, and for the step
+// from one round to two between 64 x 64 and 128 x 128 (256 tiles on 2048 contraction elements: 64 x 192 105 us, two per unit
+// 192 us a pair; 64 x 128 73 and 129 us).  Four chunks of 260 x 2056 on 1023 elements: 220 tiles of 64 x 192 in 55 us, 204 of
+// 128 x 128 or 660 of 64 x 64 in 63; three of 500 x 1500 on 1500: 80 against 92 us; 700 x 900 x 4000 in four parts: 61
+// against 71 us; 2048^3 on 512 tiles of 64 x 128: 129 against 134 us.
 struct F32Tile { int id, bm, bn; bool pairs; double cost, shared; };      // pairs: two such workgroups fit a compute unit
 constexpr F32Tile F32_TILES[] = {{F32_FIRST, 256, 128, false, 1.0, 0.0}, {F32_FIRST + 1, 128, 192, false, 1.0 / 0.967, 0.0},
                                  {F32_FIRST + 2, 128, 128, true, 1.0 / 0.918, 1.88}, {F32_FIRST + 3, 64, 64, true, 1.0 / 0.78, 1.78},
-                                 {F32_FIRST + 4, 192, 192, false, 1.0 / 0.93, 0.0}};
+                                 {F32_FIRST + 4, 192, 192, false, 1.0 / 0.93, 0.0},
+                                 {F32_NARROW, 64, 192, true, 1.0 / 0.87, 1.85}, {F32_NARROW + 1, 64, 128, true, 1.0 / 0.85, 1.82}};
 
 int launch_f32_id(int id, bool share, int splits, const Problem &p, const DevFacts &dev, hipStream_t stream) {
   switch (id) {
@@ -562,6 +572,8 @@ int launch_f32_id(int id, bool share, int splits, const Problem &p, const DevFac
     case F32_FIRST + 1: return launch_f32_tile<4, 2, 1, 3>(p, dev, stream, id, false, splits);
     case F32_FIRST + 2: return launch_f32_tile<2, 2, 2, 2>(p, dev, stream, id, share, splits);
     case F32_FIRST + 3: return launch_f32_tile<2, 2, 1, 1>(p, dev, stream, id, share, splits);
+    case F32_NARROW: return launch_f32_tile<2, 2, 1, 3>(p, dev, stream, id, share, splits);
+    case F32_NARROW + 1: return launch_f32_tile<2, 2, 1, 2>(p, dev, stream, id, share, splits);
     default: return launch_f32_tile<2, 2, 3, 3>(p, dev, stream, id, false, splits);
   }
 }

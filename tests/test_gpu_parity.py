@@ -199,6 +199,15 @@ def test_fp32_random_cases_on_every_tile(flow, tile):
         assert lib.ms_query(_lib.MS_QUERY_LAST_VARIANT) == tile
 
 
+@pytest.mark.parametrize("tile,flow,m,n,k,S", [(26, "rs", 260, 2056, 1023, 4), (26, "os", 700, 900, 1332, 3), (26, "rs", 500, 1500, 36, 3),
+                                               (27, "ls", 1500, 520, 132, 4), (27, "os", 2047, 2044, 100, 1), (27, "rs", 508, 2044, 65, 4)])
+def test_fp32_narrow_tiles_where_the_chooser_takes_them(tile, flow, m, n, k, S):
+    """64x192 (id 26) and 64x128 (id 27): rows and columns that end inside a tile, K tails; fp32 results to 1e-5, like every fp32 tile."""
+    ops = _rand_case(flow, m, n, k, S, seed=tile + m, dtype=torch.float32)
+    _run_and_compare(flow, ops, torch.float32, TOL_F32)
+    assert _lib.load().ms_query(_lib.MS_QUERY_LAST_VARIANT) == tile
+
+
 @pytest.mark.parametrize("flow", ["os", "ls", "rs"])
 def test_fp32_long_all_positive_contraction_is_summed_in_blocks(flow):
     """16384 all-positive terms per output: one fp32 accumulator through the whole contraction drifts to about 2e-6 of
