@@ -339,3 +339,24 @@ def test_both_shipped_compute_terms_lead_to_the_same_slice_counts():
                 assert t[k] <= 1.005 * min(t.values()), (mesh, layer, kind, k, t)
         same += picks["normal", mesh] == picks["ones", mesh]
     assert same >= 2      # (at the time of writing the 8x8 mesh's two feed-forward layers pick 4 against 3: 14.412 against 14.419 ms)
+
+
+def test_neighbouring_shards_are_gathered_as_one_view():
+    """_spanning: the shards of a matrix in axis order are one view; anything else is gathered peer by peer."""
+    G = torch.arange(12 * 40.0).reshape(12, 40)
+    big = torch.arange(20 * 64.0).reshape(20, 64)[3:15, 5:45]       # a window of a larger matrix, at an odd offset
+    for M in (G, big):
+        grid = TP._shards(M, 3, 5)
+        for i in range(3):
+            assert torch.equal(TP._spanning(grid[i], 1), torch.cat(grid[i], 1))
+        for j in range(5):
+            column = [grid[i][j] for i in range(3)]
+            assert torch.equal(TP._spanning(column, 0), torch.cat(column, 0))
+            assert TP._spanning(column, 0).data_ptr() == column[0].data_ptr()
+        assert TP._spanning([grid[0][1], grid[0][0]], 1) is None and TP._spanning([grid[0][0], grid[0][2]], 1) is None
+        assert TP._spanning([grid[0][0], grid[0][1].clone()], 1) is None and TP._spanning([grid[0][0], grid[0][0]], 0) is None
+        assert TP._spanning([grid[0][4], M[0:4, 0:8]], 1) is None                # the next row's columns are not neighbours
+        assert TP._spanning([grid[0][0].t(), grid[0][1].t()], 0) is None
+    assert TP._spanning([G[:4, :32], G[:4, 32:40]], 1) is None and torch.equal(TP._spanning([G[:4]], 0), G[:4])
+    tall = torch.zeros(1, 8).expand(TP.PANEL_MAX_ROWS + 8, 8)
+    assert TP._spanning([tall], 1) is None                                      # more rows than one launch takes
