@@ -175,6 +175,17 @@ int ms_gemm_rs_ex(const void *const *X_slices, int ldx, const void *W, int ldw, 
                   int m_slice, int n, int k,
                   void *const *Y_chunks, int ldy, int in_dtype, int out_dtype, void *stream);
 
+/* ms_gemm_ls_ex / ms_gemm_rs_ex for P mesh devices of equal shapes in one launch (the devices of a mesh row, LS, or of a mesh
+ * column, RS, whose partial chunks one reduce-scatter adds up): A (LS) / W (RS) holds the P devices' own shards, the slice
+ * and chunk tables hold P * S <= MS_MAX_SLICES entries, device-major: Y[p*S+s] = A[p] @ W[p*S+s]^T, or X[p*S+s]^T @ W[p].
+ * All entries of a table share one leading dimension. */
+int ms_gemm_ls_peers(const void *const *A, int lda, const void *const *W_slices, int ldw, int P, int S,
+                     int m, int n_slice, int k,
+                     void *const *Y_chunks, int ldy, int in_dtype, int out_dtype, void *stream);
+int ms_gemm_rs_peers(const void *const *X_slices, int ldx, const void *const *W, int ldw, int P, int S,
+                     int m_slice, int n, int k,
+                     void *const *Y_chunks, int ldy, int in_dtype, int out_dtype, void *stream);
+
 /* ms_gemm_ls_ex / ms_gemm_rs_ex with completion counters, so that the reduce-scatter of chunk s (the psum_scatter that
  * follows each einsum in MeshFlow_LS / MeshFlow_RS, TensorParallel.py:182-189, :204-212) can start while the later
  * chunks are still being computed.  chunk_done points to S unsigned counters in device memory, zero before the call;

@@ -6,7 +6,8 @@ bodies ``MeshFlow_OS/LS/RS`` (:153-214) and the builder ``SPMD`` (:346-377).  Di
 by having one GPU and no tracing compiler:
 
 * the callable returned by ``OS/LS/RS`` takes the GLOBAL operands (torch tensors on the GPU), logically
-  sharded ``P(row, col)``, and returns the GLOBAL result; it runs every mesh device's body in turn;
+  sharded ``P(row, col)``, and returns the GLOBAL result; the devices' gathers, products and reduce-scatters run in
+  one launch each where the shapes allow it (_fits_whole_mesh), else it runs every mesh device's body in turn;
 * ``.device(i, j)`` runs ONE device's body and returns what that device produces before any
   cross-device reduction: its output block (OS) or its S fp32 partial chunks (LS / RS);
 * all_gather / psum_scatter move data between the emulated devices' buffers on the one GPU: the
@@ -381,6 +382,63 @@ def _finish(chunks_by_peer, me, axis, B, dtype):
     return slice_layout.unpack_chunks([[t] for t in partial], _block(width, 8), axis, window=0, parts=1, out_dtype=dtype)
 
 
+# ------------------------------------------------------------------------------------------------
+# the whole mesh at once.  On the one GPU that plays every device, the devices of a mesh row or column receive the same
+# gathered slices, and their products differ only in which rows and columns of them they take: one kernel gathers an operand
+# for all of them (see _spanning), one product covers them all.  Device by device a training step of a small layer is some
+# 150 launches of 2 to 40 us, bound by the host that issues them: 512 x 256 x 1024 on a 4x2 mesh 3.6 ms, in this way 0.48;
+# 2048 x 3072 x 12288 on a 2x4 mesh 5.1 ms, in this way 0.62.
+# ------------------------------------------------------------------------------------------------
+
+WHOLE_MESH_MAX_CHUNK_BYTES = 4 << 30      # partial chunks alive at once; device by device it is one mesh line's
+
+
+def _fits_whole_mesh(dataflow, X, W, R, C, K) -> bool:
+    """Whether the mesh's products can run as one: every device's own extents are ones that the kernels take (a mesh whose
+    devices would be refused is refused), no operand reaches the 2 GiB that a kernel addresses, the line's chunks fit one
+    pointer table (64) and a bounded buffer, and rows fit one launch of the layout kernels."""
+    q = 16 // X.element_size()
+    if X.device != W.device or X.dtype not in (torch.float32, torch.bfloat16) or X.stride(1) != 1 or W.stride(1) != 1:
+        return False
+    if max(X.shape[0], W.shape[0]) > PANEL_MAX_ROWS or min(X.numel(), W.numel()) == 0:
+        return False
+    if any(t.shape[0] * max(t.stride(0), t.shape[1]) * t.element_size() >= 1 << 31 for t in (X, W)):
+        return False
+    if dataflow == "os":
+        return (W.shape[1] // C) % q == 0 and (X.shape[1] // K) % q == 0 and K <= 64
+    if dataflow == "ls":
+        peers, m, n, aligned = C, X.shape[0], W.shape[0], (X.shape[1] // C, W.shape[0] // K, W.shape[0] // C)
+    else:
+        peers, m, n, aligned = R, X.shape[1], W.shape[1], (W.shape[1] // C, X.shape[1] // K, W.shape[1])
+    return peers * K <= 64 and peers * m * n * 4 <= WHOLE_MESH_MAX_CHUNK_BYTES and m <= PANEL_MAX_ROWS and not any(v % q for v in aligned)
+
+
+def _whole_ls(X, W, C, K, B, sliced):
+    """Every device's partial chunks in one launch and their reduce-scatters in another: mesh column j multiplies its columns
+    of X (the rows of all mesh rows together) with its columns of the gathered slices of W; the sum over j is fp32 in peer
+    order, as in _finish, and the windows of all devices together are the whole chunks."""
+    slices = slice_layout.pack_slices(W, K, B, 0) if sliced else [_gather([W], 0)]
+    w = X.shape[1] // C
+    A = _usable([X[:, j * w:(j + 1) * w] for j in range(C)])
+    chunks = local_gemm.gemm_ls_peers(A, [[t[:, j * w:(j + 1) * w] for t in slices] for j in range(C)])
+    return slice_layout.unpack_chunks(chunks, B if sliced else _block(W.shape[0], 8), 1, out_dtype=X.dtype)
+
+
+def _whole_rs(X, W, R, K, B, sliced):
+    """The same for the right-hand-stationary dataflow: mesh row i multiplies its rows of the gathered slices of X with its
+    rows of W."""
+    slices = slice_layout.pack_slices(X, K, B, 1) if sliced else [_gather([X], 1)]
+    h = X.shape[0] // R
+    own = _usable([W[i * h:(i + 1) * h] for i in range(R)])
+    chunks = local_gemm.gemm_rs_peers([[t[i * h:(i + 1) * h] for t in slices] for i in range(R)], own)
+    return slice_layout.unpack_chunks(chunks, B if sliced else _block(X.shape[1], 8), 0, out_dtype=X.dtype)
+
+
+# (the bodies launched ahead of their gathers keep a product per device where that produces chunks; the ring bodies' slices
+# are half-blocks in an order of each device's own)
+_WHOLE_MESH_BODIES = {"os": (Collective_OS, MeshFlow_OS, MeshFlow_OS_overlap), "ls": (Collective_LS, MeshFlow_LS), "rs": (Collective_RS, MeshFlow_RS)}
+
+
 class ShardedMatmul:
     """What ``SPMD.OS/LS/RS(K)`` returns: ``f(X, W) -> Y`` on global operands, plus ``f.device(i, j)``."""
 
@@ -434,6 +492,10 @@ class ShardedMatmul:
         R, C = self.R, self.C
         K = self.K if self.sliced else 1
         B = self.B if self.sliced else 1
+        if self.body in _WHOLE_MESH_BODIES[self.dataflow] and _fits_whole_mesh(self.dataflow, X, W, R, C, K):
+            if self.dataflow == "os":      # (the output blocks of all devices are one product: the body on a mesh of one)
+                return self.body([[X]], [[W]], 0, 0, 1, 1, self.K, self.B)
+            return _whole_ls(X, W, C, K, B, self.sliced) if self.dataflow == "ls" else _whole_rs(X, W, R, K, B, self.sliced)
         Xs, Ws = _shards(X, R, C), _shards(W, R, C)
         run = lambda i, j: self.body(Xs, Ws, i, j, R, C, self.K, self.B)
         if self.dataflow == "os":

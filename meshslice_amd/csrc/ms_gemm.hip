@@ -245,8 +245,8 @@ int launch_bf16_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, 
   for (int i = 0; i < p.nc; i++) g.c[i] = p.c[i];
   g.nchunks = p.flow == OS ? 1 : p.S;
   g.nkslices = p.flow == OS ? p.S : 1;
-  g.a_by_chunk = p.flow == RS;
-  g.b_by_chunk = p.flow == LS;
+  g.a_by_chunk = p.flow == RS || (p.flow == LS && p.na > 1);      // (several devices' products: a pointer for every chunk)
+  g.b_by_chunk = p.flow == LS || (p.flow == RS && p.nb > 1);
   g.M = p.M; g.N = p.N; g.K = p.K;
   g.lda = p.lda; g.ldb = p.ldb; g.ldc = p.ldc;
   g.tiles_m = (p.M + BM - 1) / BM;
@@ -494,8 +494,8 @@ int launch_f32_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, i
   for (int i = 0; i < p.nc; i++) g.c[i] = p.c[i];
   g.nchunks = p.flow == OS ? 1 : p.S;
   g.nkslices = p.flow == OS ? p.S : 1;
-  g.a_by_chunk = p.flow == RS;
-  g.b_by_chunk = p.flow == LS;
+  g.a_by_chunk = p.flow == RS || (p.flow == LS && p.na > 1);      // (several devices' products: a pointer for every chunk)
+  g.b_by_chunk = p.flow == LS || (p.flow == RS && p.nb > 1);
   g.M = p.M; g.N = p.N; g.K = p.K;
   g.lda = p.lda; g.ldb = p.ldb; g.ldc = p.ldc;
   g.tiles_m = (p.M + BM - 1) / BM;
@@ -931,6 +931,32 @@ MS_API int ms_gemm_rs_ex(const void *const *X_slices, int ldx, const void *W, in
                          void *const *Y_chunks, int ldy, int in_dtype, int out_dtype, void *stream) {
   const void *w1[1] = {W};
   return run(make_rs(X_slices, ldx, w1, ldw, S, m_slice, n, k, Y_chunks, ldy, in_dtype, out_dtype), stream);
+}
+
+// The chunk-producing products of several mesh devices in one launch: device p's S chunks are chunks p * S .. of one call
+// whose stationary operand has an entry for every chunk.  The devices of a mesh line have equal shapes, and one of them alone
+// often leaves compute units idle (see the header).
+namespace {
+int spread_over_chunks(const void *const *per_device, int P, int S, const void **per_chunk, const char *fn) {
+  if (P < 1 || S < 1 || (long)P * S > MS_MAX_SLICES) return fail(MS_ERR_ARG, "%s: P * S = %d * %d outside [1, %d]", fn, P, S, MS_MAX_SLICES);
+  if (!per_device) return fail(MS_ERR_ARG, "%s: null pointer table", fn);
+  for (int c = 0; c < P * S; c++) per_chunk[c] = per_device[c / S];
+  return MS_OK;
+}
+}  // namespace
+
+MS_API int ms_gemm_ls_peers(const void *const *A, int lda, const void *const *W_slices, int ldw, int P, int S, int m, int n_slice, int k,
+                            void *const *Y_chunks, int ldy, int in_dtype, int out_dtype, void *stream) {
+  const void *a[MS_MAX_SLICES];
+  if (int rc = spread_over_chunks(A, P, S, a, "ms_gemm_ls_peers")) return rc;
+  return run(make_problem(LS, a, W_slices, Y_chunks, P * S, P * S, P * S, P * S, m, n_slice, k, lda, ldw, ldy, in_dtype, out_dtype), stream);
+}
+
+MS_API int ms_gemm_rs_peers(const void *const *X_slices, int ldx, const void *const *W, int ldw, int P, int S, int m_slice, int n, int k,
+                            void *const *Y_chunks, int ldy, int in_dtype, int out_dtype, void *stream) {
+  const void *w[MS_MAX_SLICES];
+  if (int rc = spread_over_chunks(W, P, S, w, "ms_gemm_rs_peers")) return rc;
+  return run(make_problem(RS, X_slices, w, Y_chunks, P * S, P * S, P * S, P * S, m_slice, n, k, ldx, ldw, ldy, in_dtype, out_dtype), stream);
 }
 
 // the chunk-producing calls with completion counters

@@ -312,6 +312,49 @@ def gemm_rs(X_slices: Sequence[torch.Tensor], W: torch.Tensor,
     return call.out
 
 
+def gemm_ls_peers(A_shards: Sequence[torch.Tensor], W_slices_by_peer: Sequence[Sequence[torch.Tensor]]) -> List[List[torch.Tensor]]:
+    """``gemm_ls`` of the P devices of a mesh row in one launch (``ms_gemm_ls_peers``): fp32 chunks
+    ``[p][s] = A_shards[p] @ W_slices_by_peer[p][s]^T``, all shards and all slices of one shape and leading dimension."""
+    a0 = _same(A_shards, "A_shards")
+    flat = [w for peer in W_slices_by_peer for w in peer]
+    w0 = _same(flat, "W_slices")
+    P, S = len(A_shards), len(flat) // len(A_shards)
+    if any(len(peer) != S for peer in W_slices_by_peer) or len(W_slices_by_peer) != P:
+        raise ValueError("every device must bring the same number of slices")
+    if a0.shape[1] != w0.shape[1] or a0.dtype != w0.dtype or a0.device != w0.device:
+        raise ValueError(f"shapes do not contract: {tuple(a0.shape)} @ {tuple(w0.shape)}^T")
+    m, k = a0.shape; ns = w0.shape[0]
+    return _peers(_lib.load().ms_gemm_ls_peers, A_shards, flat, P, S, (m, ns), (m, ns, k))
+
+
+def gemm_rs_peers(X_slices_by_peer: Sequence[Sequence[torch.Tensor]], W_shards: Sequence[torch.Tensor]) -> List[List[torch.Tensor]]:
+    """``gemm_rs`` of the P devices of a mesh column in one launch (``ms_gemm_rs_peers``): fp32 chunks
+    ``[p][s] = X_slices_by_peer[p][s]^T @ W_shards[p]``."""
+    w0 = _same(W_shards, "W_shards")
+    flat = [x for peer in X_slices_by_peer for x in peer]
+    x0 = _same(flat, "X_slices")
+    P, S = len(W_shards), len(flat) // len(W_shards)
+    if any(len(peer) != S for peer in X_slices_by_peer) or len(X_slices_by_peer) != P:
+        raise ValueError("every device must bring the same number of slices")
+    if x0.shape[0] != w0.shape[0] or x0.dtype != w0.dtype or x0.device != w0.device:
+        raise ValueError(f"shapes do not contract: {tuple(x0.shape)}^T @ {tuple(w0.shape)}")
+    k, ms = x0.shape; n = w0.shape[1]
+    return _peers(_lib.load().ms_gemm_rs_peers, flat, W_shards, P, S, (ms, n), (ms, n, k))
+
+
+def _peers(entry, first, second, P, S, chunk, extents):
+    f0, s0 = first[0], second[0]
+    buf = torch.empty((P * S,) + chunk, dtype=torch.float32, device=f0.device)
+    pf, _kf = _lib.ptr_array([t.data_ptr() for t in first])
+    ps, _ks = _lib.ptr_array([t.data_ptr() for t in second])
+    step, base = buf.stride(0) * 4, buf.data_ptr()
+    py, _ky = _lib.ptr_array([base + i * step for i in range(P * S)])
+    with torch.cuda.device(f0.device):
+        rc = entry(pf, f0.stride(0), ps, s0.stride(0), P, S, *extents, py, chunk[1], _dt(f0), _lib.MS_DTYPE_F32, _stream())
+    _lib.check(rc)
+    return [[buf[p * S + s] for s in range(S)] for p in range(P)]
+
+
 def _check_counters(chunk_done: torch.Tensor, S: int, device) -> None:
     if not (isinstance(chunk_done, torch.Tensor) and chunk_done.is_cuda and chunk_done.device == device
             and chunk_done.dtype == torch.int32 and chunk_done.is_contiguous() and chunk_done.numel() >= S):

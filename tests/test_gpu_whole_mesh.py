@@ -1,0 +1,73 @@
+"""Global products of an emulated mesh in one launch per dataflow step against the same products device by device."""
+import ctypes
+
+import pytest
+import torch
+
+from meshslice_amd import TensorParallel as TP, _lib, local_gemm
+from meshslice_amd.mesh import Mesh, create_device_mesh
+
+pytestmark = pytest.mark.gpu
+
+# mesh, K, B, units of (rows, columns, contraction) in the smallest extents that divide
+CASES = [(4, 2, 4, 8, 3, 2, 1), (2, 4, 8, 8, 5, 1, 2), (1, 2, 2, 8, 7, 3, 1), (3, 2, 3, 8, 1, 2, 3), (2, 2, 2, 2, 9, 4, 8)]
+
+
+def _operands(flow, R, C, K, B, u, v, w, dtype):
+    g = torch.Generator(device="cuda").manual_seed(u * 100 + v * 10 + w)
+    q, edge = R * C * K * B, R * C * 8
+    m, n, k = {"os": (R * u, edge * v, q * w), "ls": (R * u, q * v, edge * w), "rs": (q * v, edge * u, R * 5 * w)}[flow]
+    x, y = {"os": ((m, k), (k, n)), "ls": ((m, k), (n, k)), "rs": ((k, m), (k, n))}[flow]
+    rnd = lambda s: torch.randn(s, generator=g, device="cuda").to(dtype)
+    return rnd(x), rnd(y)
+
+
+def _dense(flow, X, W):
+    X, W = X.double().cpu(), W.double().cpu()
+    return X @ W if flow == "os" else X @ W.t() if flow == "ls" else X.t() @ W
+
+
+@pytest.mark.parametrize("algorithm", ["meshflow", "collective"])
+@pytest.mark.parametrize("flow", ["os", "ls", "rs"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("R,C,K,B,u,v,w", CASES)
+def test_whole_mesh_products_equal_the_devices_products(R, C, K, B, u, v, w, dtype, flow, algorithm, monkeypatch):
+    """Both ways add the same fp32 products, OS perhaps in another order: each is one rounding (2^-9 of an element, bf16) or
+    the 1e-5 of the fp32 path from the float64 product.  Operands that are windows of wider matrices, at row pitches the
+    kernels can and cannot address in place, give the same bits."""
+    X, W = _operands(flow, R, C, K, B, u, v, w, dtype)
+    f = getattr(TP.SPMD(Mesh(create_device_mesh((R, C)), ("row", "col")), algorithm, B), flow.upper())(K)
+    tol = 2.0 ** -8 if dtype == torch.bfloat16 else 1e-5
+    got = f(X, W)
+    for pad in (8, 3):
+        Xp = torch.zeros(X.shape[0], X.shape[1] + pad, dtype=dtype, device="cuda")[:, pad:].copy_(X)
+        Wp = torch.zeros(W.shape[0], W.shape[1] + pad, dtype=dtype, device="cuda")[:, pad:].copy_(W)
+        assert torch.equal(f(Xp, Wp), got)
+    monkeypatch.setattr(TP, "_fits_whole_mesh", lambda *a: False)
+    each = f(X, W)
+    want = _dense(flow, X, W)
+    for y in (got, each):
+        assert y.dtype == dtype and y.is_contiguous() and tuple(y.shape) == tuple(want.shape)
+        assert float((y.double().cpu() - want).norm() / want.norm()) <= tol
+
+
+@pytest.mark.parametrize("flow", ["os", "ls", "rs"])
+def test_a_mesh_whose_devices_would_be_refused_is_refused(flow):
+    """Four columns of the product (LS: of the contraction) per device: not a multiple of the kernels' eight bf16 elements."""
+    mesh = Mesh(create_device_mesh((1, 4)), ("row", "col"))
+    rnd = lambda *s: torch.randn(*s, device="cuda").bfloat16()
+    X, W = {"os": (rnd(64, 64), rnd(64, 16)), "ls": (rnd(64, 16), rnd(64, 16)), "rs": (rnd(64, 64), rnd(64, 16))}[flow]
+    with pytest.raises(ValueError):
+        getattr(TP.SPMD(mesh, "meshflow"), flow.upper())(2)(X, W)
+
+
+def test_peers_products_check_their_tables():
+    a, w = torch.randn(16, 32, device="cuda"), torch.randn(24, 32, device="cuda")
+    got = local_gemm.gemm_ls_peers([a, 2 * a], [[w, w], [w, w]])
+    assert len(got) == 2 and torch.equal(got[0][1], got[0][0]) and torch.equal(got[1][0], 2 * got[0][0])
+    with pytest.raises(ValueError):
+        local_gemm.gemm_ls_peers([a, a], [[w, w], [w]])
+    with pytest.raises(ValueError):
+        local_gemm.gemm_rs_peers([[w.t().contiguous()] * 33] * 2, [w.t().contiguous()] * 2)        # 66 chunks
+    lib = _lib.load()
+    assert lib.ms_gemm_ls_peers(None, 32, None, 32, 2, 2, 16, 24, 32, None, 24, 0, 0, ctypes.c_void_p(0)) == _lib.MS_ERR_ARG

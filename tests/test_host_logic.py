@@ -360,3 +360,21 @@ def test_neighbouring_shards_are_gathered_as_one_view():
     assert TP._spanning([G[:4, :32], G[:4, 32:40]], 1) is None and torch.equal(TP._spanning([G[:4]], 0), G[:4])
     tall = torch.zeros(1, 8).expand(TP.PANEL_MAX_ROWS + 8, 8)
     assert TP._spanning([tall], 1) is None                                      # more rows than one launch takes
+
+
+def test_which_meshes_run_as_one_product():
+    """_fits_whole_mesh looks at shapes and strides only: extents of one device that the kernels refuse, tables of more than
+    64 chunks, operands of 2 GiB, transposed operands and unknown types stay with the device-by-device path."""
+    z = lambda *s, dtype=torch.bfloat16: torch.empty((1,) * len(s), dtype=dtype).expand(*s)        # shape only
+    row = lambda r, c, dtype=torch.bfloat16: torch.empty(r, c, dtype=dtype, device="meta")
+    fits = TP._fits_whole_mesh
+    assert fits("os", row(64, 256), row(256, 64), 2, 4, 4) and not fits("os", row(64, 256), row(256, 16), 2, 4, 4)
+    assert fits("os", row(64, 256, torch.float32), row(256, 16, torch.float32), 2, 4, 4)
+    assert fits("ls", row(64, 64), row(512, 64), 2, 4, 8) and not fits("ls", row(64, 16), row(512, 16), 2, 4, 8)
+    assert fits("ls", row(64, 256), row(512, 256), 2, 4, 16) and not fits("ls", row(64, 256), row(2048, 256), 2, 4, 32)
+    assert fits("rs", row(64, 512), row(64, 64), 2, 4, 8) and not fits("rs", row(64, 512), row(64, 16), 2, 4, 8)
+    assert not fits("os", row(64, 256).t(), row(64, 64), 2, 4, 2) and not fits("os", z(64, 256), z(256, 64), 2, 4, 4)
+    assert not fits("os", row(64, 256, torch.float16), row(256, 64, torch.float16), 2, 4, 4)
+    assert not fits("os", row(1 << 15, 1 << 15), row(1 << 15, 64), 2, 4, 4)         # 2 GiB
+    assert not fits("ls", row(1 << 14, 64), row(1 << 15, 64), 1, 4, 8)              # 8 GiB of chunks
+    assert not fits("os", row(TP.PANEL_MAX_ROWS + 8, 64), row(64, 64), 2, 4, 2)
