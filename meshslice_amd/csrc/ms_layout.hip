@@ -27,46 +27,62 @@ long long table_stride(const void *const *tab, int n) {
   return d;
 }
 
-int grid_for(int rows, int ucols, int tx, dim3 *g, const char *fn) {
-  const int rows_per_block = (256 / tx) * msk::LAYOUT_RT;
+// Rows per thread: one.  A thread then has little in flight by itself, but the launch has eight times the blocks, and these
+// kernels live on loads in flight over the whole device.  S = 4 or 8 slices, eight rows per thread -> one: reducing four
+// peers' fp32 chunks to a bf16 shard of 512 x 256 15.3 -> 3.9 us, 1024 x 768 18.4 -> 5.7, 2048 x 3072 30.2 -> 24.5,
+// 4096 x 12288 171 -> 159; cutting 1024 x 768 bf16 3.3 -> 2.8, 4096 x 12288 35.3 -> 34.2 us.  Eight rows stay for what
+// one row cannot launch (the grid's second extent ends at 65535) and for shards that move element by element, where the
+// two divisions per thread weigh most, once eight rows fill the device (512 blocks, two per compute unit).
+constexpr int GRID_Y_MAX = 65535, FULL_BLOCKS = 512;
+int rows_per_thread(int rows, int ucols, int tx, bool wide) {
+  const int rows_per_block = 256 / tx;
+  const long long blocks8 = ((long long)rows + rows_per_block * msk::LAYOUT_RT - 1) / (rows_per_block * msk::LAYOUT_RT) * ((ucols + tx - 1) / tx);
+  const bool fits = ((long long)rows + rows_per_block - 1) / rows_per_block <= GRID_Y_MAX;
+  return fits && (wide || blocks8 < FULL_BLOCKS) ? msk::LAYOUT_RT_SMALL : msk::LAYOUT_RT;
+}
+
+int grid_for(int rows, int ucols, int tx, int rt, dim3 *g, const char *fn) {
+  const int rows_per_block = (256 / tx) * rt;
   const long long gy = ((long long)rows + rows_per_block - 1) / rows_per_block;
-  if (gy > 65535) return fail(MS_ERR_UNSUPPORTED, "%s: %d rows exceed one launch", fn, rows);
+  if (gy > GRID_Y_MAX) return fail(MS_ERR_UNSUPPORTED, "%s: %d rows exceed one launch", fn, rows);
   *g = dim3((unsigned)((ucols + tx - 1) / tx), (unsigned)gy, 1);
   return MS_OK;
 }
 
 template <int UB>
-int launch_pack(int axis, int tx, dim3 g, hipStream_t st, const msk::PackArgs &a) {
-#define MS_PACK(TX)                                                                                  \
-  if (tx == TX) {                                                                                    \
-    if (axis == 1) hipLaunchKernelGGL((msk::pack_cols_kernel<UB, TX>), g, dim3(256), 0, st, a);      \
-    else hipLaunchKernelGGL((msk::pack_rows_kernel<UB, TX>), g, dim3(256), 0, st, a);                \
+int launch_pack(int axis, int tx, int rt, dim3 g, hipStream_t st, const msk::PackArgs &a) {
+#define MS_PACK(TX, RT)                                                                                  \
+  if (tx == TX && rt == RT) {                                                                            \
+    if (axis == 1) hipLaunchKernelGGL((msk::pack_cols_kernel<UB, TX, RT>), g, dim3(256), 0, st, a);      \
+    else hipLaunchKernelGGL((msk::pack_rows_kernel<UB, TX, RT>), g, dim3(256), 0, st, a);                \
   }
-  MS_PACK(64) MS_PACK(128) MS_PACK(256)
+  MS_PACK(64, msk::LAYOUT_RT) MS_PACK(128, msk::LAYOUT_RT) MS_PACK(256, msk::LAYOUT_RT)
+  MS_PACK(64, msk::LAYOUT_RT_SMALL) MS_PACK(128, msk::LAYOUT_RT_SMALL) MS_PACK(256, msk::LAYOUT_RT_SMALL)
 #undef MS_PACK
   MS_HIP(hipGetLastError());
   return MS_OK;
 }
 
 template <typename TIN, typename TOUT, int VEC>
-int launch_unpack(int axis, int tx, dim3 g, hipStream_t st, const msk::UnpackArgs &a) {
-#define MS_UNPACK(TX)                                                                                          \
-  if (tx == TX) {                                                                                              \
-    if (axis == 1) hipLaunchKernelGGL((msk::unpack_cols_kernel<TIN, TOUT, VEC, TX>), g, dim3(256), 0, st, a);  \
-    else hipLaunchKernelGGL((msk::unpack_rows_kernel<TIN, TOUT, VEC, TX>), g, dim3(256), 0, st, a);            \
+int launch_unpack(int axis, int tx, int rt, dim3 g, hipStream_t st, const msk::UnpackArgs &a) {
+#define MS_UNPACK(TX, RT)                                                                                          \
+  if (tx == TX && rt == RT) {                                                                                      \
+    if (axis == 1) hipLaunchKernelGGL((msk::unpack_cols_kernel<TIN, TOUT, VEC, TX, RT>), g, dim3(256), 0, st, a);  \
+    else hipLaunchKernelGGL((msk::unpack_rows_kernel<TIN, TOUT, VEC, TX, RT>), g, dim3(256), 0, st, a);            \
   }
-  MS_UNPACK(64) MS_UNPACK(128) MS_UNPACK(256)
+  MS_UNPACK(64, msk::LAYOUT_RT) MS_UNPACK(128, msk::LAYOUT_RT) MS_UNPACK(256, msk::LAYOUT_RT)
+  MS_UNPACK(64, msk::LAYOUT_RT_SMALL) MS_UNPACK(128, msk::LAYOUT_RT_SMALL) MS_UNPACK(256, msk::LAYOUT_RT_SMALL)
 #undef MS_UNPACK
   MS_HIP(hipGetLastError());
   return MS_OK;
 }
 
 template <int VEC>
-int launch_unpack_typed(int in_dtype, int out_dtype, int axis, int tx, dim3 g, hipStream_t st, const msk::UnpackArgs &a) {
+int launch_unpack_typed(int in_dtype, int out_dtype, int axis, int tx, int rt, dim3 g, hipStream_t st, const msk::UnpackArgs &a) {
   typedef unsigned short bf16_bits;
   if (in_dtype == MS_DTYPE_F32)
-    return out_dtype == MS_DTYPE_F32 ? launch_unpack<float, float, VEC>(axis, tx, g, st, a) : launch_unpack<float, bf16_bits, VEC>(axis, tx, g, st, a);
-  return out_dtype == MS_DTYPE_F32 ? launch_unpack<bf16_bits, float, VEC>(axis, tx, g, st, a) : launch_unpack<bf16_bits, bf16_bits, VEC>(axis, tx, g, st, a);
+    return out_dtype == MS_DTYPE_F32 ? launch_unpack<float, float, VEC>(axis, tx, rt, g, st, a) : launch_unpack<float, bf16_bits, VEC>(axis, tx, rt, g, st, a);
+  return out_dtype == MS_DTYPE_F32 ? launch_unpack<bf16_bits, float, VEC>(axis, tx, rt, g, st, a) : launch_unpack<bf16_bits, bf16_bits, VEC>(axis, tx, rt, g, st, a);
 }
 
 }  // namespace
@@ -103,11 +119,11 @@ MS_API int ms_pack_slices(const void *src, int ld_src, int rows, int cols, int a
   a.S = S;
   a.G = axis == 1 ? B * es / ub : B;
   a.tab_stride = table_stride(dst_slices, S);
-  const int tx = pick_tx(a.ucols);
+  const int tx = pick_tx(a.ucols), rt = rows_per_thread(rows, a.ucols, tx, wide);
   dim3 g;
-  if (int rc = grid_for(rows, a.ucols, tx, &g, fn)) return rc;
+  if (int rc = grid_for(rows, a.ucols, tx, rt, &g, fn)) return rc;
   hipStream_t st = (hipStream_t)stream;
-  return ub == 16 ? launch_pack<16>(axis, tx, g, st, a) : ub == 4 ? launch_pack<4>(axis, tx, g, st, a) : launch_pack<2>(axis, tx, g, st, a);
+  return ub == 16 ? launch_pack<16>(axis, tx, rt, g, st, a) : ub == 4 ? launch_pack<4>(axis, tx, rt, g, st, a) : launch_pack<2>(axis, tx, rt, g, st, a);
 }
 
 MS_API int ms_unpack_chunks(const void *const *chunks, int P, int S, int ld_chunk, int row_off, int col_off,
@@ -148,10 +164,10 @@ MS_API int ms_unpack_chunks(const void *const *chunks, int P, int S, int ld_chun
   a.S = S;
   a.B = B;
   a.tab_stride = table_stride(chunks, P * S);
-  const int tx = pick_tx(a.ucols);
+  const int tx = pick_tx(a.ucols), rt = rows_per_thread(rows, a.ucols, tx, wide);
   dim3 g;
-  if (int rc = grid_for(rows, a.ucols, tx, &g, fn)) return rc;
+  if (int rc = grid_for(rows, a.ucols, tx, rt, &g, fn)) return rc;
   hipStream_t st = (hipStream_t)stream;
-  if (move_f32) return launch_unpack<float, float, 4>(axis, tx, g, st, a);
-  return wide ? launch_unpack_typed<8>(in_dtype, out_dtype, axis, tx, g, st, a) : launch_unpack_typed<1>(in_dtype, out_dtype, axis, tx, g, st, a);
+  if (move_f32) return launch_unpack<float, float, 4>(axis, tx, rt, g, st, a);
+  return wide ? launch_unpack_typed<8>(in_dtype, out_dtype, axis, tx, rt, g, st, a) : launch_unpack_typed<1>(in_dtype, out_dtype, axis, tx, rt, g, st, a);
 }

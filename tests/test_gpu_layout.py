@@ -253,3 +253,26 @@ def test_layout_calls_reject_bad_arguments():
     assert L.ms_pack_slices(ctypes.c_void_p(x.data_ptr()), 64, 64, 64, 1, 2, 8, ptrs, 32, 7, null) == _lib.MS_ERR_UNSUPPORTED
     assert L.ms_pack_slices(ctypes.c_void_p(x.data_ptr()), 64, 64, 64, 1, 2, 8, None, 32, 1, null) == _lib.MS_ERR_ARG
     assert L.ms_pack_slices(ctypes.c_void_p(x.data_ptr()), 32, 64, 64, 1, 2, 8, ptrs, 32, 1, null) == _lib.MS_ERR_ARG
+
+
+# rows, cols, S, B, axis, P, dtype: more rows than one launch covers at one row per thread (65535 blocks), sliced either way;
+# shards moved element by element (blocks of two) that fill the device at eight rows per thread, with a ragged last group;
+# more peers than are loaded at a time, and a count that ends inside a group
+ROWS_PER_THREAD_CASES = [(65544, 1056, 2, 8, 1, 1, torch.bfloat16), (65552, 1048, 2, 8, 0, 2, torch.bfloat16), (4101, 1024, 4, 2, 1, 3, torch.bfloat16),
+                         (4104, 516, 3, 2, 0, 2, torch.float32), (37, 512, 4, 8, 1, 5, torch.float32), (48, 264, 2, 8, 0, 8, torch.bfloat16)]
+
+
+@pytest.mark.parametrize("r,c,S,B,axis,P,dtype", ROWS_PER_THREAD_CASES)
+def test_every_count_of_rows_per_thread_moves_every_element_once(r, c, S, B, axis, P, dtype):
+    """Against torch's own indexing, bit for bit: placement is exact, and the fp32 sum runs in peer order on both sides."""
+    g = torch.Generator(device="cuda").manual_seed(r + c)
+    x = torch.randn(r, c, generator=g, device="cuda").to(dtype)
+    cut = (lambda t: [s.reshape(r, -1) for s in t.reshape(r, -1, S, B).unbind(2)]) if axis == 1 else (lambda t: [s.reshape(-1, c) for s in t.reshape(-1, S, B, c).unbind(1)])
+    for got, want in zip(sl.pack_slices(x, S, B, axis), cut(x)):
+        assert torch.equal(got, want)
+    whole = [torch.randn(r, c, generator=g, device="cuda") for _ in range(P)]
+    want = whole[0].clone()
+    for t in whole[1:]:
+        want += t
+    got = sl.unpack_chunks([[s.contiguous() for s in cut(t)] for t in whole], B, axis, out_dtype=dtype)
+    assert torch.equal(got, want.to(dtype))
