@@ -158,5 +158,5 @@ def check(rc: int) -> None:
 
 
 def ptr_array(ptrs):
-    arr = (ctypes.c_void_p * len(ptrs))(*[int(p) for p in ptrs])
-    return ctypes.cast(arr, ctypes.POINTER(ctypes.c_void_p)), arr
+    arr = (ctypes.c_void_p * len(ptrs))(*map(int, ptrs))
+    return arr, arr       # (a c_void_p array is taken where a pointer to c_void_p is declared)

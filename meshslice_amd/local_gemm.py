@@ -7,6 +7,7 @@ libmeshslice_hip.so.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import threading
 from typing import List, Optional, Sequence
@@ -39,11 +40,21 @@ def _same(ts: Sequence[torch.Tensor], name: str):
     if len(ts) < 1:
         raise ValueError(f"{name}: need at least one slice")
     s0 = ts[0]
+    _check2d(s0, name)
+    shape, strides, dtype, device = s0.shape, s0.stride(), s0.dtype, s0.device
     for t in ts:
-        _check2d(t, name)
-        if t.shape != s0.shape or t.dtype != s0.dtype or t.stride(0) != s0.stride(0) or t.device != s0.device:
+        if t.shape != shape or t.stride() != strides or t.dtype != dtype or t.device != device:
+            _check2d(t, name)
             raise ValueError(f"{name}: all slices must share shape, dtype, leading dimension and device")
     return s0
+
+
+_HERE = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    """``torch.cuda.device(device)``, without its two device switches where the device is the current one already."""
+    return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 _workspaces = {}            # (device index, stream handle) -> uint8 tensor, least recently used first
@@ -130,6 +141,12 @@ def _prepare_os(A_slices, B_slices, out, out_dtype) -> _Call:
     return _Call(a0.device, args, out, (_ka, _kb))
 
 
+def _chunk_views(buf: torch.Tensor):
+    """The [rows, columns] parts of a fresh 3-D buffer and their addresses."""
+    step, base = buf.stride(0) * buf.element_size(), buf.data_ptr()
+    return [buf.select(0, s) for s in range(buf.shape[0])], [base + s * step for s in range(buf.shape[0])]
+
+
 def _prepare_ls(A, W_slices, out, out_dtype) -> _Call:
     _check2d(A, "A"); w0 = _same(W_slices, "W_slices")
     if A.shape[1] != w0.shape[1] or A.dtype != w0.dtype or A.device != w0.device:
@@ -137,13 +154,15 @@ def _prepare_ls(A, W_slices, out, out_dtype) -> _Call:
     m, k = A.shape; ns = w0.shape[0]; S = len(W_slices)
     dt = _chunk_dtype(out, out_dtype)
     if out is None:
-        buf = torch.empty((S, m, ns), dtype=dt, device=A.device)
-        out = [buf[s] for s in range(S)]
-    o0 = _same(out, "out")
-    if len(out) != S or tuple(o0.shape) != (m, ns) or o0.dtype not in (torch.float32, torch.bfloat16) or o0.device != A.device:
-        raise ValueError("out must be S fp32 or bf16 chunks of shape [m, n_slice] on the operands' device")
+        out, ptrs = _chunk_views(torch.empty((S, m, ns), dtype=dt, device=A.device))
+        o0 = out[0]
+    else:
+        o0 = _same(out, "out")
+        if len(out) != S or tuple(o0.shape) != (m, ns) or o0.dtype not in (torch.float32, torch.bfloat16) or o0.device != A.device:
+            raise ValueError("out must be S fp32 or bf16 chunks of shape [m, n_slice] on the operands' device")
+        ptrs = [t.data_ptr() for t in out]
     pw, _kw = _lib.ptr_array([t.data_ptr() for t in W_slices])
-    py, _ky = _lib.ptr_array([t.data_ptr() for t in out])
+    py, _ky = _lib.ptr_array(ptrs)
     args = (ctypes.c_void_p(A.data_ptr()), A.stride(0), pw, w0.stride(0), S, m, ns, k, py, o0.stride(0), _dt(A), _dt(o0))
     return _Call(A.device, args, list(out), (_kw, _ky))
 
@@ -155,13 +174,15 @@ def _prepare_rs(X_slices, W, out, out_dtype) -> _Call:
     k, ms = x0.shape; n = W.shape[1]; S = len(X_slices)
     dt = _chunk_dtype(out, out_dtype)
     if out is None:
-        buf = torch.empty((S, ms, n), dtype=dt, device=W.device)
-        out = [buf[s] for s in range(S)]
-    o0 = _same(out, "out")
-    if len(out) != S or tuple(o0.shape) != (ms, n) or o0.dtype not in (torch.float32, torch.bfloat16) or o0.device != W.device:
-        raise ValueError("out must be S fp32 or bf16 chunks of shape [m_slice, n] on the operands' device")
+        out, ptrs = _chunk_views(torch.empty((S, ms, n), dtype=dt, device=W.device))
+        o0 = out[0]
+    else:
+        o0 = _same(out, "out")
+        if len(out) != S or tuple(o0.shape) != (ms, n) or o0.dtype not in (torch.float32, torch.bfloat16) or o0.device != W.device:
+            raise ValueError("out must be S fp32 or bf16 chunks of shape [m_slice, n] on the operands' device")
+        ptrs = [t.data_ptr() for t in out]
     px, _kx = _lib.ptr_array([t.data_ptr() for t in X_slices])
-    py, _ky = _lib.ptr_array([t.data_ptr() for t in out])
+    py, _ky = _lib.ptr_array(ptrs)
     args = (px, x0.stride(0), ctypes.c_void_p(W.data_ptr()), W.stride(0), S, ms, n, k, py, o0.stride(0), _dt(W), _dt(o0))
     return _Call(W.device, args, list(out), (_kx, _ky))
 
@@ -193,11 +214,13 @@ def gemm_os(A_slices: Sequence[torch.Tensor], B_slices: Sequence[torch.Tensor],
                     and t.device == out.device):
                 raise ValueError("row moments must be contiguous fp32 GPU vectors of length m on the output's device")
             moments[idx] = ctypes.c_void_p(t.data_ptr())
-    ws_ptr, ws_bytes, _ws_keep = _ws_args(call.device)
-    with torch.cuda.device(call.device):
+    with _on(call.device):
+        stream = torch.cuda.current_stream()
+        ws = workspace(call.device, stream)
         rc = _lib.load().ms_gemm_os_ws(*call.args,
                                        _lib.MS_ACT_GELU if activation == "gelu" else _lib.MS_ACT_NONE,
-                                       res_ptr, ldr, moments[0], moments[1], ws_ptr, ws_bytes, _stream())
+                                       res_ptr, ldr, moments[0], moments[1], ctypes.c_void_p(ws.data_ptr()), ws.numel(),
+                                       ctypes.c_void_p(stream.cuda_stream))
     _lib.check(rc)
     return out
 
@@ -228,7 +251,7 @@ def gemm_os_gated(A_slices: Sequence[torch.Tensor], B_slices: Sequence[torch.Ten
     call = _prepare_os(A_slices, B_slices, out, out_dtype)
     _check_flags(slice_ready, len(A_slices), call.device)
     ws_ptr, ws_bytes, _ws_keep = _ws_args(call.device)
-    with torch.cuda.device(call.device):
+    with _on(call.device):
         rc = _lib.load().ms_gemm_os_gated(*call.args, ws_ptr, ws_bytes, ctypes.c_void_p(slice_ready.data_ptr()),
                                           int(timeout_ms), _stream())
     _lib.check(rc)
@@ -247,7 +270,7 @@ def _chunks_gated(entry, call, S, slice_ready, chunk_done, timeout_ms):
     tiles = ctypes.c_int(0)
     if chunk_done is not None:
         _check_counters(chunk_done, S, call.device)
-    with torch.cuda.device(call.device):
+    with _on(call.device):
         rc = entry(*call.args, ctypes.c_void_p(chunk_done.data_ptr()) if chunk_done is not None else None,
                    ctypes.byref(tiles) if chunk_done is not None else None,
                    ctypes.c_void_p(slice_ready.data_ptr()), int(timeout_ms), _stream())
@@ -296,7 +319,7 @@ def gemm_ls(A: torch.Tensor, W_slices: Sequence[torch.Tensor],
     the reduce-scatter); ``out_dtype=torch.bfloat16`` gives what the reference's einsum returns for bf16
     operands (TensorParallel.py:181-189): one rounding of the fp32 accumulator, half the bytes."""
     call = _prepare_ls(A, W_slices, out, out_dtype)
-    with torch.cuda.device(call.device):
+    with _on(call.device):
         rc = _lib.load().ms_gemm_ls_ex(*call.args, _stream())
     _lib.check(rc)
     return call.out
@@ -306,7 +329,7 @@ def gemm_rs(X_slices: Sequence[torch.Tensor], W: torch.Tensor,
             out: Optional[List[torch.Tensor]] = None, out_dtype: Optional[torch.dtype] = None) -> List[torch.Tensor]:
     """``Y_s = X_s^T @ W``, X_s stored ``[k, m_slice]``; chunks fp32 by default, bf16 on request (see gemm_ls)."""
     call = _prepare_rs(X_slices, W, out, out_dtype)
-    with torch.cuda.device(call.device):
+    with _on(call.device):
         rc = _lib.load().ms_gemm_rs_ex(*call.args, _stream())
     _lib.check(rc)
     return call.out
@@ -347,12 +370,12 @@ def _peers(entry, first, second, P, S, chunk, extents):
     buf = torch.empty((P * S,) + chunk, dtype=torch.float32, device=f0.device)
     pf, _kf = _lib.ptr_array([t.data_ptr() for t in first])
     ps, _ks = _lib.ptr_array([t.data_ptr() for t in second])
-    step, base = buf.stride(0) * 4, buf.data_ptr()
-    py, _ky = _lib.ptr_array([base + i * step for i in range(P * S)])
-    with torch.cuda.device(f0.device):
+    chunks, ptrs = _chunk_views(buf)
+    py, _ky = _lib.ptr_array(ptrs)
+    with _on(f0.device):
         rc = entry(pf, f0.stride(0), ps, s0.stride(0), P, S, *extents, py, chunk[1], _dt(f0), _lib.MS_DTYPE_F32, _stream())
     _lib.check(rc)
-    return [[buf[p * S + s] for s in range(S)] for p in range(P)]
+    return [chunks[p * S:(p + 1) * S] for p in range(P)]
 
 
 def _check_counters(chunk_done: torch.Tensor, S: int, device) -> None:
@@ -370,7 +393,7 @@ def gemm_ls_signal(A: torch.Tensor, W_slices: Sequence[torch.Tensor], chunk_done
     call = _prepare_ls(A, W_slices, out, out_dtype)
     _check_counters(chunk_done, len(W_slices), call.device)
     tiles = ctypes.c_int(0)
-    with torch.cuda.device(call.device):
+    with _on(call.device):
         rc = _lib.load().ms_gemm_ls_signal(*call.args, ctypes.c_void_p(chunk_done.data_ptr()), ctypes.byref(tiles), _stream())
     _lib.check(rc)
     return call.out, tiles.value
@@ -383,7 +406,7 @@ def gemm_rs_signal(X_slices: Sequence[torch.Tensor], W: torch.Tensor, chunk_done
     call = _prepare_rs(X_slices, W, out, out_dtype)
     _check_counters(chunk_done, len(X_slices), call.device)
     tiles = ctypes.c_int(0)
-    with torch.cuda.device(call.device):
+    with _on(call.device):
         rc = _lib.load().ms_gemm_rs_signal(*call.args, ctypes.c_void_p(chunk_done.data_ptr()), ctypes.byref(tiles), _stream())
     _lib.check(rc)
     return call.out, tiles.value
@@ -406,7 +429,7 @@ def time_call(flow: str, operands, out, warmup: int = 5, reps: int = 20) -> List
         call = _prepare_os(first, second, out, None)
         ms = (ctypes.c_float * int(reps))()
         ws_ptr, ws_bytes, _ws_keep = _ws_args(call.device)
-        with torch.cuda.device(call.device):
+        with _on(call.device):
             rc = lib.ms_time_os_ws(*call.args, ws_ptr, ws_bytes, _stream(), int(warmup), int(reps), ms)
         _lib.check(rc)
         return list(ms)
@@ -415,7 +438,7 @@ def time_call(flow: str, operands, out, warmup: int = 5, reps: int = 20) -> List
     else:
         call, fn = _prepare_rs(first, second, out, None), lib.ms_time_rs_ex
     ms = (ctypes.c_float * int(reps))()
-    with torch.cuda.device(call.device):
+    with _on(call.device):
         rc = fn(*call.args, _stream(), int(warmup), int(reps), ms)
     _lib.check(rc)
     return list(ms)

@@ -15,7 +15,7 @@ from typing import List, Optional, Sequence
 import torch
 
 from . import _lib
-from .local_gemm import _check2d, _dt, _same, _stream
+from .local_gemm import _check2d, _chunk_views, _dt, _on, _same, _stream
 
 
 def pack_slices(block: torch.Tensor, S: int, B: int, axis: int,
@@ -32,13 +32,15 @@ def pack_slices(block: torch.Tensor, S: int, B: int, axis: int,
         raise ValueError(f"sliced extent {c if axis == 1 else r} is not a multiple of S*B = {S}*{B}")
     shape = (r, c // S) if axis == 1 else (r // S, c)
     if out is None:
-        buf = torch.empty((S,) + shape, dtype=block.dtype, device=block.device)
-        out = [buf[s] for s in range(S)]
-    o0 = _same(out, "out")
-    if len(out) != S or tuple(o0.shape) != shape or o0.dtype != block.dtype or o0.device != block.device:
-        raise ValueError(f"out must be S slices of shape {shape} and the dtype of block")
-    pd, _kd = _lib.ptr_array([t.data_ptr() for t in out])
-    with torch.cuda.device(block.device):
+        out, ptrs = _chunk_views(torch.empty((S,) + shape, dtype=block.dtype, device=block.device))
+        o0 = out[0]
+    else:
+        o0 = _same(out, "out")
+        if len(out) != S or tuple(o0.shape) != shape or o0.dtype != block.dtype or o0.device != block.device:
+            raise ValueError(f"out must be S slices of shape {shape} and the dtype of block")
+        ptrs = [t.data_ptr() for t in out]
+    pd, _kd = _lib.ptr_array(ptrs)
+    with _on(block.device):
         rc = _lib.load().ms_pack_slices(ctypes.c_void_p(block.data_ptr()), block.stride(0), r, c, axis, S, B,
                                         pd, o0.stride(0), _dt(block), _stream())
     _lib.check(rc)
@@ -77,7 +79,7 @@ def unpack_chunks(chunks_by_peer: Sequence[Sequence[torch.Tensor]], B: int, axis
     if tuple(out.shape) != (rows, cols) or out.device != c0.device or (out_dtype is not None and out.dtype != out_dtype):
         raise ValueError(f"out must be a [{rows}, {cols}] tensor of the requested dtype on the chunks' device")
     pc, _kc = _lib.ptr_array([t.data_ptr() for t in flat])
-    with torch.cuda.device(c0.device):
+    with _on(c0.device):
         rc = _lib.load().ms_unpack_chunks(pc, P, S, c0.stride(0), row_off, col_off, rows, cols, axis, B,
                                           ctypes.c_void_p(out.data_ptr()), out.stride(0), _dt(c0), _dt(out), _stream())
     _lib.check(rc)
