@@ -22,6 +22,7 @@ by having one GPU and no tracing compiler:
 """
 from __future__ import annotations
 
+import threading
 from typing import Callable, List, Sequence
 
 import torch
@@ -158,7 +159,11 @@ def MeshFlow_OS(X, W, i, j, R, C, K, B):
     return local_gemm.gemm_os(A_slices, B_slices)
 
 
-_gather_streams = {}
+_gather_streams = {}           # (device, handle of the product's stream) -> the stream for its gathers, or None
+_gather_streams_lock = threading.Lock()
+_GATHER_STREAMS_MAX = 16
+_GATHER_STREAM_TRIES = 6
+_PROBE_TIMEOUT_MS = 50
 OVERLAP_RESERVED_CUS = 32      # compute units left to the emulated gathers' copy kernels beside the waiting product
 
 
@@ -189,28 +194,83 @@ def _row_slice_filler(peers, K, B):
     return buf, fill
 
 
+def _runs_beside(cur, other, dev) -> bool:
+    """Whether kernels on stream ``other`` run while a launch on ``cur`` waits.  The streams of a process share a few
+    hardware queues and two that share one run in order, so the device is asked: the smallest gated product waits, at
+    most _PROBE_TIMEOUT_MS, for a flag that ``other`` raises."""
+    ready = torch.zeros(2, dtype=torch.int32, device=dev)
+    a = torch.zeros((8, 512), dtype=torch.bfloat16, device=dev)
+    b = torch.zeros((512, 8), dtype=torch.bfloat16, device=dev)
+    other.wait_stream(cur)
+    local_gemm.gemm_os_gated([a], [b], ready, timeout_ms=_PROBE_TIMEOUT_MS)
+    with torch.cuda.stream(other):
+        local_gemm.signal_set(ready, 0)
+    cur.wait_stream(other)
+    return not local_gemm.gate_timed_out(ready)
+
+
+def _gather_stream(dev, cur):
+    """The stream on which the gathers of an overlapped body on stream ``cur`` run: one that has been seen to run beside a
+    waiting launch there, or None if none of a few does.  Looked for once per stream (the first call waits for the device
+    to go idle, so that the search measures queues and not what stands in them)."""
+    key = (dev, cur.cuda_stream)
+    with _gather_streams_lock:
+        if key in _gather_streams:
+            return _gather_streams[key]
+    torch.cuda.synchronize(dev)
+    found = None
+    for _ in range(_GATHER_STREAM_TRIES):
+        stream = torch.cuda.Stream(dev)
+        if _runs_beside(cur, stream, dev):
+            found = stream
+            break
+    with _gather_streams_lock:
+        _gather_streams[key] = found
+        while len(_gather_streams) > _GATHER_STREAMS_MAX:
+            del _gather_streams[next(iter(_gather_streams))]
+    return found
+
+
+def _launch_beside_reserved_units(launch, ready):
+    lib = local_gemm._lib.load()
+    try:
+        lib.ms_set_reserved_cus(OVERLAP_RESERVED_CUS)
+        return launch(ready)
+    finally:
+        lib.ms_set_reserved_cus(0)
+
+
+def _fill_and_flag(K, ready, fills):
+    for k in range(K):
+        for fill in fills:
+            fill(k)
+        local_gemm.signal_set(ready, k)
+
+
 def _launch_ahead_of_gathers(K, dev, launch, fills):
     """``launch(ready)`` enqueues the gated product on the current stream with all K flags down; the emulated gather
     stream then fills slice after slice (``fills``: one callable per gathered operand) and raises its flag.  On a real
-    mesh that stream is the collective's."""
+    mesh that stream is the collective's.  Where no stream runs beside the waiting product the gathers go first; where
+    they came too late for its time limit all the same (a stream that has been given another hardware queue since, a busy
+    device), the product runs again on the slices that have arrived by then."""
     ready = torch.zeros(K + 1, dtype=torch.int32, device=dev)
-    lib = local_gemm._lib.load()
     cur = torch.cuda.current_stream(dev)
-    gather = _gather_streams.setdefault(dev, torch.cuda.Stream(dev))
+    gather = _gather_stream(dev, cur)
+    if gather is None:
+        _fill_and_flag(K, ready, fills)
+        return _launch_beside_reserved_units(launch, ready)
     gather.wait_stream(cur)                              # the flags are cleared and the shards are there
+    out = _launch_beside_reserved_units(launch, ready)
     try:
-        lib.ms_set_reserved_cus(OVERLAP_RESERVED_CUS)
-        out = launch(ready)
+        with torch.cuda.stream(gather):
+            _fill_and_flag(K, ready, fills)
     finally:
-        lib.ms_set_reserved_cus(0)
-    with torch.cuda.stream(gather):
-        for k in range(K):
-            for fill in fills:
-                fill(k)
-            local_gemm.signal_set(ready, k)
-    cur.wait_stream(gather)
+        cur.wait_stream(gather)
     if local_gemm.gate_timed_out(ready):
-        raise local_gemm._lib.MeshSliceError("the gated product gave up waiting for a slice: the gathers did not run beside it")
+        with _gather_streams_lock:
+            _gather_streams.pop((dev, cur.cuda_stream), None)
+        ready[K:].zero_()
+        out = _launch_beside_reserved_units(launch, ready)
     return out
 
 

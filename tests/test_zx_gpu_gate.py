@@ -306,3 +306,56 @@ def test_the_chunk_producing_mesh_bodies_launched_ahead_of_their_gathers_equal_m
     assert torch.equal(got, want)
     dense = (X.float() @ W.float().T) if flow == "ls" else (X.float().T @ W.float())
     assert orc.rel_frobenius(got.float().cpu().numpy(), dense.cpu().numpy()) <= 1e-2
+
+
+def _overlap_operands(flow):
+    shapes = {"os": ((256, 512), (512, 384)), "ls": ((256, 512), (384, 512)), "rs": ((512, 256), (512, 384))}[flow]
+    return _rand(shapes[0], 51, torch.bfloat16), _rand(shapes[1], 52, torch.bfloat16, 0.05)
+
+
+@pytest.mark.parametrize("flow", ["os", "ls", "rs"])
+def test_overlapped_bodies_give_the_product_on_every_stream(flow):
+    """Two streams on one hardware queue run in order, so a gather stream that shares the product's queue would stand behind
+    the product that waits for it.  Nine current streams in turn meet every queue: each gets a gather stream that runs
+    beside it, or its gathers first, and the product either way."""
+    from meshslice_amd import TensorParallel as TP
+    from meshslice_amd.mesh import Mesh, create_device_mesh
+    mesh = Mesh(create_device_mesh((2, 2)), ("x", "y"))
+    X, W = _overlap_operands(flow)
+    lib = _lib.load()
+    lib.ms_set_reserved_cus(TP.OVERLAP_RESERVED_CUS)
+    try:
+        want = getattr(TP.SPMD(mesh, "meshflow"), flow.upper())(4)(X, W)
+    finally:
+        lib.ms_set_reserved_cus(0)
+    torch.cuda.synchronize()
+    for stream in [torch.cuda.current_stream()] + [torch.cuda.Stream() for _ in range(8)]:
+        with torch.cuda.stream(stream):
+            got = getattr(TP.SPMD(mesh, "meshflow_overlap"), flow.upper())(4)(X, W)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("gathers", ["on the product's own stream", "before the product"])
+def test_a_product_whose_gathers_do_not_run_beside_it_still_comes_out(gathers, monkeypatch):
+    """The gathers put on the product's own stream stand behind it: it ends by its time limit (20 ms a slice) and is run
+    again on what has arrived.  With no stream to be had they are enqueued first."""
+    from meshslice_amd import TensorParallel as TP
+    monkeypatch.setattr(TP, "_gather_stream", lambda dev, cur: cur if "own" in gathers else None)
+    K, m, n, k = 3, 256, 384, 512
+    src_a, src_b = _slices(m, n, k, K, torch.bfloat16, seed=61)
+    A = [torch.zeros_like(t) for t in src_a]; B = [torch.zeros_like(t) for t in src_b]
+    calls = []
+
+    def launch(ready):
+        calls.append(1)
+        return ms.gemm_os_gated(A, B, ready, timeout_ms=20)
+    got = TP._launch_ahead_of_gathers(K, A[0].device, launch, (lambda i: A[i].copy_(src_a[i]), lambda i: B[i].copy_(src_b[i])))
+    lib = _lib.load()
+    lib.ms_set_reserved_cus(TP.OVERLAP_RESERVED_CUS)
+    try:
+        want = ms.gemm_os(src_a, src_b)
+    finally:
+        lib.ms_set_reserved_cus(0)
+    assert len(calls) == (2 if "own" in gathers else 1)
+    assert torch.equal(got, want)
