@@ -456,7 +456,8 @@ WHOLE_MESH_MAX_CHUNK_BYTES = 4 << 30      # partial chunks alive at once; device
 def _fits_whole_mesh(dataflow, X, W, R, C, K) -> bool:
     """Whether the mesh's products can run as one: every device's own extents are ones that the kernels take (a mesh whose
     devices would be refused is refused), no operand reaches the 2 GiB that a kernel addresses, the line's chunks fit one
-    pointer table (64) and a bounded buffer, and rows fit one launch of the layout kernels."""
+    pointer table (64) and a bounded buffer, and rows fit one launch of the layout kernels.  (Whether it all fits the memory
+    that is left shows when it is allocated, see ShardedMatmul.__call__.)"""
     q = 16 // X.element_size()
     if X.device != W.device or X.dtype not in (torch.float32, torch.bfloat16) or X.stride(1) != 1 or W.stride(1) != 1:
         return False
@@ -547,15 +548,21 @@ class ShardedMatmul:
             return self.body(_shards(X, self.R, self.C), _shards(W, self.R, self.C), i, j, self.R, self.C, self.K, self.B)
         return run
 
+    def _whole_mesh(self, X, W, K, B):
+        if self.dataflow == "os":      # (the output blocks of all devices are one product: the body on a mesh of one)
+            return self.body([[X]], [[W]], 0, 0, 1, 1, self.K, self.B)
+        return _whole_ls(X, W, self.C, K, B, self.sliced) if self.dataflow == "ls" else _whole_rs(X, W, self.R, K, B, self.sliced)
+
     def __call__(self, X: torch.Tensor, W: torch.Tensor) -> torch.Tensor:
         self._validate(X, W)
         R, C = self.R, self.C
         K = self.K if self.sliced else 1
         B = self.B if self.sliced else 1
         if self.body in _WHOLE_MESH_BODIES[self.dataflow] and _fits_whole_mesh(self.dataflow, X, W, R, C, K):
-            if self.dataflow == "os":      # (the output blocks of all devices are one product: the body on a mesh of one)
-                return self.body([[X]], [[W]], 0, 0, 1, 1, self.K, self.B)
-            return _whole_ls(X, W, C, K, B, self.sliced) if self.dataflow == "ls" else _whole_rs(X, W, R, K, B, self.sliced)
+            try:
+                return self._whole_mesh(X, W, K, B)
+            except torch.OutOfMemoryError:
+                pass       # the gathered operands and chunks of all mesh lines do not fit beside the caller's tensors: one line's may
         Xs, Ws = _shards(X, R, C), _shards(W, R, C)
         run = lambda i, j: self.body(Xs, Ws, i, j, R, C, self.K, self.B)
         if self.dataflow == "os":

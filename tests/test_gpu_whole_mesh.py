@@ -71,3 +71,26 @@ def test_peers_products_check_their_tables():
         local_gemm.gemm_rs_peers([[w.t().contiguous()] * 33] * 2, [w.t().contiguous()] * 2)        # 66 chunks
     lib = _lib.load()
     assert lib.ms_gemm_ls_peers(None, 32, None, 32, 2, 2, 16, 24, 32, None, 24, 0, 0, ctypes.c_void_p(0)) == _lib.MS_ERR_ARG
+
+
+@pytest.mark.parametrize("flow", ["os", "ls", "rs"])
+def test_a_product_that_fits_memory_only_line_by_line_still_runs(flow):
+    """An allowance below what the partial chunks (LS, RS: 512 MiB) or the gathered operands (OS: 128 MiB) of the whole mesh
+    take; a mesh line's (32 MiB, 16 MiB), the output's parts and the output fit it."""
+    R, C, K = (1, 8, 2) if flow == "os" else (16, 2, 2) if flow == "ls" else (2, 16, 2)
+    m, n, k, allowance = (64, 16384, 4096, 100) if flow == "os" else (8192, 8192, 256, 420)
+    a, b = {"os": ((m, k), (k, n)), "ls": ((m, k), (n, k)), "rs": ((k, n), (k, m))}[flow]
+    f = getattr(TP.SPMD(Mesh(create_device_mesh((R, C)), ("row", "col")), "meshflow"), flow.upper())(K)
+    X, W = torch.randn(a, device="cuda").bfloat16(), torch.randn(b, device="cuda").bfloat16()
+    want = f(X, W)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (allowance << 20)) / total)
+        with pytest.raises(torch.OutOfMemoryError):
+            f._whole_mesh(X, W, K, 8)
+        got = f(X, W)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(got, want) if flow != "os" else float((got.double() - want.double()).norm() / want.double().norm()) <= 2.0 ** -8
