@@ -209,6 +209,25 @@ def test_fp32_narrow_tiles_where_the_chooser_takes_them(tile, flow, m, n, k, S):
 
 
 @pytest.mark.parametrize("flow", ["os", "ls", "rs"])
+@pytest.mark.parametrize("m,n,k", [(520, 776, 1000), (264, 392, 9000)])
+def test_unsplit_bf16_products_have_the_same_bits_on_every_tile(m, n, k, flow):
+    """Tile shape, wave count and MFMA shape (32x32x16, 16x16x32) do not change the order in which an output element's
+    products are added; operands spread over e^+-8, so that another order would show."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    rnd = lambda *s: (torch.randn(s, generator=g, device="cuda") * torch.exp(4 * torch.randn(s, generator=g, device="cuda"))).bfloat16()
+    a, b = {"os": ((m, k), (k, n)), "ls": ((m, k), (n, k)), "rs": ((k, m), (k, n))}[flow]
+    a, b = rnd(*a), rnd(*b)
+    run = {"os": lambda: ms.gemm_os([a], [b], out_dtype=torch.float32), "ls": lambda: ms.gemm_ls(a, [b])[0], "rs": lambda: ms.gemm_rs([a], b)[0]}[flow]
+    lib = _lib.load()
+    results = []
+    for v in range(1, 15):
+        _lib.check(lib.ms_set_variant(v))
+        results.append(run())
+        assert lib.ms_query(_lib.MS_QUERY_LAST_VARIANT) == v
+    assert all(torch.equal(r, results[0]) for r in results)
+
+
+@pytest.mark.parametrize("flow", ["os", "ls", "rs"])
 def test_fp32_long_all_positive_contraction_is_summed_in_blocks(flow):
     """16384 all-positive terms per output: one fp32 accumulator through the whole contraction drifts to about 2e-6 of
     the result (measured, with the vendor library as well); summed in blocks of 128 terms the kernel stays near 2e-7.

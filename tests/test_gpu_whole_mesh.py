@@ -73,6 +73,50 @@ def test_peers_products_check_their_tables():
     assert lib.ms_gemm_ls_peers(None, 32, None, 32, 2, 2, 16, 24, 32, None, 24, 0, 0, ctypes.c_void_p(0)) == _lib.MS_ERR_ARG
 
 
+@pytest.mark.parametrize("flow,P,S", [("ls", 2, 3), ("ls", 4, 1), ("rs", 2, 3), ("rs", 4, 1)])
+@pytest.mark.parametrize("variant", list(range(15)) + [21, 22, 23, 24, 25])
+def test_peers_products_on_every_tile_equal_the_single_devices(variant, flow, P, S):
+    """Every kernel takes both of its operands' pointers by chunk here.  Several tiles each way on the largest shapes
+    (384x192, 256x384), ragged in all extents, a contraction of several stages with a tail; distinct shards and slices,
+    views at pitches wider than their rows.  The same tile gives the same bits for one device's call (ms_gemm_ls_ex /
+    ms_gemm_rs_ex), in both output types, and float64 agrees."""
+    dtype = torch.float32 if variant >= 21 else torch.bfloat16
+    m, n, k = 520, 776, 456 if dtype == torch.bfloat16 else 132
+    g = torch.Generator(device="cuda").manual_seed(variant)
+    wide = lambda r, c: torch.randn(r, c + 16, generator=g, device="cuda").to(dtype)[:, 8:8 + c]
+    if flow == "ls":
+        own, cut = [wide(m, k) for _ in range(P)], [[wide(n, k) for _ in range(S)] for _ in range(P)]
+        single = lambda p, dt: local_gemm.gemm_ls(own[p], cut[p], out_dtype=dt)
+        want = lambda p, s: own[p].double() @ cut[p][s].double().t()
+    else:
+        own, cut = [wide(k, n) for _ in range(P)], [[wide(k, m) for _ in range(S)] for _ in range(P)]
+        single = lambda p, dt: local_gemm.gemm_rs(cut[p], own[p], out_dtype=dt)
+        want = lambda p, s: cut[p][s].double().t() @ own[p].double()
+    lib = _lib.load()
+    bf16 = torch.empty(P * S, m, n, dtype=torch.bfloat16, device="cuda")
+    table = lambda ts: _lib.ptr_array([t.data_ptr() for t in ts])[0]
+    flat = [t for peer in cut for t in peer]
+    try:
+        assert lib.ms_set_variant(variant) == 0
+        got = local_gemm.gemm_ls_peers(own, cut) if flow == "ls" else local_gemm.gemm_rs_peers(cut, own)
+        used = lib.ms_query(_lib.MS_QUERY_LAST_VARIANT)
+        first, second = (own, flat) if flow == "ls" else (flat, own)
+        _lib.check((lib.ms_gemm_ls_peers if flow == "ls" else lib.ms_gemm_rs_peers)(
+            table(first), first[0].stride(0), table(second), second[0].stride(0), P, S, m, n, k, table(bf16.unbind(0)), n,
+            _lib.MS_DTYPE_F32 if dtype == torch.float32 else _lib.MS_DTYPE_BF16, _lib.MS_DTYPE_BF16, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        for p in range(P):
+            each = single(p, torch.float32)
+            for s in range(S):
+                assert torch.equal(got[p][s], each[s])
+                assert torch.equal(bf16[p * S + s], each[s].to(torch.bfloat16))
+                ref = want(p, s)
+                # fp32 accumulation of exact products (bf16) or the fp32 path's 1e-5
+                assert float((got[p][s].double() - ref).norm() / ref.norm()) <= 1e-5
+    finally:
+        lib.ms_set_variant(0)
+    assert variant in (0, used)
+
+
 @pytest.mark.parametrize("flow", ["os", "ls", "rs"])
 def test_a_product_that_fits_memory_only_line_by_line_still_runs(flow):
     """An allowance below what the partial chunks (LS, RS: 512 MiB) or the gathered operands (OS: 128 MiB) of the whole mesh

@@ -255,8 +255,9 @@ def test_the_gated_chunk_calls_check_their_arguments():
 
 
 def test_the_mesh_body_that_launches_the_product_ahead_of_its_gathers_equals_meshflow():
-    """SPMD(mesh, 'meshflow_overlap').OS(K): every device launches its gated product first and fills the gathered slices
-    afterwards on a second stream, slice by slice; the global result equals MeshFlow's bit for bit."""
+    """SPMD(mesh, 'meshflow_overlap').OS(K): the gated product is launched first and the gathered slices are filled
+    afterwards on a second stream, slice by slice; the global result equals MeshFlow's bit for bit.  (A global product of
+    this size is one launch for the whole mesh; single devices' bodies are compared below.)"""
     from meshslice_amd import TensorParallel as TP
     from meshslice_amd.mesh import Mesh, create_device_mesh
     mesh = Mesh(create_device_mesh((2, 2)), ("x", "y"))
@@ -358,4 +359,52 @@ def test_a_product_whose_gathers_do_not_run_beside_it_still_comes_out(gathers, m
     finally:
         lib.ms_set_reserved_cus(0)
     assert len(calls) == (2 if "own" in gathers else 1)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("flow", ["os", "ls", "rs"])
+def test_every_devices_overlapped_body_equals_its_meshflow_body(flow):
+    """One device at a time: two peers' parts are placed in every gathered slice (of both operands, OS) behind one flag."""
+    from meshslice_amd import TensorParallel as TP
+    from meshslice_amd.mesh import Mesh, create_device_mesh
+    mesh = Mesh(create_device_mesh((2, 2)), ("x", "y"))
+    X, W = _overlap_operands(flow)
+    lib = _lib.load()
+    for i in range(2):
+        for j in range(2):
+            lib.ms_set_reserved_cus(TP.OVERLAP_RESERVED_CUS)
+            try:
+                want = getattr(TP.SPMD(mesh, "meshflow"), flow.upper())(4).device(i, j)(X, W)
+            finally:
+                lib.ms_set_reserved_cus(0)
+            got = getattr(TP.SPMD(mesh, "meshflow_overlap"), flow.upper())(4).device(i, j)(X, W)
+            torch.cuda.synchronize()
+            for g, w in zip([got] if flow == "os" else got, [want] if flow == "os" else want, strict=True):
+                assert torch.equal(g, w)
+
+
+@pytest.mark.parametrize("flow", ["ls", "rs"])
+def test_overlapped_chunk_bodies_equal_meshflow_where_the_two_take_different_tiles(flow):
+    """2048 x 4096 x 4096 on 2x2: one launch for the whole mesh takes the 256x384 tile (16x16x32 MFMA), a device's own
+    product a 256x192 one (32x32x16).  Unsplit bf16 products add in the same order on every tile."""
+    from meshslice_amd import TensorParallel as TP
+    from meshslice_amd.mesh import Mesh, create_device_mesh
+    mesh = Mesh(create_device_mesh((2, 2)), ("x", "y"))
+    m, n, k = 2048, 4096, 4096
+    if flow == "ls":
+        X, W = _rand((m, k), 71, torch.bfloat16), _rand((n, k), 72, torch.bfloat16, 0.05)
+    else:
+        X, W = _rand((k, n), 73, torch.bfloat16), _rand((k, m), 74, torch.bfloat16, 0.05)
+    lib = _lib.load()
+    tiles = []
+    lib.ms_set_reserved_cus(TP.OVERLAP_RESERVED_CUS)
+    try:
+        want = getattr(TP.SPMD(mesh, "meshflow"), flow.upper())(4)(X, W)
+        tiles.append(lib.ms_query(_lib.MS_QUERY_LAST_VARIANT))
+    finally:
+        lib.ms_set_reserved_cus(0)
+    got = getattr(TP.SPMD(mesh, "meshflow_overlap"), flow.upper())(4)(X, W)
+    tiles.append(lib.ms_query(_lib.MS_QUERY_LAST_VARIANT))
+    torch.cuda.synchronize()
+    assert tiles[0] != tiles[1]
     assert torch.equal(got, want)
