@@ -581,10 +581,13 @@ int launch_f32_id(int id, bool share, int splits, const Problem &p, const DevFac
 // An output-stationary fp32 product whose tiles leave compute units idle may split its contraction like the bf16 ones
 // (work items = tiles x splits, see split_k_exchange).  The exchange of the partial tiles is priced, in the chooser's
 // unit (the 256 x 128 tile's time per output element and contraction step, 3.5e-6 us), at
-// (F32_SPLIT_FIX + splits x m x n x F32_SPLIT_PER_ELEMENT) / K: about 5 us plus 2 us per million partial elements,
-// fitted to 2048 x 2048 x 8192 (128 tiles of 256 x 128 in two parts: 484 us against 513 us unsplit on 128 x 128) and
-// 1536 x 1536 x 4096 (72 tiles in three parts: 179 us against 224 us on 64 x 64 tiles in three rounds).
-constexpr double F32_SPLIT_FIX = 1.43e6, F32_SPLIT_PER_ELEMENT = 0.6;
+// (F32_SPLIT_FIX + splits x (F32_SPLIT_PART + m x n x F32_SPLIT_PER_ELEMENT)) / K: about 4 us, 0.35 us a part and 2 us per
+// million partial elements.  A part's K loop runs whole summation blocks (four steps of 32): 60 steps in seven parts are
+// twelve steps each, not nine.  Priced as shares of the contraction, 140 x 1360 x 1888 took 64 x 128 in seven parts (23 us)
+// for 64 x 64 in three (five blocks, 19 us), and one product in thirty was more than 2 % slower than on the tiles with ids up
+// to 25 alone.  Fitted to every tile and split count on 400 products from 64 x 256 x 256 to 8192 x 12288 x 12288 (2e10 operations at
+// most): the choice takes 1.006 of the best pair's time in the geometric mean, 1.03 at the 95th percentile (shares: 1.015, 1.09).
+constexpr double F32_SPLIT_FIX = 1.2e6, F32_SPLIT_PART = 1e5, F32_SPLIT_PER_ELEMENT = 0.6;
 constexpr long F32_SPLIT_MIN_K = 256;      // contraction elements per split item, at least
 
 // the fp32 tile, whether its workgroups pair up on the units, and the split count with the lowest estimated cost (id 0: a
@@ -593,6 +596,7 @@ struct F32Pick { int id, splits; bool share; };
 F32Pick pick_f32(const Problem &p, const DevFacts &dev) {
   const long chunks = p.flow == OS ? 1 : p.S;
   const long total_k = (long)p.K * (p.flow == OS ? p.S : 1);
+  const long ksteps = (long)((p.K + 31) / 32) * (p.flow == OS ? p.S : 1);
   const bool forced_tile = g_variant >= F32_FIRST;
   F32Pick best = {0, 1, false};
   double best_cost = 0.0;
@@ -605,13 +609,14 @@ F32Pick pick_f32(const Problem &p, const DevFacts &dev) {
       if (!forced_tile && g_splits != 0) { if (splits > 1) break; }      // (a split forced for the bf16 tiles says nothing here)
       if (splits > 1 && (f32_split_refused(p, dev, t.bm, t.bn, splits) || (!(forced_tile && g_splits != 0) && total_k / splits < F32_SPLIT_MIN_K))) continue;
       const long items = tiles * splits;
-      double cost = (double)((items + dev.cus - 1) / dev.cus) * area / splits;
+      const double item = area * 128.0 * (double)(((ksteps + splits - 1) / splits + 3) / 4) / total_k;      // whole summation blocks
+      double cost = (double)((items + dev.cus - 1) / dev.cus) * item;
       bool share = false;
       if (t.pairs && g_reserved_cus == 0 && items > dev.cus) {
-        const double both = (double)((items + 2L * dev.cus - 1) / (2L * dev.cus)) * area * t.shared / splits;
+        const double both = (double)((items + 2L * dev.cus - 1) / (2L * dev.cus)) * item * t.shared;
         if (both < cost) { cost = both; share = true; }
       }
-      if (splits > 1) cost += (F32_SPLIT_FIX + (double)splits * p.M * p.N * F32_SPLIT_PER_ELEMENT) / total_k;
+      if (splits > 1) cost += (F32_SPLIT_FIX + splits * (F32_SPLIT_PART + (double)p.M * p.N * F32_SPLIT_PER_ELEMENT)) / total_k;
       if (best.id == 0 || cost < best_cost) { best = {t.id, splits, share}; best_cost = cost; }
     }
   }

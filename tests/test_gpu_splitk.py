@@ -103,6 +103,37 @@ def test_fp32_forced_split_matches_oracle_and_is_bit_reproducible(tile, splits):
     assert torch.equal(ms.gemm_os(A, B, out_dtype=torch.bfloat16), got.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("tile,splits,m,n,ks,S", [(26, 4, 700, 904, 4000, 1), (26, 3, 147, 4312, 7216, 1), (26, 7, 359, 912, 2640, 1),
+                                                  (27, 5, 935, 344, 432, 4), (27, 8, 460, 408, 3928, 2), (27, 3, 310, 2104, 1080, 2)])
+def test_fp32_default_split_on_the_narrow_tiles(tile, splits, m, n, ks, S):
+    """64x192 (id 26) and 64x128 (id 27), which only the chooser takes: rows and columns that end inside a tile, K tails,
+    slices that a part crosses.  Against float64, the unsplit product, itself again, and one rounding to bf16."""
+    L = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(100 * tile + splits)
+    A = [torch.randn((m, ks), generator=g, device="cuda") for _ in range(S)]
+    B = [torch.randn((ks, n), generator=g, device="cuda") * 0.05 for _ in range(S)]
+    got = ms.gemm_os(A, B)
+    assert (L.ms_query(_lib.MS_QUERY_LAST_VARIANT), L.ms_query(_lib.MS_QUERY_LAST_SPLITS)) == (tile, splits)
+    want = sum(a.double() @ b.double() for a, b in zip(A, B))
+    assert float((got.double() - want).norm() / want.norm()) <= 1e-5
+    assert orc.rel_frobenius(_f64(got), _f64(_unsplit(A, B))) <= 1e-6
+    for _ in range(3):
+        assert torch.equal(ms.gemm_os(A, B), got)
+    torch.cuda.synchronize()
+    assert int(_counters().abs().sum()) == 0
+    assert torch.equal(ms.gemm_os(A, B, out_dtype=torch.bfloat16), got.to(torch.bfloat16))
+
+
+def test_fp32_split_choice_counts_whole_summation_blocks():
+    """140 x 1360 x 1888: 60 steps in seven parts run twelve steps each.  64x64 in three parts (twenty steps) takes 19 us,
+    64x128 in seven 23 us."""
+    L = _lib.load()
+    A = [torch.randn((140, 944), device="cuda") for _ in range(2)]
+    B = [torch.randn((944, 1360), device="cuda") * 0.05 for _ in range(2)]
+    ms.gemm_os(A, B)
+    assert (L.ms_query(_lib.MS_QUERY_LAST_VARIANT), L.ms_query(_lib.MS_QUERY_LAST_SPLITS)) == (24, 3)
+
+
 def test_fp32_product_of_well_under_one_round_is_split_by_default():
     """1536 x 1536 x 4096 in fp32: 72 tiles of 256x128 (or 576 of 64x64 in three rounds) for 256 compute units."""
     L = _lib.load()
