@@ -130,7 +130,13 @@ def test_a_product_that_fits_memory_only_line_by_line_still_runs(flow):
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(0).total_memory
+    held = []
     try:
+        # what earlier work left free inside the allocator's segments counts as taken
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+        with pytest.raises(torch.OutOfMemoryError):
+            for _ in range(10000):
+                held.append(torch.empty(32 << 20, dtype=torch.uint8, device="cuda"))
         torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (allowance << 20)) / total)
         with pytest.raises(torch.OutOfMemoryError):
             f._whole_mesh(X, W, K, 8)

@@ -408,3 +408,31 @@ def test_overlapped_chunk_bodies_equal_meshflow_where_the_two_take_different_til
     torch.cuda.synchronize()
     assert tiles[0] != tiles[1]
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("tile,flow,m,n,k,S", [(26, "os", 700, 904, 1332, 3), (27, "os", 2047, 2048, 100, 1), (27, "os", 935, 344, 432, 4),
+                                               (26, "ls", 260, 2056, 132, 4), (26, "rs", 260, 2056, 1023, 4),
+                                               (27, "ls", 1500, 520, 132, 4), (27, "rs", 508, 2048, 65, 4)])
+def test_the_narrow_fp32_tiles_behind_the_gate_and_counted(tile, flow, m, n, k, S):
+    """64x192 and 64x128 on products that the chooser gives them (OS: split and unsplit): every flag set, the gated call and
+    the counted chunks equal the plain call's, in both output types."""
+    lib = _lib.load()
+    ready = torch.ones(S + 1, dtype=torch.int32, device="cuda"); ready[S] = 0
+    done = torch.zeros(S, dtype=torch.int32, device="cuda")
+    if flow == "os":
+        A, B = _slices(m, n, k, S, torch.float32, seed=tile)
+        for dt in (torch.float32, torch.bfloat16):
+            want = ms.gemm_os(A, B, out_dtype=dt)
+            got = ms.gemm_os_gated(A, B, ready, out_dtype=dt)
+            assert lib.ms_query(_lib.MS_QUERY_LAST_VARIANT) == tile
+            assert torch.equal(got, want)
+    else:
+        ops, _ = _chunk_operands(flow, m, n, k, S, torch.float32, seed=tile)
+        for dt in (torch.float32, torch.bfloat16):
+            want = _plain(flow, ops, out_dtype=dt)
+            got, tiles = _gated(flow, ops, ready, chunk_done=done.zero_(), out_dtype=dt)
+            assert lib.ms_query(_lib.MS_QUERY_LAST_VARIANT) == tile
+            torch.cuda.synchronize()
+            assert done.tolist() == [tiles] * S and tiles == -(-m // 64) * -(-n // (192 if tile == 26 else 128))
+            assert all(torch.equal(g, w) for g, w in zip(got, want, strict=True))
+    assert not ms.gate_timed_out(ready)
