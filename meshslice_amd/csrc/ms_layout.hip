@@ -27,18 +27,31 @@ long long table_stride(const void *const *tab, int n) {
   return d;
 }
 
-// Rows per thread: one.  A thread then has little in flight by itself, but the launch has eight times the blocks, and these
-// kernels live on loads in flight over the whole device.  S = 4 or 8 slices, eight rows per thread -> one: reducing four
-// peers' fp32 chunks to a bf16 shard of 512 x 256 15.3 -> 3.9 us, 1024 x 768 18.4 -> 5.7, 2048 x 3072 30.2 -> 24.5,
-// 4096 x 12288 171 -> 159; cutting 1024 x 768 bf16 3.3 -> 2.8, 4096 x 12288 35.3 -> 34.2 us.  Eight rows stay for what
-// one row cannot launch (the grid's second extent ends at 65535) and for shards that move element by element, where the
-// two divisions per thread weigh most, once eight rows fill the device (512 blocks, two per compute unit).
+// Rows per thread, 16-byte units: one.  A thread then has little in flight by itself, but the launch has eight times the
+// blocks of eight rows, and these kernels live on loads in flight over the whole device.  S = 4 or 8 slices, eight rows per
+// thread -> one: reducing four peers' fp32 chunks to a bf16 shard of 512 x 256 15.3 -> 3.9 us, 1024 x 768 18.4 -> 5.7,
+// 2048 x 3072 30.2 -> 24.5, 4096 x 12288 171 -> 159; cutting 1024 x 768 bf16 3.3 -> 2.8, 4096 x 12288 35.3 -> 34.2 us.
+// Two for what only moves (a cut, or one peer's chunks) in rows that leave a fifth of their waves' lanes idle, as long as
+// that fills the device (512 blocks, two per compute unit): there the waves to start are what costs (one row, two, eight:
+// 14427 x 72 fp32 cut in three 5.0, 4.3, 4.2 us; 12992 x 232 bf16 cut by rows 5.0, 4.4, 4.4; one peer's 15874 x 352 fp32 9.4,
+// 8.6, 8.4).  Of 409 cuts from 16 x 64 to 16384 x 16384 one in forty is more than 3 % slower than with eight rows; with one row
+// for all it was one in thirteen.
+// Shards that move element by element take the largest count that fills the device: the two divisions per thread weigh most
+// there (254 x 3536 bf16: one row 4.5, four 3.5, eight 3.7 us; 6984 x 7244 fp32 of four peers 304, 190, 190 us).
+// More rows than the grid's second extent covers double the count.
 constexpr int GRID_Y_MAX = 65535, FULL_BLOCKS = 512;
-int rows_per_thread(int rows, int ucols, int tx, bool wide) {
+int rows_per_thread(int rows, int ucols, int tx, bool wide, bool moves) {
   const int rows_per_block = 256 / tx;
-  const long long blocks8 = ((long long)rows + rows_per_block * msk::LAYOUT_RT - 1) / (rows_per_block * msk::LAYOUT_RT) * ((ucols + tx - 1) / tx);
-  const bool fits = ((long long)rows + rows_per_block - 1) / rows_per_block <= GRID_Y_MAX;
-  return fits && (wide || blocks8 < FULL_BLOCKS) ? msk::LAYOUT_RT_SMALL : msk::LAYOUT_RT;
+  const auto blocks_y = [&](int rt) { return ((long long)rows + rows_per_block * rt - 1) / (rows_per_block * rt); };
+  const auto full = [&](int rt) { return blocks_y(rt) * ((ucols + tx - 1) / tx) >= FULL_BLOCKS; };
+  int rt = 1;
+  if (!wide) {
+    for (rt = msk::LAYOUT_RT; rt > 1 && !full(rt);) rt /= 2;
+  } else if (moves && 5LL * ucols < 4LL * ((ucols + 63) / 64 * 64) && full(2)) {
+    rt = 2;
+  }
+  while (rt < msk::LAYOUT_RT && blocks_y(rt) > GRID_Y_MAX) rt *= 2;
+  return rt;
 }
 
 int grid_for(int rows, int ucols, int tx, int rt, dim3 *g, const char *fn) {
@@ -56,8 +69,10 @@ int launch_pack(int axis, int tx, int rt, dim3 g, hipStream_t st, const msk::Pac
     if (axis == 1) hipLaunchKernelGGL((msk::pack_cols_kernel<UB, TX, RT>), g, dim3(256), 0, st, a);      \
     else hipLaunchKernelGGL((msk::pack_rows_kernel<UB, TX, RT>), g, dim3(256), 0, st, a);                \
   }
-  MS_PACK(64, msk::LAYOUT_RT) MS_PACK(128, msk::LAYOUT_RT) MS_PACK(256, msk::LAYOUT_RT)
-  MS_PACK(64, msk::LAYOUT_RT_SMALL) MS_PACK(128, msk::LAYOUT_RT_SMALL) MS_PACK(256, msk::LAYOUT_RT_SMALL)
+  MS_PACK(64, 1) MS_PACK(128, 1) MS_PACK(256, 1)
+  MS_PACK(64, 2) MS_PACK(128, 2) MS_PACK(256, 2)
+  MS_PACK(64, 4) MS_PACK(128, 4) MS_PACK(256, 4)
+  MS_PACK(64, 8) MS_PACK(128, 8) MS_PACK(256, 8)
 #undef MS_PACK
   MS_HIP(hipGetLastError());
   return MS_OK;
@@ -70,8 +85,10 @@ int launch_unpack(int axis, int tx, int rt, dim3 g, hipStream_t st, const msk::U
     if (axis == 1) hipLaunchKernelGGL((msk::unpack_cols_kernel<TIN, TOUT, VEC, TX, RT>), g, dim3(256), 0, st, a);  \
     else hipLaunchKernelGGL((msk::unpack_rows_kernel<TIN, TOUT, VEC, TX, RT>), g, dim3(256), 0, st, a);            \
   }
-  MS_UNPACK(64, msk::LAYOUT_RT) MS_UNPACK(128, msk::LAYOUT_RT) MS_UNPACK(256, msk::LAYOUT_RT)
-  MS_UNPACK(64, msk::LAYOUT_RT_SMALL) MS_UNPACK(128, msk::LAYOUT_RT_SMALL) MS_UNPACK(256, msk::LAYOUT_RT_SMALL)
+  MS_UNPACK(64, 1) MS_UNPACK(128, 1) MS_UNPACK(256, 1)
+  MS_UNPACK(64, 2) MS_UNPACK(128, 2) MS_UNPACK(256, 2)
+  MS_UNPACK(64, 4) MS_UNPACK(128, 4) MS_UNPACK(256, 4)
+  MS_UNPACK(64, 8) MS_UNPACK(128, 8) MS_UNPACK(256, 8)
 #undef MS_UNPACK
   MS_HIP(hipGetLastError());
   return MS_OK;
@@ -119,7 +136,7 @@ MS_API int ms_pack_slices(const void *src, int ld_src, int rows, int cols, int a
   a.S = S;
   a.G = axis == 1 ? B * es / ub : B;
   a.tab_stride = table_stride(dst_slices, S);
-  const int tx = pick_tx(a.ucols), rt = rows_per_thread(rows, a.ucols, tx, wide);
+  const int tx = pick_tx(a.ucols), rt = rows_per_thread(rows, a.ucols, tx, wide, true);
   dim3 g;
   if (int rc = grid_for(rows, a.ucols, tx, rt, &g, fn)) return rc;
   hipStream_t st = (hipStream_t)stream;
@@ -164,7 +181,7 @@ MS_API int ms_unpack_chunks(const void *const *chunks, int P, int S, int ld_chun
   a.S = S;
   a.B = B;
   a.tab_stride = table_stride(chunks, P * S);
-  const int tx = pick_tx(a.ucols), rt = rows_per_thread(rows, a.ucols, tx, wide);
+  const int tx = pick_tx(a.ucols), rt = rows_per_thread(rows, a.ucols, tx, wide, P == 1);
   dim3 g;
   if (int rc = grid_for(rows, a.ucols, tx, rt, &g, fn)) return rc;
   hipStream_t st = (hipStream_t)stream;

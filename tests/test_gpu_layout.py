@@ -261,6 +261,12 @@ def test_layout_calls_reject_bad_arguments():
 ROWS_PER_THREAD_CASES = [(65544, 1056, 2, 8, 1, 1, torch.bfloat16), (65552, 1048, 2, 8, 0, 2, torch.bfloat16), (4101, 1024, 4, 2, 1, 3, torch.bfloat16),
                          (4104, 516, 3, 2, 0, 2, torch.float32), (37, 512, 4, 8, 1, 5, torch.float32), (48, 264, 2, 8, 0, 8, torch.bfloat16)]
 
+# ... two rows per thread (cuts whose rows leave lanes idle, with and without a ragged last group; by rows with blocks that two
+# rows divide and do not), and element-wise shards at two and four
+ROWS_PER_THREAD_CASES += [(4101, 72, 3, 8, 1, 1, torch.float32), (12992, 232, 4, 8, 0, 1, torch.bfloat16), (4098, 232, 2, 3, 0, 1, torch.bfloat16),
+                          (511, 1048, 2, 2, 1, 2, torch.bfloat16), (401, 520, 2, 2, 1, 5, torch.float32), (252, 3588, 2, 3, 0, 3, torch.bfloat16),
+                          (131084, 1048, 2, 2, 0, 1, torch.bfloat16)]
+
 
 @pytest.mark.parametrize("r,c,S,B,axis,P,dtype", ROWS_PER_THREAD_CASES)
 def test_every_count_of_rows_per_thread_moves_every_element_once(r, c, S, B, axis, P, dtype):
