@@ -227,6 +227,22 @@ def test_unsplit_bf16_products_have_the_same_bits_on_every_tile(m, n, k, flow):
     assert all(torch.equal(r, results[0]) for r in results)
 
 
+@pytest.mark.parametrize("flow", ["ls", "rs"])
+def test_unsplit_fp32_products_have_the_same_bits_on_every_tile(flow):
+    """Every fp32 tile sums blocks of 128 contraction elements and adds the blocks in order."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda") * torch.exp(4 * torch.randn(s, generator=g, device="cuda"))
+    m, n, k = 520, 776, 1000
+    a, b = (rnd(m, k), rnd(n, k)) if flow == "ls" else (rnd(k, m), rnd(k, n))
+    run = lambda: ms.gemm_ls(a, [b])[0] if flow == "ls" else ms.gemm_rs([a], b)[0]
+    lib = _lib.load()
+    results = []
+    for v in (21, 22, 23, 24, 25):
+        _lib.check(lib.ms_set_variant(v))
+        results.append(run())
+    assert all(torch.equal(r, results[0]) for r in results)
+
+
 @pytest.mark.parametrize("flow", ["os", "ls", "rs"])
 def test_fp32_long_all_positive_contraction_is_summed_in_blocks(flow):
     """16384 all-positive terms per output: one fp32 accumulator through the whole contraction drifts to about 2e-6 of
