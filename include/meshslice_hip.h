@@ -55,7 +55,8 @@ extern "C" {
                                    would leave much of the last round of compute units idle is done in two launches) */
 #define MS_QUERY_LAST_SPLITS 7   /* ways in which that launch split the contraction (1: not split) */
 #define MS_QUERY_LAST_VARIANT 6  /* kernel variant (tile shape, see ms_set_variant) of the first of those launches: 1..14 for
-                                   the bf16 kernels, 21..27 for the fp32 kernel.  Lets a measurement name the kernel it timed. */
+                                   the bf16 kernels, 21..27 for the fp32 kernel (26, 27: 64x192 and 64x128, which only the library's choice
+                                   takes).  Lets a measurement name the kernel it timed. */
 #define MS_QUERY_LAST_GRID 8     /* workgroups of the first of those launches: the compute units it ran on (at most the
                                    device's, less the reserved ones; fewer when that fills every round of the launch) */
 
@@ -325,7 +326,7 @@ int ms_probe_mfma_stream(const void *operands, float *sink, int iters, int warmu
                          float *ms_out, double *flops_per_launch, void *stream);
 
 /* Measurement aid (no counterpart in the reference): the output-stationary 256x384x64 kernel on the 16x16x32 MFMA
- * (bf16 in, bf16 out; what ms_gemm_os runs on BASELINE's configuration 2) with parts of its K loop left out, timed on
+ * (bf16 in, bf16 out; what ms_gemm_os runs on a 4096 x 12288 x 12288 product) with parts of its K loop left out, timed on
  * the caller's operands: what a part costs is the difference to skip = 0 on the same data, tile loop and clock.
  * skip (one of the built combinations 0, 1, 2, 3, 4, 8, 16, 24) is a sum of
  *   1  no global -> LDS loads inside the K loop (the stage buffers keep the tile's first two stages),
@@ -353,7 +354,7 @@ int ms_probe_l2_lds_stream(const void *buffer, size_t buffer_bytes, int region_s
  * (1..14, 0 = the library's choice) and split the contraction `variant / 100` ways (2..8, 0 = the library's choice;
  * a forced split needs a workspace and an output-stationary product).  21..25 name the fp32 kernel's tiles instead
  * (256x128, 128x192, 128x128, 64x64, 192x192; split counts as above): fp32 calls then use that tile and bf16 calls the library's choice,
- * as fp32 calls do under 1..14.  Unknown ids are rejected with MS_ERR_ARG. */
+ * as fp32 calls do under 1..14.  Unknown ids are rejected with MS_ERR_ARG, 26 and 27 (MS_QUERY_LAST_VARIANT) among them. */
 int ms_set_variant(int variant);
 
 /* Compute units that the GEMM launches of the calling thread leave free (default 0; returns MS_ERR_ARG outside

@@ -97,7 +97,8 @@ def _gather_col_slices(peers: Sequence[torch.Tensor], K: int, B: int) -> List[to
     gathered slice k (all_gather over the peers' axis, tiled along the columns).  One kernel per peer writes
     its K slices straight into their places; there is no separate concatenation.  A shard is a whole number of rounds of
     K blocks, so peers that lie side by side in one matrix are cut by one kernel: the block-cyclic slices of the whole
-    are the peers' slices side by side (the LS body of one device of a 2x4 mesh, 4096 x 4096 x 8192 in eight slices: 130 -> 91 us)."""
+    are the peers' slices side by side (the LS body of one device of a 2x4 mesh, 4096 x 4096 x 8192 in eight slices,
+    128 -> 72 us, cheaper calls included)."""
     r, c = peers[0].shape
     _need(c, K * B, "sliced extent")
     w = c // K
@@ -278,7 +279,8 @@ def MeshFlow_OS_overlap(X, W, i, j, R, C, K, B):
     """MeshFlow_OS in the order the reference's schedule runs it (:163-171): the product is launched once, before any
     slice has arrived, and multiplies slice k while the gathers of the later slices are still under way
     (``gemm_os_gated``).  The emulated gather stream fills slice k of both operands, peer by peer, and raises flag k.
-    Same result as MeshFlow_OS, bit for bit."""
+    Same result as MeshFlow_OS on the compute units left to it, bit for bit, where that is one launch split the same way (a
+    gated product is never done in two)."""
     if K == 1:
         raise ValueError("the sliced OS body is undefined for K == 1 (the reference adds slice 0 twice); "
                          "use algorithm='collective' for the unsliced product")
@@ -446,8 +448,9 @@ def _finish(chunks_by_peer, me, axis, B, dtype):
 # the whole mesh at once.  On the one GPU that plays every device, the devices of a mesh row or column receive the same
 # gathered slices, and their products differ only in which rows and columns of them they take: one kernel gathers an operand
 # for all of them (see _spanning), one product covers them all.  Device by device a training step of a small layer is some
-# 150 launches of 2 to 40 us, bound by the host that issues them: 512 x 256 x 1024 on a 4x2 mesh 3.6 ms, in this way 0.48;
-# 2048 x 3072 x 12288 on a 2x4 mesh 5.1 ms, in this way 0.62.
+# 150 launches of 2 to 40 us, bound by the host that issues them: 512 x 256 x 1024 on a 4x2 mesh 3.7 ms, in this way 0.40;
+# 2048 x 3072 x 12288 on a 2x4 mesh 5.1 ms, in this way 0.56.  The price is memory: gathered operands and partial chunks of
+# all mesh lines are alive at once, where device by device it is one line's.
 # ------------------------------------------------------------------------------------------------
 
 WHOLE_MESH_MAX_CHUNK_BYTES = 4 << 30      # partial chunks alive at once; device by device it is one mesh line's

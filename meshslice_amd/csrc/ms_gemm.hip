@@ -93,7 +93,7 @@ namespace {
 thread_local int g_variant = 0;
 thread_local int g_splits = 0;    // forced split count of the contraction (0 = library default)
 thread_local int g_launches = 0;   // kernels launched by the last GEMM call of this thread
-thread_local int g_last_variant = 0;   // kernel variant of that call's first launch (bf16 tiles 1..VARIANTS, fp32 tiles F32_FIRST..F32_LAST)
+thread_local int g_last_variant = 0;   // kernel variant of that call's first launch (bf16 tiles 1..VARIANTS, fp32 tiles F32_FIRST..F32_NARROW + 1)
 thread_local int g_last_splits = 1;    // and the number of ways it split the contraction
 thread_local int g_last_grid = 0;      // and its workgroup count
 thread_local int g_reserved_cus = 0;   // compute units the GEMM launches of this thread leave free (ms_set_reserved_cus)
@@ -136,7 +136,7 @@ enum Flow { OS = 0, LS = 1, RS = 2 };
 // One local contraction, in kernel terms.
 struct Problem {
   Flow flow;
-  const void *const *a;  // nkslices (OS) or nchunks (RS) or 1 pointers
+  const void *const *a;  // nkslices (OS), nchunks (the operand cut into chunks, and both in several devices' calls) or 1 pointers
   const void *const *b;
   void *const *c;
   int na, nb, nc;
@@ -319,7 +319,7 @@ struct Pick { int v, splits; double cost; };
 
 constexpr int VARIANTS = 14;
 constexpr int F32_FIRST = 21, F32_LAST = 25;      // ids of the fp32 kernel's tiles (ms_set_variant, MS_QUERY_LAST_VARIANT)
-constexpr int F32_NARROW = 26;                    // and of the two that only the chooser takes (64 x 192, 64 x 128)
+constexpr int F32_NARROW = 26;                    // and of the two that only the chooser takes (64 x 192, 64 x 128; not ms_set_variant)
 struct TileShape { int bm, bn; };
 constexpr TileShape TILE_OF[VARIANTS + 1] = {{0, 0},     {256, 256}, {256, 256}, {128, 128}, {256, 256}, {256, 192},
                                              {192, 256}, {256, 256}, {256, 192}, {192, 256}, {256, 384}, {384, 192},

@@ -2,7 +2,7 @@
 
 Three probes, each a thin wrapper over one C entry point, and a command line that prints them as one JSON object:
 
-* ``os_parts``: BASELINE's configuration 2 (or any output-stationary bf16 product) on the 256x384x64 kernel of the
+* ``os_parts``: the 4096 x 12288 x 12288 product (or any output-stationary bf16 product) on the 256x384x64 kernel of the
   16x16x32 MFMA with parts of its K loop left out (``ms_probe_os_parts``): the whole kernel, without its global -> LDS
   loads, without its fragment reads, the MFMAs alone, the operand stream alone, without the wait / the barrier of a
   K step;
