@@ -26,9 +26,9 @@
   template __global__ void msk::gemm_bf16_ring_kernel<BM, BN, BK, NS, WGM, WGN, false, false, false, false>(const msk::GemmArgs); \
   template __global__ void msk::gemm_bf16_ring_kernel<BM, BN, BK, NS, WGM, WGN, false, false, true, false>(const msk::GemmArgs);
 MS_INSTANTIATE_RING(256, 256, 64, 2, 2, 2)
-MS_INSTANTIATE_RING(256, 256, 32, 4, 2, 4)
+MS_INSTANTIATE_RING(192, 192, 64, 3, 2, 2)
 MS_INSTANTIATE_RING(128, 128, 64, 2, 2, 2)
-MS_INSTANTIATE_RING(256, 256, 32, 4, 2, 2)
+MS_INSTANTIATE_RING(128, 192, 64, 3, 2, 2)
 MS_INSTANTIATE_RING(256, 192, 32, 4, 2, 2)
 MS_INSTANTIATE_RING(192, 256, 32, 4, 2, 2)
 MS_INSTANTIATE_RING(256, 256, 64, 2, 2, 4)
@@ -294,46 +294,46 @@ int launch_bf16_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, 
 }
 
 // Kernel variants (tile, waves, ring stages x k-elements per stage):
-//   1: 256x256, 4 waves, 2 x 64     2: 256x256, 8 waves, 4 x 32     3: 128x128, 4 waves, 2 x 64
-//   4: 256x256, 4 waves, 4 x 32     5: 256x192, 4 waves, 4 x 32     6: 192x256, 4 waves, 4 x 32
+//   1: 256x256, 4 waves, 2 x 64     2: 192x192, 4 waves, 3 x 64     3: 128x128, 4 waves, 2 x 64
+//   4: 128x192, 4 waves, 3 x 64     5: 256x192, 4 waves, 4 x 32     6: 192x256, 4 waves, 4 x 32
 //   7: 256x256, 8 waves, 2 x 64     8: 256x192, 4 waves, 2 x 64     9: 192x256, 4 waves, 2 x 64
 //  10: 256x384, 4 waves, 2 x 64 (gemm_bf16_big_kernel<4, 6>)     11: 384x192, 4 waves, 2 x 64 (gemm_bf16_big_kernel<6, 3>)
 //  12: 256x384, 4 waves, 2 x 64 on the 16x16x32 MFMA (gemm_bf16_x16_kernel)     13: 256x256, the same kernel
 //  14: 128x128, 4 waves, 3 x 64 (one workgroup per unit: for products of at most one round of such tiles, where a third
 //      stage covers the load latency that two 64-deep stages do not: 2048^3 in 20.7 us against 26.3 us, 1536^3 14.7 against 18.8)
-// The default picks the tile shape that wastes the least of the machine: a launch runs in
-// ceil(work items / CUs) rounds of one item per CU (a partly filled last round is charged in part, see
-// balanced_grid), so the estimate is rounds x tile area / relative tile
-// efficiency (measured on the GPT-3-sized products, per flop, 256x256 = 1: the 256x384 tile, on the 16x16x32 kernel
-// that every such pick runs on, reaches 1.15 (OS) / 1.20 (LS) with a k-contiguous A and 1.16 without, the 384x192 tile 1.04,
-// 192-wide ring tiles about 0.93, 128x128 tiles about 0.55, or 0.42 per workgroup with two of them on a unit).  The ring-kernel defaults use four waves over two 64-deep stages when an operand is
-// k-contiguous: whole 128-byte lines per request, half as many barriers as 32-deep stages.
+//      2 and 4 are for outputs of one or two hundred such tiles, where 128x128 pays for more operand bytes per FLOP and
+//      256-wide tiles leave units idle: 2048 x 3072 x 4096 on 128x192 43 us, 128x128 50, 256x192 61; 3072^3 on 192x192 48 us, 256x192
+//      52; 1499 x 4104 x 3096 on 192x192 46 us, 128x128 57.  (128x256, 256x128 and 192x128 as well would give another 0.3 % over drawn products.)
+// The default picks the tile shape that wastes the least of the machine: a launch runs in ceil(work items / CUs) rounds of
+// one item per CU (a partly filled last round is charged in part, see balanced_grid), so the estimate is rounds x tile area x
+// (contraction + a tile's overhead) / the tile's rate (TILE_RATES).  With two m/n-contiguous operands (RS) the 192-wide ring tiles
+// do best on four 32-deep stages, else on two 64-deep ones: whole 128-byte lines per request, half as many barriers.
 //
 // An output-stationary product with fewer tiles than compute units may split its contraction (work items = tiles x
 // splits, see split_k_exchange): a split item costs 1 / splits of the tile, and the whole launch pays for the exchange
 // of partial tiles, which is bound by memory bandwidth (splits x m x n fp32 values written through to memory and read
 // back: about 2.8 TB/s) plus a fixed few microseconds.  In the estimate's units (tile area x share of the contraction,
-// one compute unit doing about 5.7 TFLOP/s) that is (SPLIT_FIX + splits x m x n x SPLIT_PER_ELEMENT) / K.  Measured on
-// 2048 x 1536 x 12288 (64 tiles of 256x192): 170 us unsplit, 100 / 85 / 88 us with 2 / 3 / 4 splits.
+// one compute unit doing about 5.7 TFLOP/s) that is (SPLIT_FIX + splits x (SPLIT_PER_PART + m x n x SPLIT_PER_ELEMENT)) / K.
+// Measured on 2048 x 1536 x 12288: 80 us unsplit on 192 tiles of 128x128, 73 on 128 of 128x192 in two parts, 79 on 64 of 256x192 in four.
 struct Pick { int v, splits; double cost; };
 
 constexpr int VARIANTS = 14;
 constexpr int F32_FIRST = 21, F32_LAST = 25;      // ids of the fp32 kernel's tiles (ms_set_variant, MS_QUERY_LAST_VARIANT)
 constexpr int F32_NARROW = 26;                    // and of the two that only the chooser takes (64 x 192, 64 x 128; not ms_set_variant)
 struct TileShape { int bm, bn; };
-constexpr TileShape TILE_OF[VARIANTS + 1] = {{0, 0},     {256, 256}, {256, 256}, {128, 128}, {256, 256}, {256, 192},
+constexpr TileShape TILE_OF[VARIANTS + 1] = {{0, 0},     {256, 256}, {192, 192}, {128, 128}, {128, 192}, {256, 192},
                                              {192, 256}, {256, 256}, {256, 192}, {192, 256}, {256, 384}, {384, 192},
                                              {256, 384}, {256, 256}, {128, 128}};
-// unsplit 256x256: the 16x16x32 kernel (variant 13) against the eight-wave ring kernel (variant 7); with two m/n-contiguous
-// operands (RS) it gains 0-6 % only, and beyond some 6000 contraction elements per chunk it loses (10240 x 2560 x 12288 in
-// two chunks: 0.622 against 0.555 ms), so there the ring kernel stays
-constexpr double X16_OVER_RING_256 = 1.10, X16_OVER_RING_256_LS = 1.13, X16_OVER_RING_256_RS = 1.03;
+// unsplit 256x256 is the 16x16x32 kernel (variant 13), split the eight-wave ring kernel (variant 7); with two m/n-contiguous operands (RS)
+// the former loses beyond some 6000 contraction elements per chunk (10240 x 2560 x 12288 in two chunks: 0.622 against 0.555 ms),
+// so there the ring kernel stays
 constexpr int X16_RS_MAX_K = 6144;
 constexpr int SPLIT_CHOICES[] = {1, 2, 3, 4, 6, 8};
 constexpr int SPLIT_MAX = 8;
-constexpr long SPLIT_MIN_K = 512;            // contraction elements per split item, at least
-constexpr double SPLIT_FIX = 1.4e7;          // fixed cost of an exchange (about 5 us)
-constexpr double SPLIT_PER_ELEMENT = 8.2;    // per split and output element (8 bytes through memory)
+constexpr long SPLIT_MIN_K = 256;            // contraction elements per split item, at least
+constexpr double SPLIT_FIX = 1.3e7;          // fixed cost of an exchange (about 4 us),
+constexpr double SPLIT_PER_PART = 1.3e6;     // per part (half a microsecond: the last arriver reads the parts one after the other),
+constexpr double SPLIT_PER_ELEMENT = 7.9;    // per part and output element (8 bytes through memory)
 
 const char *const SPLIT_REFUSALS[] = {"", "only output-stationary products split their contraction", "no workspace was given",
                                       "more work items than compute units", "too many output tiles for the workspace's counters",
@@ -345,7 +345,7 @@ const char *const SPLIT_REFUSALS[] = {"", "only output-stationary products split
 int split_refused(const Problem &p, const DevFacts &dev, int v, int splits) {
   const int bm = TILE_OF[v].bm, bn = TILE_OF[v].bn;
   if (splits < 2 || splits > SPLIT_MAX) return 7;
-  if (v == 1 || v == 4 || v == 12 || v == 13) return 8;     // 256x256 on four waves: see ring_can_split; the 16x16x32 kernels have none
+  if (v == 1 || v == 12 || v == 13) return 8;     // 256x256 on four waves: see ring_can_split; the 16x16x32 kernels have none
   if (p.act || p.res || p.row_sum || p.row_sumsq) return 9;   // see ring_can_split, big_can_split
   if (p.flow != OS) return 1;
   if (!p.ws) return 2;
@@ -357,45 +357,52 @@ int split_refused(const Problem &p, const DevFacts &dev, int v, int splits) {
   return 0;
 }
 
+// Relative rates of the tiles as the chooser prices them, by dataflow (256x256 on the eight-wave ring kernel of an OS product = 1): `os`,
+// `ls`, `rs` for an unsplit product (128x128 in two stages: a unit that holds one workgroup, PAIRED_* per workgroup where two
+// share it; 7 and 10 stand for 13 and 12), `split` for a split one; 0: not for that dataflow.  Fitted, with the constants above and
+// below, to every tile and split count forced on 580 drawn products (m 64 to 8192, n and k 256 to 12288, one to sixteen slices, half of
+// them at pitches that are no whole lines): the choice takes 1.024 (OS), 1.008 (LS), 1.007 (RS) of the best pair's time in the geometric
+// mean and 1.13, 1.04, 1.03 at the 95th percentile; before this fit, and without tiles 2 and 4, 1.046, 1.026, 1.031 and 1.21, 1.14, 1.18.
+struct TileRate { int v; double os, ls, rs, split; };
+constexpr TileRate TILE_RATES[] = {{7, 1.11, 1.065, 0.945, 1.0}, {10, 1.2, 1.146, 1.076, 1.14}, {11, 0.98, 0.939, 0.986, 0.98}, {8, 0.93, 0.972, 0.0, 0.93},
+                                   {9, 0.95, 0.972, 0.0, 0.95}, {5, 0.0, 0.0, 0.994, 0.0}, {6, 0.0, 0.0, 0.959, 0.0}, {3, 0.486, 0.458, 0.5, 0.486},
+                                   {14, 0.66, 0.706, 0.69, 0.66}, {4, 0.795, 0.814, 0.86, 0.795}, {2, 0.93, 0.938, 0.96, 0.93}};
+constexpr double PAIRED_OS = 0.38, PAIRED_LS = 0.424, PAIRED_RS = 0.424;
+// prologue and write-out of a tile, as contraction elements
+constexpr double TILE_OVERHEAD_K = 80.0;
+// what a tile loses of a last round that is partly filled: units idle then let the others clock higher, but only on the tiles that
+// reach the power limit
+double partial_round_loss(int v) { return v == 3 || v == 14 ? 1.0 : v == 2 || v == 4 ? 0.87 : PARTIAL_ROUND_LOSS; }
+
 // the tile shape and split count with the lowest estimated cost for the whole problem
 Pick pick_variant(const Problem &p, const DevFacts &dev) {
-  struct Cand { int v; double eff; };
-  // with two m/n-contiguous operands (RS) the hand-scheduled tiles gain less over the 256x256 ring than with a
-  // k-contiguous operand, and the 192-wide ring tiles do best on four 32-deep stages
-  // (256x256 runs on eight waves, two per SIMD: 1-3 % faster than four waves, 10-15 % on short contractions, where
-  // prologue and write-out weigh most, and the one of the two that can split its contraction: 2048 x 2048 x 16384 in
-  // 0.125 ms on 64 tiles x 4 splits, 0.165 ms on 256 tiles of 128x128; four waves stay selectable as variant 1)
   const bool rs = p.flow == RS, ls = p.flow == LS;
-  const Cand cands[] = {{7, 1.0}, {10, rs ? 1.16 : ls ? 1.20 : 1.15}, {11, 1.04}, {rs ? 5 : 8, rs ? 0.95 : 0.93}, {rs ? 6 : 9, rs ? 0.95 : 0.93}, {3, workgroups_per_unit(3) == 2 ? 0.42 : 0.55}, {14, 0.66}};
   const long chunks = p.flow == OS ? 1 : p.S;
   const double total_k = p.flow == OS ? (double)p.K * p.S : (double)p.K;
   Pick best = {0, 1, 0};
-  for (const Cand &c : cands) {
+  for (const TileRate &c : TILE_RATES) {
     const int bm = TILE_OF[c.v].bm, bn = TILE_OF[c.v].bn;
+    const bool pairs = workgroups_per_unit(c.v) == 2;
+    const double rate = rs ? c.rs : ls ? c.ls : c.os;
     const long tiles = (long)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * chunks;
     for (int splits : SPLIT_CHOICES) {
       if (g_splits != 0 && splits != g_splits) continue;
+      if (splits == 1 ? rate == 0.0 : c.split == 0.0) continue;
       if (splits > 1 && (split_refused(p, dev, c.v, splits) || (g_splits == 0 && total_k / splits < SPLIT_MIN_K))) continue;
       // rounds the launch is charged: whole ones, or with the last round partly filled (see balanced_grid) its filled
-      // share plus PARTIAL_ROUND_LOSS of the rest
-      const long slots = (long)dev.cus * (splits == 1 ? workgroups_per_unit(c.v) : 1);     // (a split launch is one item per unit)
+      // share plus a part of the rest; a launch of less than one round is charged the same way, down to 0.7 of a round (the
+      // idle units' power lets the busy ones clock up to 1.4 times higher)
+      const long slots = (long)dev.cus * (splits == 1 && pairs ? 2 : 1);     // (a split launch is one item per unit)
       const double exact = (double)(tiles * splits) / slots;
       const double whole = (double)((tiles * splits + slots - 1) / slots);
-      // (the 128x128 kernels do not reach the power limit: their units gain no clock from idle neighbours)
-      const bool small_tile = c.v == 3 || c.v == 14;
-      const double loss = small_tile ? 1.0 : PARTIAL_ROUND_LOSS;
-      // (a launch of less than one round is charged the same way, down to 0.7 of a round: the idle units' power lets the
-      // busy ones clock up to 1.4 times higher)
+      const double loss = partial_round_loss(c.v);
       const double part = exact + loss * (1.0 - exact);
       const double rounds = exact <= 1.0 ? (part > 0.7 ? part : 0.7) : exact + loss * (whole - exact);
-      const double exchange = splits == 1 ? 0.0 : (SPLIT_FIX + (double)splits * p.M * p.N * SPLIT_PER_ELEMENT) / total_k;
-      // (a split 256x384 product stays on the 32x32x16 kernel, which carries the exchange and is about 5 % slower; an
-      // unsplit 256x256 one runs on the 16x16x32 kernel, 7-14 % faster than the eight-wave ring kernel that carries the split)
-      // (two 128x128 workgroups share a unit only where there are more tiles than units: 0.55 alone, 0.42 each when every
-      // unit holds two)
-      const double shared = c.v == 3 && workgroups_per_unit(3) == 2 ? (tiles * splits <= dev.cus ? 0.0 : tiles * splits >= 2L * dev.cus ? 1.0 : (double)(tiles * splits - dev.cus) / dev.cus) : 0.0;
-      const double eff = c.v == 3 && workgroups_per_unit(3) == 2 ? 0.55 - 0.13 * shared : c.v == 10 && splits > 1 ? c.eff / 1.05 : c.v == 7 && splits == 1 ? c.eff * (ls ? X16_OVER_RING_256_LS : !rs ? X16_OVER_RING_256 : p.K <= X16_RS_MAX_K ? X16_OVER_RING_256_RS : 1.0) : c.eff;
-      const double cost = rounds * bm * bn / eff / splits + exchange;
+      const double exchange = splits == 1 ? 0.0 : SPLIT_FIX + splits * (SPLIT_PER_PART + (double)p.M * p.N * SPLIT_PER_ELEMENT);
+      // (two 128x128 workgroups share a unit only where there are more tiles than units)
+      const double shared = !pairs || tiles * splits <= dev.cus ? 0.0 : tiles * splits >= 2L * dev.cus ? 1.0 : (double)(tiles * splits - dev.cus) / dev.cus;
+      const double eff = splits > 1 ? c.split : rate - (pairs ? (rate - (rs ? PAIRED_RS : ls ? PAIRED_LS : PAIRED_OS)) * shared : 0.0);
+      const double cost = (rounds * bm * bn / eff * (total_k / splits + TILE_OVERHEAD_K) + exchange) / total_k;
       if (best.v == 0 || cost < best.cost) best = {c.v, splits, cost};
     }
   }
@@ -412,13 +419,13 @@ Pick pick_variant(const Problem &p, const DevFacts &dev) {
 }
 
 int launch_variant(int v, int splits, const Problem &p, const DevFacts &dev, hipStream_t stream) {
-  if (p.slice_ready && (v == 1 || v == 4)) return fail(MS_ERR_UNSUPPORTED, "tile variant %d has no input gate (256x256 on four waves of the ring kernel)", v);
+  if (p.slice_ready && v == 1) return fail(MS_ERR_UNSUPPORTED, "tile variant %d has no input gate (256x256 on four waves of the ring kernel)", v);
   if (g_launches == 0) { g_last_variant = v; g_last_splits = splits; }
   switch (v) {
     case 1: return launch_bf16_tile<256, 256, 2, 2, 64, 2>(p, dev, stream, 1, splits);
-    case 2: return launch_bf16_tile<256, 256, 2, 4, 32, 4>(p, dev, stream, 2, splits);
+    case 2: return launch_bf16_tile<192, 192, 2, 2, 64, 3>(p, dev, stream, 2, splits);
     case 3: return launch_bf16_tile<128, 128, 2, 2, 64, 2>(p, dev, stream, 3, splits);
-    case 4: return launch_bf16_tile<256, 256, 2, 2, 32, 4>(p, dev, stream, 4, splits);
+    case 4: return launch_bf16_tile<128, 192, 2, 2, 64, 3>(p, dev, stream, 4, splits);
     case 5: return launch_bf16_tile<256, 192, 2, 2, 32, 4>(p, dev, stream, 5, splits);
     case 6: return launch_bf16_tile<192, 256, 2, 2, 32, 4>(p, dev, stream, 6, splits);
     case 7: return launch_bf16_tile<256, 256, 2, 4, 64, 2>(p, dev, stream, 7, splits);
@@ -446,7 +453,7 @@ int launch_bf16(const Problem &p, const DevFacts &dev, hipStream_t stream) {
   // (a gated product stays one launch: a second one would stand in the stream behind the first while that waits for slices)
   if (p.flow == OS && single.splits == 1 && g_splits == 0 && !p.slice_ready) {
     constexpr int BM = 256, BN = 384;
-    constexpr double EFF = 1.15;
+    constexpr double EFF = 1.2;      // (TILE_RATES)
     const long tiles_m = (p.M + BM - 1) / BM;
     const long total_k = (long)p.K * p.S;
     // whole rounds of the big tile: the largest count of leading tile columns whose tiles are a multiple of the CUs
@@ -459,7 +466,7 @@ int launch_bf16(const Problem &p, const DevFacts &dev, hipStream_t stream) {
       rest.ws = nullptr;   // the second launch is not split: the first may still be using the workspace's counters
       const Pick tail = pick_variant(rest, dev);
       const double second_launch = 3.4e7 / (double)total_k;      // ~12 us at the rate one CU computes tile area x K
-      const double cost = (double)(tiles_m * nb1 / dev.cus) * BM * BN / EFF + tail.cost + second_launch;
+      const double cost = (double)(tiles_m * nb1 / dev.cus) * BM * BN / EFF * (1.0 + TILE_OVERHEAD_K / (double)total_k) + tail.cost + second_launch;
       if (cost < 0.97 * single.cost) {
         const int es_in = 2, es_out = p.out_dtype == MS_DTYPE_BF16 ? 2 : 4;
         Problem head = p;
@@ -866,7 +873,7 @@ MS_API int ms_gemm_os_noalloc(const void *const *A_slices, const void *const *B_
   if (rc) return rc;
   // what the library would do with room to spare decides whether the built-in scratch is needed, and whether it is enough
   p.ws = reinterpret_cast<void *>(uintptr_t(256));    // stands for "a workspace": only its size is looked at here
-  p.ws_bytes = ~size_t(0);
+  p.ws_bytes = g_variant ? ~size_t(0) : NOALLOC_SCRATCH_BYTES;      // (the library's own choice is one that fits)
   int splits = 1, bm = 0, bn = 0;
   if (in_dtype == MS_DTYPE_BF16) {
     const Pick want = g_variant >= 1 && g_variant <= VARIANTS ? Pick{g_variant, g_splits > 1 ? g_splits : 1, 0.0} : pick_variant(p, usable(*dev));
