@@ -55,7 +55,7 @@ extern "C" {
                                    would leave much of the last round of compute units idle is done in two launches) */
 #define MS_QUERY_LAST_SPLITS 7   /* ways in which that launch split the contraction (1: not split) */
 #define MS_QUERY_LAST_VARIANT 6  /* kernel variant (tile shape, see ms_set_variant) of the first of those launches: 1..14 for
-                                   the bf16 kernels, 21..27 for the fp32 kernel (26, 27: 64x192 and 64x128, which only the library's choice
+                                   the bf16 kernels (15, 16, 17: the tiles 14, 4, 2 of ms_gemm_ls_sum and ms_gemm_rs_sum), 21..27 for the fp32 kernel (26, 27: 64x192 and 64x128, which only the library's choice
                                    takes).  Lets a measurement name the kernel it timed. */
 #define MS_QUERY_LAST_GRID 8     /* workgroups of the first of those launches: the compute units it ran on (at most the
                                    device's, less the reserved ones; fewer when that fills every round of the launch) */
@@ -186,6 +186,19 @@ int ms_gemm_ls_peers(const void *const *A, int lda, const void *const *W_slices,
 int ms_gemm_rs_peers(const void *const *X_slices, int ldx, const void *const *W, int ldw, int P, int S,
                      int m_slice, int n, int k,
                      void *const *Y_chunks, int ldy, int in_dtype, int out_dtype, void *stream);
+
+/* What the P devices of a mesh line hold between them after their reduce-scatter, in one launch and without the partial
+ * chunks: C = sum_p A[p] @ W[p]^T (LS: A[p] [m,k], W[p] [n,k]) or sum_p X[p]^T @ W[p] (RS: X[p] [k,m], W[p] [k,n]), where
+ * table entry p is device p's shard of the contraction.  Every device's partial sum is accumulated by itself in fp32 and they are
+ * added up in fp32 in table order, then rounded once: the bits of ms_gemm_*_peers followed by ms_unpack_chunks.  bf16
+ * operands and results only (MS_ERR_UNSUPPORTED otherwise); 1 <= P <= MS_MAX_SLICES.  workspace as for ms_gemm_os_ws, or
+ * null: with one, few output tiles are worked on by one workgroup per device. */
+int ms_gemm_ls_sum(const void *const *A, int lda, const void *const *W, int ldw, int P, int m, int n, int k,
+                   void *C, int ldc, int in_dtype, int out_dtype,
+                   void *workspace, size_t workspace_bytes, void *stream);
+int ms_gemm_rs_sum(const void *const *X, int ldx, const void *const *W, int ldw, int P, int m, int n, int k,
+                   void *C, int ldc, int in_dtype, int out_dtype,
+                   void *workspace, size_t workspace_bytes, void *stream);
 
 /* ms_gemm_ls_ex / ms_gemm_rs_ex with completion counters, so that the reduce-scatter of chunk s (the psum_scatter that
  * follows each einsum in MeshFlow_LS / MeshFlow_RS, TensorParallel.py:182-189, :204-212) can start while the later
@@ -354,7 +367,9 @@ int ms_probe_l2_lds_stream(const void *buffer, size_t buffer_bytes, int region_s
  * (1..14, 0 = the library's choice) and split the contraction `variant / 100` ways (2..8, 0 = the library's choice;
  * a forced split needs a workspace and an output-stationary product).  21..25 name the fp32 kernel's tiles instead
  * (256x128, 128x192, 128x128, 64x64, 192x192; split counts as above): fp32 calls then use that tile and bf16 calls the library's choice,
- * as fp32 calls do under 1..14.  Unknown ids are rejected with MS_ERR_ARG, 26 and 27 (MS_QUERY_LAST_VARIANT) among them. */
+ * as fp32 calls do under 1..14.  Unknown ids are rejected with MS_ERR_ARG, the others
+ * of MS_QUERY_LAST_VARIANT (15 to 17, 26, 27) among them.  The sums over devices have the tiles 2, 4 and 14 and take the library's
+ * choice under every other id. */
 int ms_set_variant(int variant);
 
 /* Compute units that the GEMM launches of the calling thread leave free (default 0; returns MS_ERR_ARG outside

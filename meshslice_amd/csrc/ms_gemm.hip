@@ -36,6 +36,14 @@ MS_INSTANTIATE_RING(256, 192, 64, 2, 2, 2)
 MS_INSTANTIATE_RING(192, 256, 64, 2, 2, 2)
 MS_INSTANTIATE_RING(128, 128, 64, 3, 2, 2)
 #undef MS_INSTANTIATE_RING
+// several devices' partial sums in one product (Problem::sum): the tiles on three stages, whose waves have room for the totals
+#define MS_INSTANTIATE_SUM(BM, BN)                                                                                           \
+  template __global__ void msk::gemm_bf16_ring_kernel<BM, BN, 64, 3, 2, 2, true, true, true, false, true>(const msk::GemmArgs); \
+  template __global__ void msk::gemm_bf16_ring_kernel<BM, BN, 64, 3, 2, 2, false, false, true, false, true>(const msk::GemmArgs);
+MS_INSTANTIATE_SUM(128, 128)
+MS_INSTANTIATE_SUM(128, 192)
+MS_INSTANTIATE_SUM(192, 192)
+#undef MS_INSTANTIATE_SUM
 #define MS_INSTANTIATE_BIG(TM, TN)                                                                             \
   template __global__ void msk::gemm_bf16_big_kernel<TM, TN, true, false, true, false>(const msk::GemmArgs);   \
   template __global__ void msk::gemm_bf16_big_kernel<TM, TN, true, false, false, false>(const msk::GemmArgs);  \
@@ -144,6 +152,8 @@ struct Problem {
   int M, N, K;           // per-chunk rows/cols, per-slice contraction
   int lda, ldb, ldc;
   int in_dtype, out_dtype;
+  // LS / RS: C = sum over the S entries of both tables, each entry's partial sum by itself, added up in fp32 in their order
+  bool sum = false;
   // fused OS epilogue (all zero / null = plain product)
   int act = 0;
   const void *res = nullptr;
@@ -243,10 +253,11 @@ int launch_bf16_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, 
   for (int i = 0; i < p.na; i++) g.a[i] = p.a[i];
   for (int i = 0; i < p.nb; i++) g.b[i] = p.b[i];
   for (int i = 0; i < p.nc; i++) g.c[i] = p.c[i];
-  g.nchunks = p.flow == OS ? 1 : p.S;
-  g.nkslices = p.flow == OS ? p.S : 1;
-  g.a_by_chunk = p.flow == RS || (p.flow == LS && p.na > 1);      // (several devices' products: a pointer for every chunk)
-  g.b_by_chunk = p.flow == LS || (p.flow == RS && p.nb > 1);
+  const bool one_output = p.flow == OS || p.sum;
+  g.nchunks = one_output ? 1 : p.S;
+  g.nkslices = one_output ? p.S : 1;
+  g.a_by_chunk = !one_output && (p.flow == RS || p.na > 1);      // (several devices' products: a pointer for every chunk)
+  g.b_by_chunk = !one_output && (p.flow == LS || p.nb > 1);
   g.M = p.M; g.N = p.N; g.K = p.K;
   g.lda = p.lda; g.ldb = p.ldb; g.ldc = p.ldc;
   g.tiles_m = (p.M + BM - 1) / BM;
@@ -272,7 +283,14 @@ int launch_bf16_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, 
   const bool obf = p.out_dtype == MS_DTYPE_BF16;
   g.act = p.act; g.res = p.res; g.ldr = p.ldr; g.row_sum = p.row_sum; g.row_sumsq = p.row_sumsq;
   const bool epi = p.act != 0 || p.res || p.row_sum || p.row_sumsq;
-  if (p.flow == OS) {
+  if (p.sum) {
+    if constexpr (KIND == 0 && NS == 3) {
+      if (p.flow == LS) msk::gemm_bf16_ring_kernel<BM, BN, BK_, NS, WGM, WGN, true, true, true, false, true><<<gd, bd, 0, stream>>>(g);
+      else msk::gemm_bf16_ring_kernel<BM, BN, BK_, NS, WGM, WGN, false, false, true, false, true><<<gd, bd, 0, stream>>>(g);
+    } else {
+      return fail(MS_ERR_UNSUPPORTED, "tile variant %d does not add up several devices' partial sums", variant);
+    }
+  } else if (p.flow == OS) {
     if (epi) {
       if (obf) launch_one<KIND, BM, BN, BK_, NS, WGM, WGN, true, false, true, true>(gd, bd, stream, g);
       else launch_one<KIND, BM, BN, BK_, NS, WGM, WGN, true, false, false, true>(gd, bd, stream, g);
@@ -347,7 +365,7 @@ int split_refused(const Problem &p, const DevFacts &dev, int v, int splits) {
   if (splits < 2 || splits > SPLIT_MAX) return 7;
   if (v == 1 || v == 12 || v == 13) return 8;     // 256x256 on four waves: see ring_can_split; the 16x16x32 kernels have none
   if (p.act || p.res || p.row_sum || p.row_sumsq) return 9;   // see ring_can_split, big_can_split
-  if (p.flow != OS) return 1;
+  if (p.sum ? splits != p.S : p.flow != OS) return 1;      // (the parts of a sum over devices are the devices)
   if (!p.ws) return 2;
   const long tiles = (long)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
   if (tiles * splits > dev.cus) return 3;
@@ -374,13 +392,19 @@ constexpr double TILE_OVERHEAD_K = 80.0;
 // reach the power limit
 double partial_round_loss(int v) { return v == 3 || v == 14 ? 1.0 : v == 2 || v == 4 ? 0.87 : PARTIAL_ROUND_LOSS; }
 
+// tiles that carry the sum over devices, and what the end of a device's share costs them (its accumulators join the totals,
+// 0.7 to 1 us of vector work), as contraction elements
+bool carries_sum(int v) { return v == 2 || v == 4 || v == 14; }
+constexpr double FOLD_K = 90.0;
+
 // the tile shape and split count with the lowest estimated cost for the whole problem
 Pick pick_variant(const Problem &p, const DevFacts &dev) {
   const bool rs = p.flow == RS, ls = p.flow == LS;
-  const long chunks = p.flow == OS ? 1 : p.S;
-  const double total_k = p.flow == OS ? (double)p.K * p.S : (double)p.K;
+  const long chunks = p.flow == OS || p.sum ? 1 : p.S;
+  const double total_k = p.flow == OS || p.sum ? (double)p.K * p.S : (double)p.K;
   Pick best = {0, 1, 0};
   for (const TileRate &c : TILE_RATES) {
+    if (p.sum && !carries_sum(c.v)) continue;
     const int bm = TILE_OF[c.v].bm, bn = TILE_OF[c.v].bn;
     const bool pairs = workgroups_per_unit(c.v) == 2;
     const double rate = rs ? c.rs : ls ? c.ls : c.os;
@@ -402,10 +426,11 @@ Pick pick_variant(const Problem &p, const DevFacts &dev) {
       // (two 128x128 workgroups share a unit only where there are more tiles than units)
       const double shared = !pairs || tiles * splits <= dev.cus ? 0.0 : tiles * splits >= 2L * dev.cus ? 1.0 : (double)(tiles * splits - dev.cus) / dev.cus;
       const double eff = splits > 1 ? c.split : rate - (pairs ? (rate - (rs ? PAIRED_RS : ls ? PAIRED_LS : PAIRED_OS)) * shared : 0.0);
-      const double cost = (rounds * bm * bn / eff * (total_k / splits + TILE_OVERHEAD_K) + exchange) / total_k;
+      const double cost = (rounds * bm * bn / eff * (total_k / splits + TILE_OVERHEAD_K + (p.sum && splits == 1 ? FOLD_K * p.S : 0.0)) + exchange) / total_k;
       if (best.v == 0 || cost < best.cost) best = {c.v, splits, cost};
     }
   }
+  if (p.sum) return best;
   // An unsplit 256x384 product runs on the 16x16x32 kernel: 4-8 % faster than the 32x32x16 one, which stays selectable
   // as variant 10 and carries the split contraction.
   if (best.splits == 1 && best.v == 10) best.v = 12;
@@ -420,7 +445,8 @@ Pick pick_variant(const Problem &p, const DevFacts &dev) {
 
 int launch_variant(int v, int splits, const Problem &p, const DevFacts &dev, hipStream_t stream) {
   if (p.slice_ready && v == 1) return fail(MS_ERR_UNSUPPORTED, "tile variant %d has no input gate (256x256 on four waves of the ring kernel)", v);
-  if (g_launches == 0) { g_last_variant = v; g_last_splits = splits; }
+  // (the kernels that add up devices' sums go by ids of their own: 15 to 17 for the tiles 14, 4 and 2)
+  if (g_launches == 0) { g_last_variant = !p.sum ? v : v == 14 ? 15 : v == 4 ? 16 : 17; g_last_splits = splits; }
   switch (v) {
     case 1: return launch_bf16_tile<256, 256, 2, 2, 64, 2>(p, dev, stream, 1, splits);
     case 2: return launch_bf16_tile<192, 192, 2, 2, 64, 3>(p, dev, stream, 2, splits);
@@ -448,7 +474,7 @@ int launch_variant(int v, int splits, const Problem &p, const DevFacts &dev, hip
 // their chunks are promised in slice order.
 int launch_bf16(const Problem &p, const DevFacts &dev, hipStream_t stream) {
   if (!dev.gfx950) return fail(MS_ERR_UNSUPPORTED, "the bf16 kernels need a gfx950 device");
-  if (g_variant >= 1 && g_variant <= VARIANTS) return launch_variant(g_variant, g_splits > 1 ? g_splits : 1, p, dev, stream);
+  if (g_variant >= 1 && g_variant <= VARIANTS && (!p.sum || carries_sum(g_variant))) return launch_variant(g_variant, g_splits > 1 ? g_splits : 1, p, dev, stream);
   const Pick single = pick_variant(p, dev);
   // (a gated product stays one launch: a second one would stand in the stream behind the first while that waits for slices)
   if (p.flow == OS && single.splits == 1 && g_splits == 0 && !p.slice_ready) {
@@ -969,6 +995,29 @@ MS_API int ms_gemm_rs_peers(const void *const *X_slices, int ldx, const void *co
   const void *w[MS_MAX_SLICES];
   if (int rc = spread_over_chunks(W, P, S, w, "ms_gemm_rs_peers")) return rc;
   return run(make_problem(RS, X_slices, w, Y_chunks, P * S, P * S, P * S, P * S, m_slice, n, k, ldx, ldw, ldy, in_dtype, out_dtype), stream);
+}
+
+// The same products with the devices' partial sums added up on the way out instead of in chunks through memory (see the header).
+namespace {
+int run_sum(Problem p, void *workspace, size_t workspace_bytes, void *stream, const char *fn) {
+  if (p.S < 1 || p.S > MS_MAX_SLICES) return fail(MS_ERR_ARG, "%s: P = %d outside [1, %d]", fn, p.S, MS_MAX_SLICES);
+  if (p.in_dtype != MS_DTYPE_BF16 || p.out_dtype != MS_DTYPE_BF16) return fail(MS_ERR_UNSUPPORTED, "%s: bf16 operands and results only", fn);
+  p.sum = p.S > 1;      // (one device's partial sum is its product)
+  if (p.sum) { p.ws = workspace; p.ws_bytes = workspace ? workspace_bytes : 0; }
+  return run(p, stream);
+}
+}  // namespace
+
+MS_API int ms_gemm_ls_sum(const void *const *A, int lda, const void *const *W, int ldw, int P, int m, int n, int k, void *C, int ldc,
+                          int in_dtype, int out_dtype, void *workspace, size_t workspace_bytes, void *stream) {
+  void *c1[1] = {C};
+  return run_sum(make_problem(LS, A, W, c1, P, P, 1, P, m, n, k, lda, ldw, ldc, in_dtype, out_dtype), workspace, workspace_bytes, stream, "ms_gemm_ls_sum");
+}
+
+MS_API int ms_gemm_rs_sum(const void *const *X, int ldx, const void *const *W, int ldw, int P, int m, int n, int k, void *C, int ldc,
+                          int in_dtype, int out_dtype, void *workspace, size_t workspace_bytes, void *stream) {
+  void *c1[1] = {C};
+  return run_sum(make_problem(RS, X, W, c1, P, P, 1, P, m, n, k, ldx, ldw, ldc, in_dtype, out_dtype), workspace, workspace_bytes, stream, "ms_gemm_rs_sum");
 }
 
 // the chunk-producing calls with completion counters

@@ -378,6 +378,39 @@ def _peers(entry, first, second, P, S, chunk, extents):
     return [chunks[p * S:(p + 1) * S] for p in range(P)]
 
 
+def gemm_ls_sum(X: torch.Tensor, W: torch.Tensor, P: int) -> torch.Tensor:
+    """``X @ W^T`` as the P devices of a mesh row compute it between them (``ms_gemm_ls_sum``): the contraction in P equal
+    windows, each window's partial sum in fp32 by itself, the partial sums added up in window order and rounded once.  bf16."""
+    _check2d(X, "X"); _check2d(W, "W")
+    if X.shape[1] != W.shape[1] or X.dtype != W.dtype or X.device != W.device or X.shape[1] % P:
+        raise ValueError(f"shapes do not contract in {P} windows: {tuple(X.shape)} @ {tuple(W.shape)}^T")
+    step = X.shape[1] // P * X.element_size()
+    return _sum(_lib.load().ms_gemm_ls_sum, X, W, P, step, step, X.shape[0], W.shape[0], X.shape[1] // P)
+
+
+def gemm_rs_sum(X: torch.Tensor, W: torch.Tensor, P: int) -> torch.Tensor:
+    """``X^T @ W`` in the same way (``ms_gemm_rs_sum``): the P windows are those of the devices of a mesh column."""
+    _check2d(X, "X"); _check2d(W, "W")
+    if X.shape[0] != W.shape[0] or X.dtype != W.dtype or X.device != W.device or X.shape[0] % P:
+        raise ValueError(f"shapes do not contract in {P} windows: {tuple(X.shape)}^T @ {tuple(W.shape)}")
+    k = X.shape[0] // P
+    return _sum(_lib.load().ms_gemm_rs_sum, X, W, P, k * X.stride(0) * X.element_size(), k * W.stride(0) * W.element_size(), X.shape[1], W.shape[1], k)
+
+
+def _sum(entry, X, W, P, x_step, w_step, m, n, k):
+    out = torch.empty((m, n), dtype=X.dtype, device=X.device)
+    x0, w0 = X.data_ptr(), W.data_ptr()
+    px, _kx = _lib.ptr_array([x0 + p * x_step for p in range(P)])
+    pw, _kw = _lib.ptr_array([w0 + p * w_step for p in range(P)])
+    with _on(X.device):
+        stream = torch.cuda.current_stream()
+        ws = workspace(X.device, stream)
+        rc = entry(px, X.stride(0), pw, W.stride(0), P, m, n, k, ctypes.c_void_p(out.data_ptr()), n, _dt(X), _dt(out),
+                   ctypes.c_void_p(ws.data_ptr()), ws.numel(), ctypes.c_void_p(stream.cuda_stream))
+    _lib.check(rc)
+    return out
+
+
 def _check_counters(chunk_done: torch.Tensor, S: int, device) -> None:
     if not (isinstance(chunk_done, torch.Tensor) and chunk_done.is_cuda and chunk_done.device == device
             and chunk_done.dtype == torch.int32 and chunk_done.is_contiguous() and chunk_done.numel() >= S):
