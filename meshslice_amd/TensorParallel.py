@@ -50,6 +50,49 @@ def _shards(G: torch.Tensor, R: int, C: int) -> List[List[torch.Tensor]]:
     return [[G[i * h:(i + 1) * h, j * w:(j + 1) * w] for j in range(C)] for i in range(R)]
 
 
+class _Line:
+    """The shards of one mesh row or column of a global matrix, in axis order: the views, made where they are asked for, and
+    the one view that covers them."""
+
+    def __init__(self, panel: torch.Tensor, n: int, axis: int):
+        self.panel, self.n, self.axis, self.step = panel, n, axis, panel.shape[axis] // n
+
+    def __len__(self):
+        return self.n
+
+    def __getitem__(self, p):
+        if not -self.n <= p < self.n:
+            raise IndexError(p)
+        return self.panel.narrow(self.axis, p % self.n * self.step, self.step)
+
+
+class _Grid:
+    """_shards without the R * C views: ``grid[i]`` is mesh row i's shards, ``_column(grid, j)`` mesh column j's."""
+
+    def __init__(self, G: torch.Tensor, R: int, C: int):
+        if G.dim() != 2:
+            raise ValueError("operands must be 2-D")
+        if G.shape[0] % R or G.shape[1] % C:
+            raise ValueError(f"matrix {tuple(G.shape)} does not shard evenly over a {R}x{C} mesh")
+        self.G, self.R, self.C, self.h, self.w = G, R, C, G.shape[0] // R, G.shape[1] // C
+
+    def __len__(self):
+        return self.R
+
+    def __getitem__(self, i):
+        if not -self.R <= i < self.R:
+            raise IndexError(i)
+        return _Line(self.G.narrow(0, i % self.R * self.h, self.h), self.C, 1)
+
+
+def _row(grid, i, C):
+    return grid[i] if isinstance(grid, _Grid) else [grid[i][j] for j in range(C)]
+
+
+def _column(grid, j, R):
+    return _Line(grid.G.narrow(1, j * grid.w, grid.w), R, 0) if isinstance(grid, _Grid) else [grid[i][j] for i in range(R)]
+
+
 def _need(v: int, d: int, what: str) -> None:
     if d <= 0 or v % d:
         raise ValueError(f"{what} = {v} is not a multiple of {d}")
@@ -75,6 +118,8 @@ PANEL_MAX_ROWS = 65535 * 8      # rows that one launch of the layout kernels alw
 def _spanning(parts: Sequence[torch.Tensor], axis: int):
     """The one view that covers ``parts`` when they are neighbouring blocks of one matrix in axis order (the shards of a
     global operand are), else None."""
+    if isinstance(parts, _Line):
+        return parts.panel if parts.axis == axis and parts.panel.stride(1) == 1 and parts.panel.shape[0] <= PANEL_MAX_ROWS else None
     p0 = parts[0]
     step = p0.shape[1] if axis == 1 else p0.shape[0] * p0.stride(0)
     at, base = p0.storage_offset(), p0.untyped_storage().data_ptr()
@@ -133,20 +178,20 @@ def _gather_row_slices(peers: Sequence[torch.Tensor], K: int, B: int) -> List[to
 
 def Collective_OS(X, W, i, j, R, C, K, B):
     """reference TensorParallel.py:19-22: gather X over col, W over row, one contraction."""
-    Xi = _gather([X[i][jj] for jj in range(C)], 1)
-    Wj = _gather([W[ii][j] for ii in range(R)], 0)
+    Xi = _gather(_row(X, i, C), 1)
+    Wj = _gather(_column(W, j, R), 0)
     return local_gemm.gemm_os([Xi], [Wj])
 
 
 def Collective_LS(X, W, i, j, R, C, K, B):
     """reference :24-27: gather W over row; partial product X_ij @ Wj^T (input of psum_scatter)."""
-    Wj = _gather([W[ii][j] for ii in range(R)], 0)
+    Wj = _gather(_column(W, j, R), 0)
     return local_gemm.gemm_ls(_own(X[i][j]), [Wj])
 
 
 def Collective_RS(X, W, i, j, R, C, K, B):
     """reference :29-32: gather X over col; partial product Xi^T @ W_ij (input of psum_scatter)."""
-    Xi = _gather([X[i][jj] for jj in range(C)], 1)
+    Xi = _gather(_row(X, i, C), 1)
     return local_gemm.gemm_rs([Xi], _own(W[i][j]))
 
 
@@ -155,8 +200,8 @@ def MeshFlow_OS(X, W, i, j, R, C, K, B):
     if K == 1:
         raise ValueError("the sliced OS body is undefined for K == 1 (the reference adds slice 0 twice); "
                          "use algorithm='collective' for the unsliced product")
-    A_slices = _gather_col_slices([X[i][jj] for jj in range(C)], K, B)
-    B_slices = _gather_row_slices([W[ii][j] for ii in range(R)], K, B)
+    A_slices = _gather_col_slices(_row(X, i, C), K, B)
+    B_slices = _gather_row_slices(_column(W, j, R), K, B)
     return local_gemm.gemm_os(A_slices, B_slices)
 
 
@@ -284,8 +329,8 @@ def MeshFlow_OS_overlap(X, W, i, j, R, C, K, B):
     if K == 1:
         raise ValueError("the sliced OS body is undefined for K == 1 (the reference adds slice 0 twice); "
                          "use algorithm='collective' for the unsliced product")
-    bufA, fillA = _col_slice_filler([X[i][jj] for jj in range(C)], K, B)
-    bufB, fillB = _row_slice_filler([W[ii][j] for ii in range(R)], K, B)
+    bufA, fillA = _col_slice_filler(_row(X, i, C), K, B)
+    bufB, fillB = _row_slice_filler(_column(W, j, R), K, B)
     return _launch_ahead_of_gathers(K, bufA.device, lambda ready: local_gemm.gemm_os_gated([bufA[k] for k in range(K)], [bufB[k] for k in range(K)], ready),
                                     (fillA, fillB))
 
@@ -293,27 +338,27 @@ def MeshFlow_OS_overlap(X, W, i, j, R, C, K, B):
 def MeshFlow_LS_overlap(X, W, i, j, R, C, K, B):
     """MeshFlow_LS with the one launch ahead of the gathers of W's row slices (:176-189; ``gemm_ls_gated``): chunk k is
     multiplied as soon as slice k has arrived.  Same chunks as MeshFlow_LS, bit for bit."""
-    bufW, fillW = _row_slice_filler([W[ii][j] for ii in range(R)], K, B)
+    bufW, fillW = _row_slice_filler(_column(W, j, R), K, B)
     own = _own(X[i][j])
     return _launch_ahead_of_gathers(K, bufW.device, lambda ready: local_gemm.gemm_ls_gated(own, [bufW[k] for k in range(K)], ready), (fillW,))
 
 
 def MeshFlow_RS_overlap(X, W, i, j, R, C, K, B):
     """MeshFlow_RS with the one launch ahead of the gathers of X's column slices (:198-212; ``gemm_rs_gated``)."""
-    bufX, fillX = _col_slice_filler([X[i][jj] for jj in range(C)], K, B)
+    bufX, fillX = _col_slice_filler(_row(X, i, C), K, B)
     own = _own(W[i][j])
     return _launch_ahead_of_gathers(K, bufX.device, lambda ready: local_gemm.gemm_rs_gated([bufX[k] for k in range(K)], own, ready), (fillX,))
 
 
 def MeshFlow_LS(X, W, i, j, R, C, K, B):
     """reference :174-193: K gathered row slices of W; K fp32 partial chunks X_ij @ W_k^T."""
-    W_slices = _gather_row_slices([W[ii][j] for ii in range(R)], K, B)
+    W_slices = _gather_row_slices(_column(W, j, R), K, B)
     return local_gemm.gemm_ls(_own(X[i][j]), W_slices)
 
 
 def MeshFlow_RS(X, W, i, j, R, C, K, B):
     """reference :195-214: K gathered column slices of X; K fp32 partial chunks X_k^T @ W_ij."""
-    X_slices = _gather_col_slices([X[i][jj] for jj in range(C)], K, B)
+    X_slices = _gather_col_slices(_row(X, i, C), K, B)
     return local_gemm.gemm_rs(X_slices, _own(W[i][j]))
 
 
@@ -350,7 +395,7 @@ def _usable(views: Sequence[torch.Tensor]) -> List[torch.Tensor]:
 
 
 def _ring_os(algorithm, X, W, i, j, R, C):
-    Wj = _gather([W[ii][j] for ii in range(R)], 0)                       # [Kd, n/C]
+    Wj = _gather(_column(W, j, R), 0)                       # [Kd, n/C]
     _need(X[i][j].shape[1], 2, "columns of an X shard"); _need(Wj.shape[0], 2 * C, "gathered rows of W")
     h = Wj.shape[0] // C // 2
     order = _ring_order(algorithm, "os", R, C, i, j)
@@ -360,7 +405,7 @@ def _ring_os(algorithm, X, W, i, j, R, C):
 
 
 def _ring_ls(algorithm, X, W, i, j, R, C):
-    Wj = _gather([W[ii][j] for ii in range(R)], 0)                       # [O, I/C]
+    Wj = _gather(_column(W, j, R), 0)                       # [O, I/C]
     _need(Wj.shape[0], 2 * C, "gathered rows of W")
     h = Wj.shape[0] // C // 2
     order = _ring_order(algorithm, "ls", R, C, i, j)
@@ -558,7 +603,7 @@ class ShardedMatmul:
 
         def run(X, W):
             self._validate(X, W)
-            return self.body(_shards(X, self.R, self.C), _shards(W, self.R, self.C), i, j, self.R, self.C, self.K, self.B)
+            return self.body(_Grid(X, self.R, self.C), _Grid(W, self.R, self.C), i, j, self.R, self.C, self.K, self.B)
         return run
 
     def _whole_mesh(self, X, W, K, B):

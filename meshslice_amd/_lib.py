@@ -10,6 +10,8 @@ import ctypes
 import os
 import threading
 
+import torch  # noqa: F401  (the native call path links against its libraries)
+
 MS_DTYPE_F32 = 0
 MS_DTYPE_BF16 = 1
 MS_OK = 0
@@ -142,6 +144,27 @@ def load():
             _declare(lib)
             _lib = lib
         return _lib
+
+
+class _HostMissing:
+    """Stands for the native call path where it has not been built: the first use says so."""
+
+    def __getattr__(self, name):
+        if name.startswith("__"):
+            raise AttributeError(name)
+        raise MeshSliceError("meshslice_amd/_host has not been built beside libmeshslice_hip.so (run __graft_entry__.build() or "
+                             "`make -C meshslice_amd/csrc`)")
+
+
+def _load_host():
+    import importlib
+    try:
+        return importlib.import_module("._host", __package__)
+    except ImportError:
+        return _HostMissing()
+
+
+host = _load_host()      # (torch is loaded by then: the modules that use it import it first)
 
 
 def last_error() -> str:

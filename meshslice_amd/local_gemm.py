@@ -49,6 +49,10 @@ def _same(ts: Sequence[torch.Tensor], name: str):
     return s0
 
 
+# The ordinary case of a call (plain GPU tensors, output left to the call) is taken by the native call path as a whole
+# (_lib.host, csrc/ms_host.cpp); it returns None for everything else, which the functions below then handle or refuse.
+# gemm_os of four slices of 512 x 256 x 512 in fp32 takes the host 18.8 us a call without it and 5.5 with it, launch included; one device of a
+# 2x4 mesh (gather and LS product) 76 and 27; a training step of 512 x 256 x 1024 on a 4x2 mesh, whose sums are one launch each, 232 and 135.
 _HERE = contextlib.nullcontext()
 
 
@@ -57,7 +61,7 @@ def _on(device: torch.device):
     return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
-_workspaces = {}            # (device index, stream handle) -> uint8 tensor, least recently used first
+_workspaces = {}            # (device index, stream handle) -> uint8 tensor; the native call path knows their addresses and when each was used last
 _workspaces_lock = threading.Lock()
 _WORKSPACE_CACHE_MAX = 8      # streams per device that keep a workspace of their own (about 100 MB each)
 
@@ -85,9 +89,9 @@ def workspace(device, stream=None) -> torch.Tensor:
     capturing = torch.cuda.is_current_stream_capturing()
     if not capturing:
         with _workspaces_lock:
-            ws = _workspaces.pop(key, None)
+            ws = _workspaces.get(key)
             if ws is not None:
-                _workspaces[key] = ws      # most recently used last
+                _lib.host.workspace_touch(*key)
                 return ws
     lib = _lib.load()
     with torch.cuda.device(idx), torch.cuda.stream(stream):
@@ -100,8 +104,12 @@ def workspace(device, stream=None) -> torch.Tensor:
         return ws
     with _workspaces_lock:
         have = _workspaces.setdefault(key, ws)      # (another thread on the same stream may have been faster)
-        mine = [k for k in _workspaces if k[0] == idx and k != key]
-        evicted = [_workspaces.pop(k) for k in mine[:max(0, len(mine) + 1 - _WORKSPACE_CACHE_MAX)]]
+        mine = sorted((k for k in _workspaces if k[0] == idx and k != key), key=lambda k: _lib.host.workspace_touch(*k, False))
+        drop = mine[:max(0, len(mine) + 1 - _WORKSPACE_CACHE_MAX)]
+        for k in drop:      # (the native call path must not hand one out that is about to go)
+            _lib.host.workspace_drop(*k)
+        evicted = [_workspaces.pop(k) for k in drop]
+        _lib.host.workspace_set(*key, have.data_ptr(), have.numel())
     if evicted:
         torch.cuda.synchronize(idx)     # their streams may still be running products that use them
         del evicted
@@ -196,6 +204,10 @@ def gemm_os(A_slices: Sequence[torch.Tensor], B_slices: Sequence[torch.Tensor],
     Optional fused epilogue (bf16 operands): ``C = act(sum) + residual`` with ``activation='gelu'`` (tanh
     form) and ``residual`` of C's shape and dtype; ``row_moments=(row_sum, row_sumsq)`` are fp32 vectors of
     length m (either may be None) to which the row sums / sums of squares of the fp32 result are ADDED."""
+    if out is None and row_moments is None and activation in (None, "gelu"):
+        y = _lib.host.gemm_os(A_slices, B_slices, out_dtype, activation is not None, residual)
+        if y is not None:
+            return y
     call = _prepare_os(A_slices, B_slices, out, out_dtype)
     out = call.out
     m, n = out.shape
@@ -318,6 +330,10 @@ def gemm_ls(A: torch.Tensor, W_slices: Sequence[torch.Tensor],
     """``Y_s = A @ W_s^T``, W_s stored ``[n_slice, k]``.  Chunks are fp32 by default (exact partial sums for
     the reduce-scatter); ``out_dtype=torch.bfloat16`` gives what the reference's einsum returns for bf16
     operands (TensorParallel.py:181-189): one rounding of the fp32 accumulator, half the bytes."""
+    if out is None:
+        chunks = _lib.host.gemm_ls(A, W_slices, out_dtype)
+        if chunks is not None:
+            return chunks
     call = _prepare_ls(A, W_slices, out, out_dtype)
     with _on(call.device):
         rc = _lib.load().ms_gemm_ls_ex(*call.args, _stream())
@@ -328,6 +344,10 @@ def gemm_ls(A: torch.Tensor, W_slices: Sequence[torch.Tensor],
 def gemm_rs(X_slices: Sequence[torch.Tensor], W: torch.Tensor,
             out: Optional[List[torch.Tensor]] = None, out_dtype: Optional[torch.dtype] = None) -> List[torch.Tensor]:
     """``Y_s = X_s^T @ W``, X_s stored ``[k, m_slice]``; chunks fp32 by default, bf16 on request (see gemm_ls)."""
+    if out is None:
+        chunks = _lib.host.gemm_rs(X_slices, W, out_dtype)
+        if chunks is not None:
+            return chunks
     call = _prepare_rs(X_slices, W, out, out_dtype)
     with _on(call.device):
         rc = _lib.load().ms_gemm_rs_ex(*call.args, _stream())
@@ -381,6 +401,9 @@ def _peers(entry, first, second, P, S, chunk, extents):
 def gemm_ls_sum(X: torch.Tensor, W: torch.Tensor, P: int) -> torch.Tensor:
     """``X @ W^T`` as the P devices of a mesh row compute it between them (``ms_gemm_ls_sum``): the contraction in P equal
     windows, each window's partial sum in fp32 by itself, the partial sums added up in window order and rounded once.  bf16."""
+    y = _lib.host.gemm_ls_sum(X, W, P)
+    if y is not None:
+        return y
     _check2d(X, "X"); _check2d(W, "W")
     if X.shape[1] != W.shape[1] or X.dtype != W.dtype or X.device != W.device or X.shape[1] % P:
         raise ValueError(f"shapes do not contract in {P} windows: {tuple(X.shape)} @ {tuple(W.shape)}^T")
@@ -390,6 +413,9 @@ def gemm_ls_sum(X: torch.Tensor, W: torch.Tensor, P: int) -> torch.Tensor:
 
 def gemm_rs_sum(X: torch.Tensor, W: torch.Tensor, P: int) -> torch.Tensor:
     """``X^T @ W`` in the same way (``ms_gemm_rs_sum``): the P windows are those of the devices of a mesh column."""
+    y = _lib.host.gemm_rs_sum(X, W, P)
+    if y is not None:
+        return y
     _check2d(X, "X"); _check2d(W, "W")
     if X.shape[0] != W.shape[0] or X.dtype != W.dtype or X.device != W.device or X.shape[0] % P:
         raise ValueError(f"shapes do not contract in {P} windows: {tuple(X.shape)}^T @ {tuple(W.shape)}")

@@ -23,6 +23,10 @@ def pack_slices(block: torch.Tensor, S: int, B: int, axis: int,
     """The S block-cyclic slices of ``block`` along ``axis`` (1 = columns, 0 = rows): slice s holds the
     B-wide blocks ``b`` with ``b % S == s`` in ascending order.  ``out`` may be S row-major views into a
     larger buffer (for example a peer's place in a gathered slice); they share one leading dimension."""
+    if out is None:
+        slices = _lib.host.pack_slices(block, S, B, axis)
+        if slices is not None:
+            return slices
     _check2d(block, "block")
     if axis not in (0, 1):
         raise ValueError("axis must be 0 or 1")
@@ -55,6 +59,10 @@ def unpack_chunks(chunks_by_peer: Sequence[Sequence[torch.Tensor]], B: int, axis
     ``window`` (what a tiled ``psum_scatter`` over ``parts`` devices hands to device ``window``); the
     windows are summed over the peers in fp32, rounded once to ``out_dtype`` and interleaved: block ``h`` of
     chunk ``s`` lands at block ``h * S + s`` of the output."""
+    if out is None:
+        shard = _lib.host.unpack_chunks(chunks_by_peer, B, axis, window, parts, out_dtype)
+        if shard is not None:
+            return shard
     P = len(chunks_by_peer)
     if P < 1:
         raise ValueError("need at least one peer's chunks")
