@@ -176,6 +176,14 @@ int ms_gemm_rs_ex(const void *const *X_slices, int ldx, const void *W, int ldw, 
                   int m_slice, int n, int k,
                   void *const *Y_chunks, int ldy, int in_dtype, int out_dtype, void *stream);
 
+/* ms_gemm_os_ws with B's slices where they lie in the matrix that they are cut from: B_s is the s-th block-cyclic row slice of
+ * W [S * k_slice, n] with blocks of eight rows (row r of it is row (r / 8 * S + s) * 8 + r % 8 of W; ms_pack_slices with axis 0
+ * and B = 8 copies the same).  k_slice is a multiple of 8; W spans less than 2 GiB.  Same bits as on the copied slices. */
+int ms_gemm_os_cyclic(const void *const *A_slices, const void *W, int S,
+                      int m, int n, int k_slice, int lda, int ldw,
+                      void *C, int ldc, int in_dtype, int out_dtype,
+                      void *workspace, size_t workspace_bytes, void *stream);
+
 /* ms_gemm_ls_ex / ms_gemm_rs_ex for P mesh devices of equal shapes in one launch (the devices of a mesh row, LS, or of a mesh
  * column, RS, whose partial chunks one reduce-scatter adds up): A (LS) / W (RS) holds the P devices' own shards, the slice
  * and chunk tables hold P * S <= MS_MAX_SLICES entries, device-major: Y[p*S+s] = A[p] @ W[p*S+s]^T, or X[p*S+s]^T @ W[p].

@@ -617,7 +617,12 @@ class ShardedMatmul:
         K = self.K if self.sliced else 1
         B = self.B if self.sliced else 1
         if self.body in _WHOLE_MESH_BODIES[self.dataflow] and _fits_whole_mesh(self.dataflow, X, W, R, C, K):
-            # (the global result is the same whatever the slices: nothing is gathered, cut or interleaved for it)
+            # (the global result is the same whatever the slices: nothing is gathered, cut or interleaved for it, but for the order in
+            # which an OS product contracts them)
+            if self.body is Collective_OS and _own(X) is X and _own(W) is W:
+                return local_gemm.gemm_os([X], [W])
+            if self.body is MeshFlow_OS and K > 1 and B == 8 and _own(W) is W:
+                return local_gemm.gemm_os_cyclic(slice_layout.pack_slices(X, K, B, 1), W)
             if self.dataflow == "ls" and _sums_on_chip(X, W):
                 return local_gemm.gemm_ls_sum(X, W, C)
             if self.dataflow == "rs" and _sums_on_chip(X, W):

@@ -151,6 +151,7 @@ struct Problem {
   int S;
   int M, N, K;           // per-chunk rows/cols, per-slice contraction
   int lda, ldb, ldc;
+  int b_blk = 0;         // OS: bytes from one block of eight rows of a B slice to its next (0: they follow each other)
   int in_dtype, out_dtype;
   // LS / RS: C = sum over the S entries of both tables, each entry's partial sum by itself, added up in fp32 in their order
   bool sum = false;
@@ -259,7 +260,7 @@ int launch_bf16_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, 
   g.a_by_chunk = !one_output && (p.flow == RS || p.na > 1);      // (several devices' products: a pointer for every chunk)
   g.b_by_chunk = !one_output && (p.flow == LS || p.nb > 1);
   g.M = p.M; g.N = p.N; g.K = p.K;
-  g.lda = p.lda; g.ldb = p.ldb; g.ldc = p.ldc;
+  g.lda = p.lda; g.ldb = p.ldb; g.ldc = p.ldc; g.b_blk = p.b_blk ? p.b_blk : p.ldb * 8 * (p.in_dtype == MS_DTYPE_BF16 ? 2 : 4);
   g.tiles_m = (p.M + BM - 1) / BM;
   g.tiles_n = (p.N + BN - 1) / BN;
   const long total = (long)g.tiles_m * g.tiles_n * g.nchunks;
@@ -530,7 +531,7 @@ int launch_f32_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, i
   g.a_by_chunk = p.flow == RS || (p.flow == LS && p.na > 1);      // (several devices' products: a pointer for every chunk)
   g.b_by_chunk = p.flow == LS || (p.flow == RS && p.nb > 1);
   g.M = p.M; g.N = p.N; g.K = p.K;
-  g.lda = p.lda; g.ldb = p.ldb; g.ldc = p.ldc;
+  g.lda = p.lda; g.ldb = p.ldb; g.ldc = p.ldc; g.b_blk = p.b_blk ? p.b_blk : p.ldb * 8 * (p.in_dtype == MS_DTYPE_BF16 ? 2 : 4);
   g.tiles_m = (p.M + BM - 1) / BM;
   g.tiles_n = (p.N + BN - 1) / BN;
   const long total = (long)g.tiles_m * g.tiles_n * g.nchunks;
@@ -847,6 +848,24 @@ MS_API int ms_gemm_os_ws(const void *const *A_slices, const void *const *B_slice
   void *c1[1] = {C};
   Problem p = make_os(A_slices, B_slices, S, m, n, k_slice, lda, ldb, c1, ldc, in_dtype, out_dtype);
   p.act = activation; p.res = residual; p.ldr = ldr; p.row_sum = row_sum; p.row_sumsq = row_sumsq;
+  p.ws = workspace; p.ws_bytes = workspace ? workspace_bytes : 0;
+  return run(p, stream);
+}
+
+// The slices of W in place: slice s begins at row 8 s and its blocks of eight rows lie S blocks apart, which for a kernel that loads
+// whole rows is another step between blocks of rows, not another access pattern.
+MS_API int ms_gemm_os_cyclic(const void *const *A_slices, const void *W, int S, int m, int n, int k_slice, int lda, int ldw, void *C, int ldc,
+                             int in_dtype, int out_dtype, void *workspace, size_t workspace_bytes, void *stream) {
+  const char *fn = "ms_gemm_os_cyclic";
+  if (S < 1 || S > MS_MAX_SLICES) return fail(MS_ERR_ARG, "%s: S = %d outside [1, %d]", fn, S, MS_MAX_SLICES);
+  const long long es = in_dtype == MS_DTYPE_BF16 ? 2 : 4;
+  if (k_slice <= 0 || k_slice % 8) return fail(MS_ERR_ARG, "%s: k_slice = %d is not a number of blocks of eight rows", fn, k_slice);
+  if (ldw < 0 || (long long)k_slice * S * ldw * es > 0x7FFFFFFFLL) return fail(MS_ERR_UNSUPPORTED, "%s: W spans 2 GiB or more", fn);
+  const void *b[MS_MAX_SLICES];
+  for (int s = 0; s < S; s++) b[s] = W ? static_cast<const char *>(W) + (long long)s * 8 * ldw * es : nullptr;
+  void *c1[1] = {C};
+  Problem p = make_os(A_slices, b, S, m, n, k_slice, lda, ldw, c1, ldc, in_dtype, out_dtype);
+  p.b_blk = (int)((long long)S * 8 * ldw * es);
   p.ws = workspace; p.ws_bytes = workspace ? workspace_bytes : 0;
   return run(p, stream);
 }

@@ -150,6 +150,23 @@ PyObject *gemm_os(PyObject *const *args) {
   return rc == MS_OK ? THPVariable_Wrap(std::move(out)) : nullptr;
 }
 
+// gemm_os_cyclic(A_slices, W) -> Tensor or None
+PyObject *gemm_os_cyclic(PyObject *const *args) {
+  const void *a[MS_MAX_SLICES];
+  int S = 0;
+  const at::Tensor *a0 = matrices(args[0], const_cast<void **>(a), &S), *w = a0 ? matrix(args[1]) : nullptr;
+  if (!w || a0->size(1) * S != w->size(0) || a0->scalar_type() != w->scalar_type() || a0->device() != w->device()) return nullptr;
+  const Place p = place_of(*a0);
+  const Workspace *ws = p.ok ? workspace_of(p) : nullptr;
+  if (!ws) return nullptr;
+  const int64_t m = a0->size(0), n = w->size(1);
+  const int code = code_of(*w);
+  at::Tensor out = at::empty({m, n}, w->options().requires_grad(false));
+  const int rc = ms_gemm_os_cyclic(a, w->data_ptr(), S, (int)m, (int)n, (int)a0->size(1), (int)a0->stride(0), (int)w->stride(0), out.data_ptr(), (int)n,
+                                   code, code, ws->ptr, ws->bytes, p.stream);
+  return rc == MS_OK ? THPVariable_Wrap(std::move(out)) : nullptr;
+}
+
 // gemm_ls(A, W_slices, out_dtype) / gemm_rs(X_slices, W, out_dtype) -> [chunks] or None
 template <bool LS>
 PyObject *gemm_chunks(PyObject *const *args) {
@@ -290,6 +307,7 @@ PyObject *workspace_touch(PyObject *, PyObject *args) {
 #define MS_ENTRY(name, impl, nargs) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<impl, nargs>)), METH_FASTCALL, nullptr}
 PyMethodDef g_methods[] = {
     MS_ENTRY("gemm_os", gemm_os, 5),
+    MS_ENTRY("gemm_os_cyclic", gemm_os_cyclic, 2),
     MS_ENTRY("gemm_ls", gemm_chunks<true>, 3),
     MS_ENTRY("gemm_rs", gemm_chunks<false>, 3),
     MS_ENTRY("gemm_ls_sum", gemm_sum<true>, 3),

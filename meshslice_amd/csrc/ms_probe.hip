@@ -151,7 +151,7 @@ MS_API int ms_probe_os_parts(int skip, const void *const *A_slices, const void *
   for (int s = 0; s < S; s++) { g.a[s] = A_slices[s]; g.b[s] = B_slices[s]; }
   g.c[0] = C;
   g.nchunks = 1; g.nkslices = S;
-  g.M = m; g.N = n; g.K = k_slice; g.lda = lda; g.ldb = ldb; g.ldc = ldc;
+  g.M = m; g.N = n; g.K = k_slice; g.lda = lda; g.ldb = ldb; g.ldc = ldc; g.b_blk = ldb * 16;
   g.tiles_m = (m + 255) / 256; g.tiles_n = (n + 383) / 384;
   g.total_tiles = g.tiles_m * g.tiles_n;
   g.group_m = 8; g.splits = 1;

@@ -237,6 +237,28 @@ def gemm_os(A_slices: Sequence[torch.Tensor], B_slices: Sequence[torch.Tensor],
     return out
 
 
+def gemm_os_cyclic(A_slices: Sequence[torch.Tensor], W: torch.Tensor) -> torch.Tensor:
+    """``gemm_os`` on the block-cyclic row slices of W (blocks of eight rows), read where they lie (``ms_gemm_os_cyclic``): the
+    bits of ``gemm_os(A_slices, pack_slices(W, len(A_slices), 8, 0))`` without that copy."""
+    y = _lib.host.gemm_os_cyclic(A_slices, W)
+    if y is not None:
+        return y
+    a0 = _same(A_slices, "A_slices"); _check2d(W, "W")
+    S = len(A_slices)
+    if S * a0.shape[1] != W.shape[0] or a0.dtype != W.dtype or a0.device != W.device:
+        raise ValueError(f"shapes do not contract: {S} slices {tuple(a0.shape)} @ {tuple(W.shape)}")
+    m, k = a0.shape; n = W.shape[1]
+    out = torch.empty((m, n), dtype=W.dtype, device=W.device)
+    pa, _ka = _lib.ptr_array([t.data_ptr() for t in A_slices])
+    with _on(W.device):
+        stream = torch.cuda.current_stream()
+        ws = workspace(W.device, stream)
+        rc = _lib.load().ms_gemm_os_cyclic(pa, ctypes.c_void_p(W.data_ptr()), S, m, n, k, a0.stride(0), W.stride(0), ctypes.c_void_p(out.data_ptr()), n,
+                                           _dt(W), _dt(W), ctypes.c_void_p(ws.data_ptr()), ws.numel(), ctypes.c_void_p(stream.cuda_stream))
+    _lib.check(rc)
+    return out
+
+
 def _chunk_dtype(out, out_dtype):
     """dtype of the LS / RS chunks: that of ``out`` if given, else ``out_dtype``, else fp32."""
     if out is not None and len(out) > 0:

@@ -29,7 +29,8 @@ def _calls(dtype, seed):
     calls = [lambda: ms.gemm_os(A, B), lambda: ms.gemm_os(tuple(A), B, out_dtype=torch.float32), lambda: ms.gemm_ls(A[0], [a[:24] for a in A]),
              lambda: ms.gemm_ls(A[0], [A[1]], out_dtype=torch.bfloat16), lambda: ms.gemm_rs([a[:, :16] for a in A], A[2]),
              lambda: pack_slices(wide, 4, 8, 1), lambda: pack_slices(wide[:, 8:40], 2, 4, 0), lambda: pack_slices(wide[:, 1:41], 5, 8, 1),
-             lambda: unpack_chunks(chunks, 8, 1, out_dtype=dtype), lambda: unpack_chunks(chunks, 8, 0, window=1, parts=2)]
+             lambda: unpack_chunks(chunks, 8, 1, out_dtype=dtype), lambda: unpack_chunks(chunks, 8, 0, window=1, parts=2),
+             lambda: local_gemm.gemm_os_cyclic([a[:, :32] for a in A[:2]], wide)]
     if dtype == torch.bfloat16:
         res = r(72, 64)[:, :56]
         calls += [lambda: ms.gemm_os(A, B, activation="gelu"), lambda: ms.gemm_os(A, B, residual=res), lambda: local_gemm.gemm_ls_sum(wide, wide, 3),
@@ -65,7 +66,7 @@ def test_the_native_path_takes_the_ordinary_calls():
     ms.gemm_os([a], [a])
     h = _host
     for got in (h.gemm_os([a], [a], None, False, None), h.gemm_os((a, a), [a, a], torch.float32, True, a.float()), h.gemm_ls(a, [a], None), h.gemm_rs([a], a, None),
-                h.gemm_ls_sum(a, a, 2), h.gemm_rs_sum(a, a, 2), h.pack_slices(a, 2, 8, 1), h.unpack_chunks([[a], [a]], 8, 1, 0, 1, None)):
+                h.gemm_ls_sum(a, a, 2), h.gemm_rs_sum(a, a, 2), h.gemm_os_cyclic([a[:, :8], a[:, 8:]], a), h.pack_slices(a, 2, 8, 1), h.unpack_chunks([[a], [a]], 8, 1, 0, 1, None)):
         assert got is not None
 
 
@@ -79,7 +80,7 @@ def test_what_the_native_path_declines():
                 h.gemm_os([a], [a.float()], None, False, None), h.gemm_os([a], [a], torch.float16, False, None), h.gemm_os([], [], None, False, None),
                 h.gemm_os([a] * 65, [a] * 65, None, False, None), h.gemm_os([odd], [odd.t().contiguous()], None, False, None), h.gemm_os(a, a, None, False, None),
                 h.gemm_os([a.as_subclass(Sub)], [a], None, False, None), h.gemm_os([a], [a], None, False, odd), h.gemm_os([None], [a], None, False, None),
-                h.gemm_ls(a, [odd], None), h.gemm_rs([a], None, None), h.gemm_ls_sum(a, a, 3), h.gemm_ls_sum(a, a, "2"), h.gemm_rs_sum(a.float(), a.float(), 2),
+                h.gemm_os_cyclic([a], odd.t()), h.gemm_os_cyclic([a, a], a), h.gemm_ls(a, [odd], None), h.gemm_rs([a], None, None), h.gemm_ls_sum(a, a, 3), h.gemm_ls_sum(a, a, "2"), h.gemm_rs_sum(a.float(), a.float(), 2),
                 h.pack_slices(a, 3, 8, 1), h.pack_slices(a, 0, 8, 1), h.pack_slices(a, 2, 8, 2), h.pack_slices(a, 2.0, 8, 1),
                 h.unpack_chunks([[a], [a, a]], 8, 1, 0, 1, None), h.unpack_chunks([], 8, 1, 0, 1, None), h.unpack_chunks([[a]], 8, 1, 2, 2, None),
                 h.unpack_chunks([[a] * 40, [a] * 40], 8, 1, 0, 1, None)]

@@ -5,6 +5,7 @@ import torch
 
 import meshslice_amd as ms
 from meshslice_amd import _lib, local_gemm
+from meshslice_amd.slice_layout import pack_slices
 
 pytestmark = pytest.mark.gpu
 
@@ -74,3 +75,32 @@ def test_the_128x192_tile_behind_the_input_gate():
         assert not local_gemm.gate_timed_out(ready)
     finally:
         lib.ms_set_variant(0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("S,k,m,n", [(2, 8, 8, 8), (3, 72, 136, 200), (8, 24, 300, 264), (5, 136, 520, 776), (16, 64, 257, 1544), (64, 16, 64, 136)])
+def test_products_on_row_slices_in_place_have_the_bits_of_copied_slices(S, k, m, n, dtype):
+    """Slices of one block to several K steps with and without a tail, rows and columns that end inside a tile, W a window of a wider
+    matrix, on the library's choice and on every tile."""
+    g = torch.Generator(device="cuda").manual_seed(S * k)
+    A = [torch.randn(m, k, generator=g, device="cuda").to(dtype) for _ in range(S)]
+    W = torch.randn(S * k, n + 16, generator=g, device="cuda").to(dtype)[:, 8:8 + n]
+    B = pack_slices(W, S, 8, 0)
+    lib = _lib.load()
+    try:
+        for variant in [0] + (list(range(1, 15)) + [204, 407] if dtype == torch.bfloat16 else [21, 22, 23, 24, 25, 224]):
+            assert lib.ms_set_variant(variant) == 0
+            try:
+                want = ms.gemm_os(A, B)
+            except ValueError:       # (a split that these sizes do not take)
+                continue
+            assert torch.equal(local_gemm.gemm_os_cyclic(A, W), want), variant
+    finally:
+        lib.ms_set_variant(0)
+
+
+def test_row_slices_in_place_are_checked():
+    a, w = torch.randn(16, 24, device="cuda").bfloat16(), torch.randn(48, 32, device="cuda").bfloat16()
+    for bad in (lambda: local_gemm.gemm_os_cyclic([a], w), lambda: local_gemm.gemm_os_cyclic([a, a], w.t()), lambda: local_gemm.gemm_os_cyclic([a[:, :12], a[:, :12]], w[:24])):
+        with pytest.raises(ValueError):
+            bad()

@@ -75,3 +75,15 @@ def test_sums_check_their_arguments():
     lib = _lib.load()
     assert lib.ms_gemm_ls_sum(None, 64, None, 64, 2, 16, 24, 32, None, 24, 1, 1, None, 0, ctypes.c_void_p(0)) == _lib.MS_ERR_ARG
     assert lib.ms_gemm_rs_sum(None, 64, None, 64, 65, 16, 24, 32, None, 24, 1, 1, None, 0, ctypes.c_void_p(0)) == _lib.MS_ERR_ARG
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("R,C,K,u,v,w", [(4, 2, 4, 3, 2, 1), (2, 4, 8, 5, 1, 2), (1, 2, 2, 7, 3, 1)])
+def test_global_output_stationary_products_have_the_bits_of_copied_slices(R, C, K, u, v, w, dtype):
+    g = torch.Generator(device="cuda").manual_seed(u)
+    m, n, k = R * u, R * C * 8 * v, R * C * K * 8 * w
+    X, W = torch.randn(m, k, generator=g, device="cuda").to(dtype), torch.randn(k, n, generator=g, device="cuda").to(dtype)
+    f = TP.SPMD(Mesh(create_device_mesh((R, C)), ("row", "col")), "meshflow").OS(K)
+    assert torch.equal(f(X, W), f._whole_mesh(X, W, K, 8))
+    f = TP.SPMD(Mesh(create_device_mesh((R, C)), ("row", "col")), "collective").OS(K)
+    assert torch.equal(f(X, W), f._whole_mesh(X, W, 1, 1))
