@@ -13,6 +13,7 @@
 #include "ms_gemm_bf16_big.hip.inc"
 #include "ms_gemm_bf16_x16.hip.inc"
 #include "ms_gemm_f32.hip.inc"
+#include "ms_gemm_f32_waves.hip.inc"
 
 // Every kernel variant is instantiated explicitly: with implicit instantiation alone the host
 // compiler leaves some of the launch stubs undefined.
@@ -83,6 +84,12 @@ MS_INSTANTIATE_F32(2, 2, 3, 3)
 MS_INSTANTIATE_F32(2, 2, 1, 3)
 MS_INSTANTIATE_F32(2, 2, 1, 2)
 #undef MS_INSTANTIATE_F32
+template __global__ void msk::gemm_f32_waves_kernel<true, false, true>(const msk::GemmArgs);
+template __global__ void msk::gemm_f32_waves_kernel<true, false, false>(const msk::GemmArgs);
+template __global__ void msk::gemm_f32_waves_kernel<true, true, true>(const msk::GemmArgs);
+template __global__ void msk::gemm_f32_waves_kernel<true, true, false>(const msk::GemmArgs);
+template __global__ void msk::gemm_f32_waves_kernel<false, false, true>(const msk::GemmArgs);
+template __global__ void msk::gemm_f32_waves_kernel<false, false, false>(const msk::GemmArgs);
 
 namespace {
 thread_local char g_err[512] = "";
@@ -101,7 +108,7 @@ namespace {
 thread_local int g_variant = 0;
 thread_local int g_splits = 0;    // forced split count of the contraction (0 = library default)
 thread_local int g_launches = 0;   // kernels launched by the last GEMM call of this thread
-thread_local int g_last_variant = 0;   // kernel variant of that call's first launch (bf16 tiles 1..VARIANTS, fp32 tiles F32_FIRST..F32_NARROW + 1)
+thread_local int g_last_variant = 0;   // kernel variant of that call's first launch (bf16 tiles 1..VARIANTS, fp32 tiles F32_FIRST..F32_WAVES)
 thread_local int g_last_splits = 1;    // and the number of ways it split the contraction
 thread_local int g_last_grid = 0;      // and its workgroup count
 thread_local int g_reserved_cus = 0;   // compute units the GEMM launches of this thread leave free (ms_set_reserved_cus)
@@ -338,6 +345,7 @@ struct Pick { int v, splits; double cost; };
 
 constexpr int VARIANTS = 14;
 constexpr int F32_FIRST = 21, F32_LAST = 25;      // ids of the fp32 kernel's tiles (ms_set_variant, MS_QUERY_LAST_VARIANT)
+constexpr int F32_WAVES = 28;                     // gemm_f32_waves_kernel
 constexpr int F32_NARROW = 26;                    // and of the two that only the chooser takes (64 x 192, 64 x 128; not ms_set_variant)
 struct TileShape { int bm, bn; };
 constexpr TileShape TILE_OF[VARIANTS + 1] = {{0, 0},     {256, 256}, {192, 192}, {128, 128}, {128, 192}, {256, 192},
@@ -518,10 +526,7 @@ int launch_bf16(const Problem &p, const DevFacts &dev, hipStream_t stream) {
 // of the 128 x 128 tile or of one of the 64-row tiles per compute unit
 int f32_split_refused(const Problem &p, const DevFacts &dev, int bm, int bn, int splits);
 
-template <int WGM, int WGN, int TM, int TN>
-int launch_f32_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, int id, bool share, int splits) {
-  constexpr int BM = 32 * TM * WGM, BN = 32 * TN * WGN;
-  msk::GemmArgs g;
+int fill_f32_args(const Problem &p, int bm, int bn, msk::GemmArgs &g, long &total) {
   memset(&g, 0, sizeof(g));
   for (int i = 0; i < p.na; i++) g.a[i] = p.a[i];
   for (int i = 0; i < p.nb; i++) g.b[i] = p.b[i];
@@ -532,9 +537,9 @@ int launch_f32_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, i
   g.b_by_chunk = p.flow == LS || (p.flow == RS && p.nb > 1);
   g.M = p.M; g.N = p.N; g.K = p.K;
   g.lda = p.lda; g.ldb = p.ldb; g.ldc = p.ldc; g.b_blk = p.b_blk ? p.b_blk : p.ldb * 8 * (p.in_dtype == MS_DTYPE_BF16 ? 2 : 4);
-  g.tiles_m = (p.M + BM - 1) / BM;
-  g.tiles_n = (p.N + BN - 1) / BN;
-  const long total = (long)g.tiles_m * g.tiles_n * g.nchunks;
+  g.tiles_m = (p.M + bm - 1) / bm;
+  g.tiles_n = (p.N + bn - 1) / bn;
+  total = (long)g.tiles_m * g.tiles_n * g.nchunks;
   if (total > 0x7FFFFFFF) return fail(MS_ERR_ARG, "problem has too many tiles");
   g.total_tiles = (int)total;
   g.group_m = 8;
@@ -542,6 +547,15 @@ int launch_f32_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, i
   g.chunk_done = p.chunk_done;
   g.slice_ready = p.slice_ready; g.gate_ticks = p.gate_ticks;
   g_last_tiles_per_chunk = g.tiles_m * g.tiles_n;
+  return MS_OK;
+}
+
+template <int WGM, int WGN, int TM, int TN>
+int launch_f32_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, int id, bool share, int splits) {
+  constexpr int BM = 32 * TM * WGM, BN = 32 * TN * WGN;
+  msk::GemmArgs g;
+  long total = 0;
+  if (int rc = fill_f32_args(p, BM, BN, g, total)) return rc;
   if (splits > 1) {
     const int why = f32_split_refused(p, dev, BM, BN, splits);
     if (why) return fail(MS_ERR_ARG, "contraction cannot be split %d ways here: %s", splits, SPLIT_REFUSALS[why]);
@@ -564,6 +578,29 @@ int launch_f32_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, i
     else msk::gemm_f32_tile_kernel<WGM, WGN, TM, TN, false, false, false><<<gd, bd, 0, stream>>>(g);
   }
   if (g_launches == 0) { g_last_grid = (int)gd.x; g_last_variant = id; g_last_splits = g.splits; }
+  g_launches++;
+  MS_HIP(hipGetLastError());
+  return MS_OK;
+}
+
+// gemm_f32_waves_kernel: 32 x 32 tiles, the contraction shared out over a workgroup's waves
+int launch_f32_waves(const Problem &p, const DevFacts &dev, hipStream_t stream) {
+  msk::GemmArgs g;
+  long total = 0;
+  if (int rc = fill_f32_args(p, 32, 32, g, total)) return rc;
+  const dim3 gd(balanced_grid(total, dev.cus)), bd(256);
+  const bool obf = p.out_dtype == MS_DTYPE_BF16;
+  if (p.flow == OS) {
+    if (obf) msk::gemm_f32_waves_kernel<true, false, true><<<gd, bd, 0, stream>>>(g);
+    else msk::gemm_f32_waves_kernel<true, false, false><<<gd, bd, 0, stream>>>(g);
+  } else if (p.flow == LS) {
+    if (obf) msk::gemm_f32_waves_kernel<true, true, true><<<gd, bd, 0, stream>>>(g);
+    else msk::gemm_f32_waves_kernel<true, true, false><<<gd, bd, 0, stream>>>(g);
+  } else {
+    if (obf) msk::gemm_f32_waves_kernel<false, false, true><<<gd, bd, 0, stream>>>(g);
+    else msk::gemm_f32_waves_kernel<false, false, false><<<gd, bd, 0, stream>>>(g);
+  }
+  if (g_launches == 0) { g_last_grid = (int)gd.x; g_last_variant = F32_WAVES; g_last_splits = 1; }
   g_launches++;
   MS_HIP(hipGetLastError());
   return MS_OK;
@@ -608,6 +645,7 @@ int launch_f32_id(int id, bool share, int splits, const Problem &p, const DevFac
     case F32_FIRST + 3: return launch_f32_tile<2, 2, 1, 1>(p, dev, stream, id, share, splits);
     case F32_NARROW: return launch_f32_tile<2, 2, 1, 3>(p, dev, stream, id, share, splits);
     case F32_NARROW + 1: return launch_f32_tile<2, 2, 1, 2>(p, dev, stream, id, share, splits);
+    case F32_WAVES: return launch_f32_waves(p, dev, stream);
     default: return launch_f32_tile<2, 2, 3, 3>(p, dev, stream, id, false, splits);
   }
 }
@@ -624,6 +662,14 @@ int launch_f32_id(int id, bool share, int splits, const Problem &p, const DevFac
 constexpr double F32_SPLIT_FIX = 1.2e6, F32_SPLIT_PART = 1e5, F32_SPLIT_PER_ELEMENT = 0.6;
 constexpr long F32_SPLIT_MIN_K = 256;      // contraction elements per split item, at least
 
+// gemm_f32_waves_kernel: a round of 32 x 32 tiles takes 0.605 us for every four steps of the contraction, and another round 2.5 us of its own
+// (fitted to 200 drawn products; 8 % off at the 95th percentile).  Chunk products take it wherever it is priced lower, output-stationary
+// ones up to 1536 contraction elements: beyond, the tiles above with their contraction split are level or ahead on nine in ten (256 x 256 x
+// 4096: 64 x 64 in eight parts 19.9 us, this 24.9).  The choice takes 1.007 of the better one's time in the geometric mean, 1.05 at the
+// 95th percentile.
+constexpr double F32_WAVES_STEPS4_US = 0.605, F32_WAVES_ROUND_US = 2.5, F32_UNIT_US = 3.5e-6;
+constexpr long F32_WAVES_OS_MAX_K = 1536;
+
 // the fp32 tile, whether its workgroups pair up on the units, and the split count with the lowest estimated cost (id 0: a
 // forced tile and split count that cannot be)
 struct F32Pick { int id, splits; bool share; };
@@ -631,7 +677,7 @@ F32Pick pick_f32(const Problem &p, const DevFacts &dev) {
   const long chunks = p.flow == OS ? 1 : p.S;
   const long total_k = (long)p.K * (p.flow == OS ? p.S : 1);
   const long ksteps = (long)((p.K + 31) / 32) * (p.flow == OS ? p.S : 1);
-  const bool forced_tile = g_variant >= F32_FIRST;
+  const bool forced_tile = g_variant >= F32_FIRST && g_variant != F32_WAVES;
   F32Pick best = {0, 1, false};
   double best_cost = 0.0;
   for (const F32Tile &t : F32_TILES) {
@@ -654,10 +700,16 @@ F32Pick pick_f32(const Problem &p, const DevFacts &dev) {
       if (best.id == 0 || cost < best_cost) { best = {t.id, splits, share}; best_cost = cost; }
     }
   }
+  if (!forced_tile && (p.flow != OS || total_k <= F32_WAVES_OS_MAX_K)) {
+    const long rounds = ((long)((p.M + 31) / 32) * ((p.N + 31) / 32) * chunks + dev.cus - 1) / dev.cus;
+    const double us = (double)(rounds * ((ksteps + 3) / 4)) * F32_WAVES_STEPS4_US + (double)(rounds - 1) * F32_WAVES_ROUND_US;
+    if (us / F32_UNIT_US / (double)total_k < best_cost) best = {F32_WAVES, 1, false};
+  }
   return best;
 }
 
 int launch_f32(const Problem &p, const DevFacts &dev, hipStream_t stream) {
+  if (g_variant == F32_WAVES) return launch_f32_waves(p, dev, stream);
   const F32Pick best = pick_f32(p, dev);
   if (best.id == 0) return fail(MS_ERR_ARG, "contraction cannot be split %d ways on fp32 tile %d here", g_splits, g_variant);
   return launch_f32_id(best.id, best.share, best.splits, p, dev, stream);
@@ -758,7 +810,7 @@ MS_API long ms_query(int what) {
 
 MS_API int ms_set_variant(int variant) {
   const int v = variant % 100, splits = variant / 100;
-  const bool known = v <= VARIANTS || (v >= F32_FIRST && v <= F32_LAST);
+  const bool known = v <= VARIANTS || (v >= F32_FIRST && v <= F32_LAST) || (v == F32_WAVES && splits == 0);
   if (variant < 0 || !known || splits == 1 || splits > SPLIT_MAX) return fail(MS_ERR_ARG, "ms_set_variant: unknown variant %d", variant);
   g_variant = v;
   g_splits = splits;
