@@ -183,6 +183,10 @@ int ms_gemm_os_cyclic(const void *const *A_slices, const void *W, int S,
                       int m, int n, int k_slice, int lda, int ldw,
                       void *C, int ldc, int in_dtype, int out_dtype,
                       void *workspace, size_t workspace_bytes, void *stream);
+/* ms_gemm_ls_ex on the same slices of W [S * n_slice, k]; n_slice is a multiple of 8. */
+int ms_gemm_ls_cyclic(const void *A, int lda, const void *W, int ldw, int S,
+                      int m, int n_slice, int k,
+                      void *const *Y_chunks, int ldy, int in_dtype, int out_dtype, void *stream);
 
 /* ms_gemm_ls_ex / ms_gemm_rs_ex for P mesh devices of equal shapes in one launch (the devices of a mesh row, LS, or of a mesh
  * column, RS, whose partial chunks one reduce-scatter adds up): A (LS) / W (RS) holds the P devices' own shards, the slice

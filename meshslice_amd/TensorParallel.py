@@ -121,6 +121,8 @@ def _spanning(parts: Sequence[torch.Tensor], axis: int):
     if isinstance(parts, _Line):
         return parts.panel if parts.axis == axis and parts.panel.stride(1) == 1 and parts.panel.shape[0] <= PANEL_MAX_ROWS else None
     p0 = parts[0]
+    if len(parts) == 1:
+        return p0 if p0.stride(1) == 1 and p0.shape[0] <= PANEL_MAX_ROWS else None
     step = p0.shape[1] if axis == 1 else p0.shape[0] * p0.stride(0)
     at, base = p0.storage_offset(), p0.untyped_storage().data_ptr()
     if p0.stride(1) != 1 or (axis == 1 and p0.stride(0) < len(parts) * p0.shape[1]):
@@ -171,6 +173,31 @@ def _gather_row_slices(peers: Sequence[torch.Tensor], K: int, B: int) -> List[to
     return [buf[k] for k in range(K)]
 
 
+def _addressable(t: torch.Tensor) -> bool:
+    """Whether the kernels can read a matrix as it stands."""
+    return _own(t) is t and t.stride(0) >= t.shape[1] and t.shape[0] * t.stride(0) * t.element_size() < 1 << 31
+
+
+def _readable(parts: Sequence[torch.Tensor], axis: int):
+    """_spanning's view where it is addressable, else None."""
+    whole = _spanning(parts, axis)
+    return whole if whole is not None and _addressable(whole) else None
+
+
+def _gathered(parts: Sequence[torch.Tensor], axis: int) -> torch.Tensor:
+    """_gather's matrix; shards that lie side by side in one matrix are that already and are not copied."""
+    whole = _readable(parts, axis)
+    return _gather(parts, axis) if whole is None else whole
+
+
+def _uncut(peers: Sequence[torch.Tensor], K: int, B: int):
+    """The gathered rows of which _gather_row_slices makes slices, where the kernels can read the slices inside them (blocks of eight rows
+    of one matrix), else None.  The peers' slices one below the other are the slices of the whole, as in _gather_col_slices; the copy
+    was 9 of 44 us of the LS body of one device of a 2x4 mesh, 4096 x 4096 x 8192 in eight slices."""
+    _need(peers[0].shape[0], K * B, "sliced extent")
+    return _readable(peers, 0) if B == 8 and K > 1 else None
+
+
 # ------------------------------------------------------------------------------------------------
 # per-device bodies.  X, W are the shard grids; (i, j) the device; the return value is what that
 # device holds after its local contractions.
@@ -178,20 +205,20 @@ def _gather_row_slices(peers: Sequence[torch.Tensor], K: int, B: int) -> List[to
 
 def Collective_OS(X, W, i, j, R, C, K, B):
     """reference TensorParallel.py:19-22: gather X over col, W over row, one contraction."""
-    Xi = _gather(_row(X, i, C), 1)
-    Wj = _gather(_column(W, j, R), 0)
+    Xi = _gathered(_row(X, i, C), 1)
+    Wj = _gathered(_column(W, j, R), 0)
     return local_gemm.gemm_os([Xi], [Wj])
 
 
 def Collective_LS(X, W, i, j, R, C, K, B):
     """reference :24-27: gather W over row; partial product X_ij @ Wj^T (input of psum_scatter)."""
-    Wj = _gather(_column(W, j, R), 0)
+    Wj = _gathered(_column(W, j, R), 0)
     return local_gemm.gemm_ls(_own(X[i][j]), [Wj])
 
 
 def Collective_RS(X, W, i, j, R, C, K, B):
     """reference :29-32: gather X over col; partial product Xi^T @ W_ij (input of psum_scatter)."""
-    Xi = _gather(_row(X, i, C), 1)
+    Xi = _gathered(_row(X, i, C), 1)
     return local_gemm.gemm_rs([Xi], _own(W[i][j]))
 
 
@@ -200,9 +227,11 @@ def MeshFlow_OS(X, W, i, j, R, C, K, B):
     if K == 1:
         raise ValueError("the sliced OS body is undefined for K == 1 (the reference adds slice 0 twice); "
                          "use algorithm='collective' for the unsliced product")
-    A_slices = _gather_col_slices(_row(X, i, C), K, B)
-    B_slices = _gather_row_slices(_column(W, j, R), K, B)
-    return local_gemm.gemm_os(A_slices, B_slices)
+    A_slices, peers = _gather_col_slices(_row(X, i, C), K, B), _column(W, j, R)
+    W_rows = _uncut(peers, K, B)
+    if W_rows is not None:
+        return local_gemm.gemm_os_cyclic(A_slices, W_rows)
+    return local_gemm.gemm_os(A_slices, _gather_row_slices(peers, K, B))
 
 
 _gather_streams = {}           # (device, handle of the product's stream) -> the stream for its gathers, or None
@@ -352,8 +381,11 @@ def MeshFlow_RS_overlap(X, W, i, j, R, C, K, B):
 
 def MeshFlow_LS(X, W, i, j, R, C, K, B):
     """reference :174-193: K gathered row slices of W; K fp32 partial chunks X_ij @ W_k^T."""
-    W_slices = _gather_row_slices(_column(W, j, R), K, B)
-    return local_gemm.gemm_ls(_own(X[i][j]), W_slices)
+    own, peers = _own(X[i][j]), _column(W, j, R)
+    W_rows = _uncut(peers, K, B)
+    if W_rows is not None:
+        return local_gemm.gemm_ls_cyclic(own, W_rows, K)
+    return local_gemm.gemm_ls(own, _gather_row_slices(peers, K, B))
 
 
 def MeshFlow_RS(X, W, i, j, R, C, K, B):
@@ -395,7 +427,7 @@ def _usable(views: Sequence[torch.Tensor]) -> List[torch.Tensor]:
 
 
 def _ring_os(algorithm, X, W, i, j, R, C):
-    Wj = _gather(_column(W, j, R), 0)                       # [Kd, n/C]
+    Wj = _gathered(_column(W, j, R), 0)                     # [Kd, n/C]
     _need(X[i][j].shape[1], 2, "columns of an X shard"); _need(Wj.shape[0], 2 * C, "gathered rows of W")
     h = Wj.shape[0] // C // 2
     order = _ring_order(algorithm, "os", R, C, i, j)
@@ -405,7 +437,7 @@ def _ring_os(algorithm, X, W, i, j, R, C):
 
 
 def _ring_ls(algorithm, X, W, i, j, R, C):
-    Wj = _gather(_column(W, j, R), 0)                       # [O, I/C]
+    Wj = _gathered(_column(W, j, R), 0)                     # [O, I/C]
     _need(Wj.shape[0], 2 * C, "gathered rows of W")
     h = Wj.shape[0] // C // 2
     order = _ring_order(algorithm, "ls", R, C, i, j)
@@ -523,6 +555,11 @@ def _fits_whole_mesh(dataflow, X, W, R, C, K) -> bool:
     return peers * K <= 64 and peers * m * n * 4 <= WHOLE_MESH_MAX_CHUNK_BYTES and m <= PANEL_MAX_ROWS and not any(v % q for v in aligned)
 
 
+def _whole_os(X, W, K, B):
+    """The output blocks of all devices are one product, whose gathered slices hold every device's."""
+    return local_gemm.gemm_os(slice_layout.pack_slices(X, K, B, 1), slice_layout.pack_slices(W, K, B, 0))
+
+
 def _whole_ls(X, W, C, K, B, sliced):
     """Every device's partial chunks in one launch and their reduce-scatters in another: mesh column j multiplies its columns
     of X (the rows of all mesh rows together) with its columns of the gathered slices of W; the sum over j is fp32 in peer
@@ -607,8 +644,8 @@ class ShardedMatmul:
         return run
 
     def _whole_mesh(self, X, W, K, B):
-        if self.dataflow == "os":      # (the output blocks of all devices are one product: the body on a mesh of one)
-            return self.body([[X]], [[W]], 0, 0, 1, 1, self.K, self.B)
+        if self.dataflow == "os":      # (the other bodies: on a mesh of one)
+            return _whole_os(X, W, K, B) if self.body is MeshFlow_OS and K > 1 else self.body([[X]], [[W]], 0, 0, 1, 1, self.K, self.B)
         return _whole_ls(X, W, self.C, K, B, self.sliced) if self.dataflow == "ls" else _whole_rs(X, W, self.R, K, B, self.sliced)
 
     def __call__(self, X: torch.Tensor, W: torch.Tensor) -> torch.Tensor:
@@ -617,11 +654,9 @@ class ShardedMatmul:
         K = self.K if self.sliced else 1
         B = self.B if self.sliced else 1
         if self.body in _WHOLE_MESH_BODIES[self.dataflow] and _fits_whole_mesh(self.dataflow, X, W, R, C, K):
-            # (the global result is the same whatever the slices: nothing is gathered, cut or interleaved for it, but for the order in
-            # which an OS product contracts them)
-            if self.body is Collective_OS and _own(X) is X and _own(W) is W:
-                return local_gemm.gemm_os([X], [W])
-            if self.body is MeshFlow_OS and K > 1 and B == 8 and _own(W) is W:
+            # (nothing that the kernels can read in place is gathered, cut or interleaved: an OS product's slices decide the order in which it
+            # contracts, the sums over a line are the same whatever the slices)
+            if self.body is MeshFlow_OS and K > 1 and B == 8 and _addressable(W):
                 return local_gemm.gemm_os_cyclic(slice_layout.pack_slices(X, K, B, 1), W)
             if self.dataflow == "ls" and _sums_on_chip(X, W):
                 return local_gemm.gemm_ls_sum(X, W, C)

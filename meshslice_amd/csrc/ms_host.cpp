@@ -187,6 +187,22 @@ PyObject *gemm_chunks(PyObject *const *args) {
   return rc == MS_OK ? chunk_list(buf) : nullptr;
 }
 
+// gemm_ls_cyclic(A, W, S) -> [chunks] or None
+PyObject *gemm_ls_cyclic(PyObject *const *args) {
+  void *y[MS_MAX_SLICES];
+  const at::Tensor *a = matrix(args[0]), *w = a ? matrix(args[1]) : nullptr;
+  const long S = PyLong_AsLong(args[2]);
+  if (!w || S < 1 || S > MS_MAX_SLICES || w->size(0) % S || a->size(1) != w->size(1) || a->scalar_type() != w->scalar_type() || a->device() != w->device()) return nullptr;
+  const Place p = place_of(*a);
+  if (!p.ok) return nullptr;
+  const int64_t m = a->size(0), n = w->size(0) / S;
+  at::Tensor buf = at::empty({S, m, n}, a->options().dtype(type_of(MS_DTYPE_F32)).requires_grad(false));
+  chunk_pointers(buf, y);
+  const int rc = ms_gemm_ls_cyclic(a->data_ptr(), (int)a->stride(0), w->data_ptr(), (int)w->stride(0), (int)S, (int)m, (int)n, (int)a->size(1), y, (int)n,
+                                   code_of(*a), MS_DTYPE_F32, p.stream);
+  return rc == MS_OK ? chunk_list(buf) : nullptr;
+}
+
 // gemm_ls_sum(X, W, P) / gemm_rs_sum(X, W, P) -> Tensor or None
 template <bool LS>
 PyObject *gemm_sum(PyObject *const *args) {
@@ -310,6 +326,7 @@ PyMethodDef g_methods[] = {
     MS_ENTRY("gemm_os_cyclic", gemm_os_cyclic, 2),
     MS_ENTRY("gemm_ls", gemm_chunks<true>, 3),
     MS_ENTRY("gemm_rs", gemm_chunks<false>, 3),
+    MS_ENTRY("gemm_ls_cyclic", gemm_ls_cyclic, 3),
     MS_ENTRY("gemm_ls_sum", gemm_sum<true>, 3),
     MS_ENTRY("gemm_rs_sum", gemm_sum<false>, 3),
     MS_ENTRY("pack_slices", pack_slices, 4),

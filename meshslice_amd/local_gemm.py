@@ -377,6 +377,25 @@ def gemm_rs(X_slices: Sequence[torch.Tensor], W: torch.Tensor,
     return call.out
 
 
+def gemm_ls_cyclic(A: torch.Tensor, W: torch.Tensor, S: int) -> List[torch.Tensor]:
+    """``gemm_ls`` on the S block-cyclic row slices of W (blocks of eight rows), read where they lie (``ms_gemm_ls_cyclic``): the fp32
+    chunks of ``gemm_ls(A, pack_slices(W, S, 8, 0))`` without that copy."""
+    chunks = _lib.host.gemm_ls_cyclic(A, W, S)
+    if chunks is not None:
+        return chunks
+    _check2d(A, "A"); _check2d(W, "W")
+    if S < 1 or W.shape[0] % S or A.shape[1] != W.shape[1] or A.dtype != W.dtype or A.device != W.device:
+        raise ValueError(f"shapes do not contract: {tuple(A.shape)} @ {S} row slices of {tuple(W.shape)}^T")
+    m, k = A.shape; n = W.shape[0] // S
+    out, ptrs = _chunk_views(torch.empty((S, m, n), dtype=torch.float32, device=A.device))
+    py, _ky = _lib.ptr_array(ptrs)
+    with _on(A.device):
+        rc = _lib.load().ms_gemm_ls_cyclic(ctypes.c_void_p(A.data_ptr()), A.stride(0), ctypes.c_void_p(W.data_ptr()), W.stride(0), S, m, n, k, py, n,
+                                           _dt(A), _dt(out[0]), _stream())
+    _lib.check(rc)
+    return out
+
+
 def gemm_ls_peers(A_shards: Sequence[torch.Tensor], W_slices_by_peer: Sequence[Sequence[torch.Tensor]]) -> List[List[torch.Tensor]]:
     """``gemm_ls`` of the P devices of a mesh row in one launch (``ms_gemm_ls_peers``): fp32 chunks
     ``[p][s] = A_shards[p] @ W_slices_by_peer[p][s]^T``, all shards and all slices of one shape and leading dimension."""
