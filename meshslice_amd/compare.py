@@ -6,7 +6,7 @@
     long shapes (``--small``: ten products from 1024^3 to 3072^3).
 
 ``python3 -m meshslice_amd.compare chooser [--cases N] [--slices S] [--seed K]``
-    how far the default tile choice is from the best of ten forced tile variants, on N shapes drawn at random per
+    how far the default tile choice is from the best of twelve forced tile variants, on N shapes drawn at random per
     dataflow (dimensions 512..16384, 0.02..3 TFLOP per product), S slices each.
 
 ``python3 -m meshslice_amd.compare fp32``
@@ -32,7 +32,7 @@ LARGE = [(1024,) * 3, (2048,) * 3, (3072,) * 3, (4096,) * 3, (5120,) * 3, (6144,
          (8192, 8192, 2048), (2048, 8192, 8192), (4096, 11008, 4096), (16384, 4096, 4096)]
 SMALL = [(1024,) * 3, (1536,) * 3, (2048,) * 3, (2560,) * 3, (3072,) * 3, (2048, 4096, 2048), (2048, 2048, 8192), (1024, 4096, 4096),
          (2048, 1536, 3072), (4096, 1536, 1536)]
-FORCED = (3, 5, 6, 7, 8, 9, 11, 12, 13, 14)
+FORCED = (2, 3, 4, 5, 6, 7, 8, 9, 11, 12, 13, 14)
 SIZES = [512, 768, 1024, 1536, 2048, 2560, 3072, 4096, 5120, 6144, 7168, 8192, 10240, 12288, 16384]
 
 
