@@ -242,6 +242,52 @@ void launch_one(dim3 gd, dim3 bd, hipStream_t stream, const msk::GemmArgs &g) {
 }
 
 using msi::balanced_grid;
+
+constexpr int ROWS_WALKED = 8;             // tile rows walked together
+constexpr double RUNS_MIN_GAIN = 0.9;      // operand panels that runs may need, of those that taking turns does
+constexpr long RUNS_MIN_SPLIT_K = 700;     // contraction elements per part, at least
+
+// Whether the eight XCDs take runs of neighbouring items (xcd_slot) or turns, item i on XCD i % 8.  A grid that is a multiple of eight takes runs.
+// Another one takes them where that lets the XCDs' L2s fetch at least a tenth fewer operand panels, counted here: on 1265 unsplit grids of that
+// kind (230 drawn products, every tile) runs take 0.89 of the time where they fetch less than half, 0.95 at 0.5 to 0.7, 0.98 at 0.8 to 0.9, and
+// 1.02 where they fetch more (tall outputs, whose eight tile rows a walk puts on eight XCDs by turns).  268 x 10288 x 3120 on 243 tiles of 128x128 45.7 -> 31.7 us,
+// 552 x 7144 x 6112 on 190 of 128x192 90 -> 64.  The parts of a split product take them from some 700 contraction elements a part (0.92
+// at 1000 to 1500); shorter ones are all exchange, which runs slow down (1.06 below 300).
+bool xcds_take_runs(const msk::GemmArgs &g, int grid, int bm, int bn, bool a_by_chunk, bool b_by_chunk) {
+  if (grid % 8 == 0) return true;
+  const long k_part = (long)g.K * g.nkslices / g.splits;
+  if (grid > 1024 || (g.splits > 1 && k_part < RUNS_MIN_SPLIT_K)) return false;
+  // panel numbers of the first round's items, in the order of the kernels' walk
+  short a[1024], b[1024];
+  int n = 0, na = 0, nb = 0;      // panels of the parts and chunks before this one
+  for (int s = 0; s < g.splits && n < grid; s++, na += g.tiles_m, nb += g.tiles_n) {
+    for (int c = 0; c < g.nchunks && n < grid; c++) {
+      if (c && a_by_chunk) na += g.tiles_m;
+      if (c && b_by_chunk) nb += g.tiles_n;
+      for (int m0 = 0; m0 < g.tiles_m && n < grid; m0 += ROWS_WALKED)
+        for (int j = 0; j < g.tiles_n && n < grid; j++)
+          for (int i = m0; i < g.tiles_m && i < m0 + ROWS_WALKED && n < grid; i++, n++) { a[n] = (short)((na + i) & 2047); b[n] = (short)((nb + j) & 2047); }
+    }
+  }
+  long fetched[2];
+  for (int runs = 0; runs < 2; runs++) {
+    signed char seen_a[2048], seen_b[2048];
+    memset(seen_a, -1, sizeof(seen_a));
+    memset(seen_b, -1, sizeof(seen_b));
+    long rows = 0, cols = 0;
+    for (int x = 0, first = 0; x < 8; x++) {
+      const int count = grid / 8 + (x < grid % 8);
+      for (int k = 0; k < count; k++) {
+        const int w = runs ? first + k : x + 8 * k;
+        if (seen_a[a[w]] != x) { seen_a[a[w]] = (signed char)x; rows++; }
+        if (seen_b[b[w]] != x) { seen_b[b[w]] = (signed char)x; cols++; }
+      }
+      first += count;
+    }
+    fetched[runs] = rows * bm + cols * bn;
+  }
+  return (double)fetched[1] < RUNS_MIN_GAIN * (double)fetched[0];
+}
 constexpr double PARTIAL_ROUND_LOSS = 0.6;
 
 // Two workgroups of the 128x128 kernel fit one compute unit (64 KB of LDS and at most 220 registers per lane each) and
@@ -273,7 +319,6 @@ int launch_bf16_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, 
   const long total = (long)g.tiles_m * g.tiles_n * g.nchunks;
   if (total > 0x7FFFFFFF) return fail(MS_ERR_ARG, "problem has too many tiles");
   g.total_tiles = (int)total;
-  g.group_m = 8;
   g.splits = 1;
   g.chunk_done = p.chunk_done;
   g.slice_ready = p.slice_ready; g.gate_ticks = p.gate_ticks;
@@ -287,6 +332,8 @@ int launch_bf16_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, 
   }
   const long items = total * g.splits;
   const int grid = balanced_grid(items, workgroups_per_unit(variant) * dev.cus);
+  g.group_m = ROWS_WALKED;
+  g.xcd_runs = xcds_take_runs(g, grid, BM, BN, g.a_by_chunk, g.b_by_chunk);
   dim3 gd(grid), bd(WGM * WGN * 64);
   const bool obf = p.out_dtype == MS_DTYPE_BF16;
   g.act = p.act; g.res = p.res; g.ldr = p.ldr; g.row_sum = p.row_sum; g.row_sumsq = p.row_sumsq;
@@ -542,7 +589,6 @@ int fill_f32_args(const Problem &p, int bm, int bn, msk::GemmArgs &g, long &tota
   total = (long)g.tiles_m * g.tiles_n * g.nchunks;
   if (total > 0x7FFFFFFF) return fail(MS_ERR_ARG, "problem has too many tiles");
   g.total_tiles = (int)total;
-  g.group_m = 8;
   g.splits = 1;
   g.chunk_done = p.chunk_done;
   g.slice_ready = p.slice_ready; g.gate_ticks = p.gate_ticks;
@@ -565,6 +611,8 @@ int launch_f32_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, i
   }
   const long items = total * g.splits;
   const int grid = !(share && WGM * WGN == 4) ? balanced_grid(items, dev.cus) : items <= 2L * dev.cus ? (int)items : balanced_grid(items, 2 * dev.cus);
+  g.group_m = ROWS_WALKED;
+  g.xcd_runs = xcds_take_runs(g, grid, BM, BN, g.a_by_chunk, g.b_by_chunk);
   dim3 gd(grid), bd(WGM * WGN * 64);
   const bool obf = p.out_dtype == MS_DTYPE_BF16;
   if (p.flow == OS) {
@@ -589,6 +637,8 @@ int launch_f32_waves(const Problem &p, const DevFacts &dev, hipStream_t stream) 
   long total = 0;
   if (int rc = fill_f32_args(p, 32, 32, g, total)) return rc;
   const dim3 gd(balanced_grid(total, dev.cus)), bd(256);
+  g.group_m = ROWS_WALKED;
+  g.xcd_runs = xcds_take_runs(g, (int)gd.x, 32, 32, g.a_by_chunk, g.b_by_chunk);
   const bool obf = p.out_dtype == MS_DTYPE_BF16;
   if (p.flow == OS) {
     if (obf) msk::gemm_f32_waves_kernel<true, false, true><<<gd, bd, 0, stream>>>(g);

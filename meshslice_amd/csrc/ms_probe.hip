@@ -154,7 +154,7 @@ MS_API int ms_probe_os_parts(int skip, const void *const *A_slices, const void *
   g.M = m; g.N = n; g.K = k_slice; g.lda = lda; g.ldb = ldb; g.ldc = ldc; g.b_blk = ldb * 16;
   g.tiles_m = (m + 255) / 256; g.tiles_n = (n + 383) / 384;
   g.total_tiles = g.tiles_m * g.tiles_n;
-  g.group_m = 8; g.splits = 1;
+  g.group_m = 8; g.xcd_runs = 1; g.splits = 1;
   const dim3 gd(msi::balanced_grid(g.total_tiles, prop.multiProcessorCount)), bd(256);
   hipStream_t st = (hipStream_t)stream;
   auto launch = [&]() -> bool {
