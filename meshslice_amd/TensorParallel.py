@@ -654,18 +654,18 @@ class ShardedMatmul:
         K = self.K if self.sliced else 1
         B = self.B if self.sliced else 1
         if self.body in _WHOLE_MESH_BODIES[self.dataflow] and _fits_whole_mesh(self.dataflow, X, W, R, C, K):
-            # (nothing that the kernels can read in place is gathered, cut or interleaved: an OS product's slices decide the order in which it
-            # contracts, the sums over a line are the same whatever the slices)
-            if self.body is MeshFlow_OS and K > 1 and B == 8 and _addressable(W):
-                return local_gemm.gemm_os_cyclic(slice_layout.pack_slices(X, K, B, 1), W)
-            if self.dataflow == "ls" and _sums_on_chip(X, W):
-                return local_gemm.gemm_ls_sum(X, W, C)
-            if self.dataflow == "rs" and _sums_on_chip(X, W):
-                return local_gemm.gemm_rs_sum(X, W, R)
             try:
+                # (nothing that the kernels can read in place is gathered, cut or interleaved: an OS product's slices decide the order in which it
+                # contracts, the sums over a line are the same whatever the slices)
+                if self.body is MeshFlow_OS and K > 1 and B == 8 and _addressable(W):
+                    return local_gemm.gemm_os_cyclic(slice_layout.pack_slices(X, K, B, 1), W)
+                if self.dataflow == "ls" and _sums_on_chip(X, W):
+                    return local_gemm.gemm_ls_sum(X, W, C)
+                if self.dataflow == "rs" and _sums_on_chip(X, W):
+                    return local_gemm.gemm_rs_sum(X, W, R)
                 return self._whole_mesh(X, W, K, B)
             except torch.OutOfMemoryError:
-                pass       # the gathered operands and chunks of all mesh lines do not fit beside the caller's tensors: one line's may
+                pass       # what all mesh lines need at once (slices of all of X, gathered operands, chunks) does not fit beside the caller's tensors: one line's may
         Xs, Ws = _shards(X, R, C), _shards(W, R, C)
         run = lambda i, j: self.body(Xs, Ws, i, j, R, C, self.K, self.B)
         if self.dataflow == "os":

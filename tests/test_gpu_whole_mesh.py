@@ -118,11 +118,12 @@ def test_peers_products_on_every_tile_equal_the_single_devices(variant, flow, P,
 
 
 @pytest.mark.parametrize("flow", ["os", "ls", "rs"])
-def test_a_product_that_fits_memory_only_line_by_line_still_runs(flow):
-    """An allowance below what the partial chunks (LS, RS: 512 MiB) or the gathered operands (OS: 128 MiB) of the whole mesh
-    take; a mesh line's (32 MiB, 16 MiB), the output's parts and the output fit it."""
-    R, C, K = (1, 8, 2) if flow == "os" else (16, 2, 2) if flow == "ls" else (2, 16, 2)
-    m, n, k, allowance = (64, 16384, 4096, 100) if flow == "os" else (8192, 8192, 256, 420)
+def test_a_product_that_fits_memory_only_line_by_line_still_runs(flow, monkeypatch):
+    """An allowance below what the partial chunks (LS, RS: 512 MiB) or the slices of all of X (OS: 128 MiB) take on the whole
+    mesh; a mesh line's (32 MiB, 16 MiB), the output's parts and the output fit it.  The bodies have run device by device then."""
+    monkeypatch.setattr(TP, "_sums_on_chip", lambda *a: False)      # (sums in registers need no chunks)
+    R, C, K = (8, 1, 2) if flow == "os" else (16, 2, 2) if flow == "ls" else (2, 16, 2)
+    m, n, k, allowance = (65536, 64, 1024, 64) if flow == "os" else (8192, 8192, 256, 420)
     a, b = {"os": ((m, k), (k, n)), "ls": ((m, k), (n, k)), "rs": ((k, n), (k, m))}[flow]
     f = getattr(TP.SPMD(Mesh(create_device_mesh((R, C)), ("row", "col")), "meshflow"), flow.upper())(K)
     X, W = torch.randn(a, device="cuda").bfloat16(), torch.randn(b, device="cuda").bfloat16()
@@ -140,7 +141,29 @@ def test_a_product_that_fits_memory_only_line_by_line_still_runs(flow):
         torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (allowance << 20)) / total)
         with pytest.raises(torch.OutOfMemoryError):
             f._whole_mesh(X, W, K, 8)
+        sharded = []
+        monkeypatch.setattr(TP, "_shards", lambda *a, shards=TP._shards: sharded.append(1) or shards(*a))
         got = f(X, W)
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
+    assert sharded      # (cut for the devices' own bodies)
     assert torch.equal(got, want) if flow != "os" else float((got.double() - want.double()).norm() / want.double().norm()) <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("flow", ["os", "ls", "rs"])
+def test_the_calls_that_need_no_chunks_fall_back_too(flow, monkeypatch):
+    """Where a product in one launch finds no memory for its slices, workspace or output the devices' bodies run."""
+    f = getattr(TP.SPMD(Mesh(create_device_mesh((2, 2)), ("row", "col")), "meshflow"), flow.upper())(2)
+    X, W = _operands(flow, 2, 2, 2, 8, 3, 1, 1, torch.bfloat16)
+    want = f(X, W)
+    name = {"os": "gemm_os_cyclic", "ls": "gemm_ls_sum", "rs": "gemm_rs_sum"}[flow]
+    refused, call = [], getattr(local_gemm, name)
+
+    def once(*a):
+        if refused:
+            return call(*a)
+        refused.append(1)
+        raise torch.OutOfMemoryError("no memory")
+    monkeypatch.setattr(local_gemm, name, once)
+    got = f(X, W)
+    assert refused and float((got.double() - want.double()).norm() / want.double().norm()) <= 2.0 ** -8
