@@ -98,12 +98,15 @@ def _need(v: int, d: int, what: str) -> None:
         raise ValueError(f"{what} = {v} is not a multiple of {d}")
 
 
+def _aligned(block: torch.Tensor) -> bool:
+    """Whether a matrix's first element and its rows are 16-byte aligned."""
+    return block.stride(1) == 1 and block.data_ptr() % 16 == 0 and (block.stride(0) * block.element_size()) % 16 == 0
+
+
 def _own(block: torch.Tensor) -> torch.Tensor:
-    """A device's shard as the kernels can address it: the view itself when its first element and its rows
-    are 16-byte aligned (a real device's shard is its own buffer), else a contiguous copy."""
-    if block.stride(1) == 1 and block.data_ptr() % 16 == 0 and (block.stride(0) * block.element_size()) % 16 == 0:
-        return block
-    return block.contiguous()
+    """A device's shard as the kernels can address it: the view itself when it is aligned (a real device's shard is its own
+    buffer), else a contiguous copy."""
+    return block if _aligned(block) else block.contiguous()
 
 
 def _gather(parts: Sequence[torch.Tensor], axis: int) -> torch.Tensor:
@@ -175,7 +178,7 @@ def _gather_row_slices(peers: Sequence[torch.Tensor], K: int, B: int) -> List[to
 
 def _addressable(t: torch.Tensor) -> bool:
     """Whether the kernels can read a matrix as it stands."""
-    return _own(t) is t and t.stride(0) >= t.shape[1] and t.shape[0] * t.stride(0) * t.element_size() < 1 << 31
+    return _aligned(t) and t.stride(0) >= t.shape[1] and t.shape[0] * t.stride(0) * t.element_size() < 1 << 31
 
 
 def _readable(parts: Sequence[torch.Tensor], axis: int):
@@ -421,7 +424,7 @@ def _ring_order(algorithm: str, dataflow: str, R: int, C: int, i: int, j: int):
 def _usable(views: Sequence[torch.Tensor]) -> List[torch.Tensor]:
     """The views themselves if the kernels can address all of them in place, else contiguous copies of all
     (slices of one call share a leading dimension)."""
-    if all(_own(v) is v for v in views):
+    if all(_aligned(v) for v in views):
         return list(views)
     return [v.contiguous() for v in views]
 

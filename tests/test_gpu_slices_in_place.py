@@ -80,3 +80,22 @@ def test_expanded_operands_are_gathered_as_before():
     X, W = (torch.randn(1, 64, device="cuda").bfloat16().expand(64, 64) for _ in range(2))
     want = f(X.contiguous(), W.contiguous())
     assert torch.equal(f(X, W), want) and torch.equal(f.device(1, 0)(X, W), want[32:, :32])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("flow,algorithm,device", [("os", "meshflow", False), ("os", "collective", False), ("os", "collective", True), ("ls", "collective", True),
+                                                   ("ls", "meshflow", True), ("rs", "collective", True)])
+def test_contiguous_operands_at_an_odd_base_are_copied(flow, algorithm, device, dtype):
+    """Whole rows of a flat buffer from its second element on: every pitch fits, the base does not."""
+    g = torch.Generator(device="cuda").manual_seed(6)
+
+    def odd(r, c, at=1):
+        return torch.randn(r * c + at, generator=g, device="cuda").to(dtype)[at:].view(r, c)
+    # the operand that is gathered lies at the odd base; a device's own shard has to be aligned
+    m, n, k = 64, 96, 128
+    X, W = {"os": (odd(m, k), odd(k, n)), "ls": (odd(m, k, 0), odd(n, k)), "rs": (odd(k, m), odd(k, n, 0))}[flow]
+    f = getattr(tp.SPMD(Mesh(create_device_mesh((2, 1) if flow == "ls" else (1, 1) if flow == "os" else (1, 2)), ("row", "col")), algorithm, 8), flow.upper())(2)
+    f = f.device(0, 0) if device else f
+    want = f(X.clone(), W.clone())
+    got = f(X, W)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

@@ -378,3 +378,16 @@ def test_which_meshes_run_as_one_product():
     assert not fits("os", row(1 << 15, 1 << 15), row(1 << 15, 64), 2, 4, 4)         # 2 GiB
     assert not fits("ls", row(1 << 14, 64), row(1 << 15, 64), 1, 4, 8)              # 8 GiB of chunks
     assert not fits("os", row(TP.PANEL_MAX_ROWS + 8, 64), row(64, 64), 2, 4, 2)
+
+
+# ---------------------------------------------------------------- what the kernels can read where it lies
+def test_asking_whether_a_matrix_can_be_read_in_place_copies_nothing(monkeypatch):
+    """Bases and pitches that are and are not whole 16 bytes; a matrix that is contiguous at an odd base is no exception."""
+    def copied(*a, **k):
+        raise AssertionError("a copy was made")
+    buf = torch.zeros(4096, dtype=torch.bfloat16)
+    assert buf.data_ptr() % 16 == 0
+    monkeypatch.setattr(torch.Tensor, "contiguous", copied)
+    assert TP._addressable(buf[:512].view(8, 64)) and TP._addressable(buf.view(64, 64)[:, 8:24])
+    for t in (buf[1:513].view(8, 64), buf.view(64, 64)[:, 1:25], buf[:8 * 60].view(8, 60), buf[:64].view(8, 8).t(), buf[:64].expand(4, 64)):
+        assert not TP._addressable(t)
