@@ -122,7 +122,8 @@ def _spanning(parts: Sequence[torch.Tensor], axis: int):
     """The one view that covers ``parts`` when they are neighbouring blocks of one matrix in axis order (the shards of a
     global operand are), else None."""
     if isinstance(parts, _Line):
-        return parts.panel if parts.axis == axis and parts.panel.stride(1) == 1 and parts.panel.shape[0] <= PANEL_MAX_ROWS else None
+        p = parts.panel      # (rows that overlap, a window slid over a buffer, are rows of the shards only)
+        return p if parts.axis == axis and p.stride(1) == 1 and p.shape[0] <= PANEL_MAX_ROWS and (axis == 0 or p.stride(0) >= p.shape[1]) else None
     p0 = parts[0]
     if len(parts) == 1:
         return p0 if p0.stride(1) == 1 and p0.shape[0] <= PANEL_MAX_ROWS else None

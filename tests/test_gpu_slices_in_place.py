@@ -99,3 +99,18 @@ def test_contiguous_operands_at_an_odd_base_are_copied(flow, algorithm, device, 
     want = f(X.clone(), W.clone())
     got = f(X, W)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("flow,algorithm", [("os", "meshflow"), ("rs", "meshflow"), ("os", "collective"), ("rs", "collective"), ("os", "meshflow_overlap")])
+def test_windows_slid_over_a_buffer(flow, algorithm, dtype):
+    """Rows closer together than they are long, farther apart than a shard's: every shard is a matrix, the whole is none."""
+    g = torch.Generator(device="cuda").manual_seed(8)
+    m, n, k = 64, 64, 256
+    r, c = (k, m) if flow == "rs" else (m, k)
+    step = c // 2
+    X = torch.randn(r * step + c, generator=g, device="cuda").to(dtype).as_strided((r, c), (step, 1))
+    W = torch.randn(k, n, generator=g, device="cuda").to(dtype)
+    f = getattr(tp.SPMD(Mesh(create_device_mesh((1, 4)), ("row", "col")), algorithm, 8), flow.upper())(2).device(0, 1)
+    got, want = f(X, W), f(X.contiguous(), W)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
