@@ -212,6 +212,11 @@ int ms_gemm_rs_sum(const void *const *X, int ldx, const void *const *W, int ldw,
                    void *C, int ldc, int in_dtype, int out_dtype,
                    void *workspace, size_t workspace_bytes, void *stream);
 
+/* Whether the library expects the sum over a mesh line sooner from ms_gemm_ls_sum (rs: ms_gemm_rs_sum) than from ms_gemm_*_peers on S slices and
+ * ms_unpack_chunks: 1 or 0, from the extents alone (P devices of k contraction elements each, an output of m x n); 1 too for
+ * extents that it cannot price.  The bits are the same either way. */
+int ms_prefers_sum(int rs, int P, int S, int m, int n, int k);
+
 /* ms_gemm_ls_ex / ms_gemm_rs_ex with completion counters, so that the reduce-scatter of chunk s (the psum_scatter that
  * follows each einsum in MeshFlow_LS / MeshFlow_RS, TensorParallel.py:182-189, :204-212) can start while the later
  * chunks are still being computed.  chunk_done points to S unsigned counters in device memory, zero before the call;

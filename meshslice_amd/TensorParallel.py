@@ -586,11 +586,10 @@ def _whole_rs(X, W, R, K, B, sliced):
 
 
 def _sums_on_chip(X, W) -> bool:
-    """Whether a line's partial sums are added up inside the product (local_gemm.gemm_ls_sum, gemm_rs_sum) instead of as fp32 chunks
-    in memory: bf16 operands that the kernel can address in place.  The sum's tiles are slower per FLOP than the 256x384 one, which has no
-    registers left for totals, but write a tenth of the bytes: LS 2048 x 3072 x 12288 of four devices 172 -> 128 us, RS 3072 x 12288 x 2048
-    of two 251 -> 131, LS 4096 x 4096 x 24576 of two (12288 contraction elements a device) still 686 -> 655, small ones a quarter
-    of the launches (512 x 256 x 1024 on 4x2 97 -> 23 us)."""
+    """Whether a line's partial sums can be added up inside the product (local_gemm.gemm_ls_sum, gemm_rs_sum) instead of as fp32 chunks
+    in memory: bf16 operands that the kernel can address in place.  That writes a tenth of the bytes: LS 2048 x 3072 x 12288 of four devices
+    172 -> 128 us, RS 3072 x 12288 x 2048 of two 251 -> 131, small ones a quarter of the launches (512 x 256 x 1024 on 4x2 97 -> 23 us).
+    Where the contraction is long it can be the slower way: local_gemm.prefers_sum prices both."""
     return X.dtype == torch.bfloat16 and all(t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0 and t.stride(0) >= t.shape[1] for t in (X, W))
 
 
@@ -663,9 +662,9 @@ class ShardedMatmul:
                 # contracts, the sums over a line are the same whatever the slices)
                 if self.body is MeshFlow_OS and K > 1 and B == 8 and _addressable(W):
                     return local_gemm.gemm_os_cyclic(slice_layout.pack_slices(X, K, B, 1), W)
-                if self.dataflow == "ls" and _sums_on_chip(X, W):
+                if self.dataflow == "ls" and _sums_on_chip(X, W) and local_gemm.prefers_sum("ls", C, K, X.shape[0], W.shape[0], X.shape[1] // C):
                     return local_gemm.gemm_ls_sum(X, W, C)
-                if self.dataflow == "rs" and _sums_on_chip(X, W):
+                if self.dataflow == "rs" and _sums_on_chip(X, W) and local_gemm.prefers_sum("rs", R, K, X.shape[1], W.shape[1], X.shape[0] // R):
                     return local_gemm.gemm_rs_sum(X, W, R)
                 return self._whole_mesh(X, W, K, B)
             except torch.OutOfMemoryError:

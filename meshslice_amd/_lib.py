@@ -37,7 +37,7 @@ LIB_PATH = os.path.join(_HERE, "libmeshslice_hip.so")
 
 EXPORTS = (
     "ms_version", "ms_last_error", "ms_query", "ms_set_variant",
-    "ms_gemm_os", "ms_gemm_os_fused", "ms_gemm_os_ws", "ms_gemm_os_noalloc", "ms_gemm_os_cyclic", "ms_gemm_os_gated", "ms_gemm_ls_gated", "ms_gemm_rs_gated", "ms_signal_set", "ms_workspace_bytes", "ms_workspace_init", "ms_time_os_ws", "ms_gemm_ls", "ms_gemm_rs", "ms_gemm_ls_ex", "ms_gemm_rs_ex", "ms_gemm_ls_cyclic", "ms_gemm_ls_peers", "ms_gemm_rs_peers", "ms_gemm_ls_sum", "ms_gemm_rs_sum", "ms_gemm_ls_signal", "ms_gemm_rs_signal", "ms_set_reserved_cus",
+    "ms_gemm_os", "ms_gemm_os_fused", "ms_gemm_os_ws", "ms_gemm_os_noalloc", "ms_gemm_os_cyclic", "ms_gemm_os_gated", "ms_gemm_ls_gated", "ms_gemm_rs_gated", "ms_signal_set", "ms_workspace_bytes", "ms_workspace_init", "ms_time_os_ws", "ms_gemm_ls", "ms_gemm_rs", "ms_gemm_ls_ex", "ms_gemm_rs_ex", "ms_gemm_ls_cyclic", "ms_gemm_ls_peers", "ms_gemm_rs_peers", "ms_gemm_ls_sum", "ms_gemm_rs_sum", "ms_prefers_sum", "ms_gemm_ls_signal", "ms_gemm_rs_signal", "ms_set_reserved_cus",
     "ms_time_os", "ms_time_ls", "ms_time_rs", "ms_time_ls_ex", "ms_time_rs_ex",
     "ms_pack_slices", "ms_unpack_chunks", "ms_probe_mfma_stream", "ms_probe_mfma_stream_ex",
     "ms_probe_os_parts", "ms_probe_l2_lds_stream",
@@ -105,6 +105,9 @@ def _declare(lib):
     lib.ms_gemm_ls_peers.argtypes = lib.ms_gemm_rs_peers.argtypes = [vpp, c_int, vpp, c_int, c_int, c_int, c_int, c_int, c_int, vpp, c_int, c_int, c_int, c_vp]
     # operands and pitches, P, m, n, k, C, ldc, in_dtype, out_dtype, workspace, workspace_bytes, stream
     lib.ms_gemm_ls_sum.argtypes = lib.ms_gemm_rs_sum.argtypes = [vpp, c_int, vpp, c_int, c_int, c_int, c_int, c_int, c_vp, c_int, c_int, c_int, c_vp, ctypes.c_size_t, c_vp]
+    # rs, P, S, m, n, k
+    lib.ms_prefers_sum.argtypes = [c_int] * 6
+    lib.ms_prefers_sum.restype = c_int
     # ..., in_dtype, out_dtype, chunk_done, tiles_per_chunk, stream
     lib.ms_gemm_ls_signal.argtypes = ls_args[:-1] + [c_int, c_vp, ctypes.POINTER(c_int), c_vp]
     lib.ms_gemm_rs_signal.argtypes = rs_args[:-1] + [c_int, c_vp, ctypes.POINTER(c_int), c_vp]

@@ -1145,6 +1145,53 @@ int run_sum(Problem p, void *workspace, size_t workspace_bytes, void *stream, co
 }
 }  // namespace
 
+// Whether the sum over a mesh line of P devices is priced lower in registers (one launch on the tiles that carry it) than in fp32 chunks that a
+// layout kernel adds up (the chunk product on any tile, its chunks out and in again, the copy of the operand that is sliced or gathered for
+// it, two more launches).  The first is one workgroup a tile for the whole contraction (or one a device, for a few line lengths): few output
+// tiles under a long contraction leave the device idle, which P times as many chunk tiles do not; and its tiles are slower per FLOP than
+// the 256x384 one, which counts where the contraction makes up for the chunks' bytes.  Measured on 1404 products drawn and listed (m and n
+// 64 to 16384, 64 to 24576 contraction elements a device, 2 to 16 devices, one to eight slices), registers -> chunks: RS 256 x 640 of sixteen
+// devices of 12864 elements 1699 -> 180 us, 1024 x 4096 of four of 16384 589 -> 454, 8192 x 12288 of two of 8192 2645 -> 2409; RS 3072 x 12288
+// x 1024 of two 76 <- 149, LS 8192 x 8192 of two of 8192 1696 <- 1713.  The choice takes 1.003 of the better one's time in the geometric mean
+// and 1.14 at the 99th percentile (1.001 and at most 1.17 on 600 products that it was not fitted to); registers always would take 1.048 and 3.5,
+// chunks always 1.86.  Up to SUM_ALWAYS_K contraction elements of the whole line registers were never behind.
+namespace {
+constexpr long SUM_ALWAYS_K = 10240;
+constexpr double SUM_UNIT_US = 3.5e-7;                                       // pick_variant's unit
+constexpr double SUM_SCALE = 0.93, SUM_LAUNCH_US = 3.0;
+constexpr double SUM_RS_PART_LINES = 0.08;                                   // RS rows that are no whole 128-byte lines: half of it for each operand
+constexpr double SUM_COLD_US_PER_MB = 0.05;                                  // operands beyond the 256 MB of the last-level cache
+constexpr double CHUNK_SCALE = 0.95, CHUNK_LAUNCHES_US = 30.0;
+constexpr double CHUNK_US_PER_MB = 0.33, CHUNK_COPY_US_PER_MB = 0.3;         // chunk bytes out and in; the operand that is copied
+// the host's part of the chunk path, which a stream of such calls cannot go below
+constexpr double CHUNK_HOST_US = 35.0, CHUNK_HOST_PEER_US = 5.0, CHUNK_HOST_SLICE_US = 2.6;
+constexpr double CHUNK_MARGIN = 0.93;                                        // chunks are taken where they are this much cheaper
+}  // namespace
+
+MS_API int ms_prefers_sum(int rs, int P, int S, int m, int n, int k) {
+  if (P < 2 || P > MS_MAX_SLICES || S < 1 || (long)P * S > MS_MAX_SLICES || m < 1 || n < 1 || k < 1 || (rs ? m : n) % S) return 1;
+  if ((long)P * k <= SUM_ALWAYS_K) return 1;
+  DevInfo *dev = nullptr;
+  if (dev_info(&dev) != MS_OK) return 1;
+  const DevFacts facts = usable(*dev);
+  Problem p;
+  p.flow = rs ? RS : LS;
+  p.in_dtype = MS_DTYPE_BF16; p.K = k;
+  Problem chunks = p;
+  p.sum = true; p.S = P; p.M = m; p.N = n; p.out_dtype = MS_DTYPE_BF16;
+  p.ws = reinterpret_cast<void *>(uintptr_t(256));      // stands for "a workspace", as in ms_gemm_os_noalloc
+  p.ws_bytes = WS_HEADER_BYTES + (size_t)dev->cus * 256 * 384 * sizeof(float);
+  chunks.S = P * S; chunks.M = rs ? m / S : m; chunks.N = rs ? n : n / S; chunks.out_dtype = MS_DTYPE_F32;
+  const double mb = 1e-6, part_lines = rs ? 0.5 * ((m % 64 != 0) + (n % 64 != 0)) : 0.0;
+  const double operands = 2.0 * ((double)m + n) * P * k, copied = 2.0 * (rs ? m : n) * (double)P * k, chunk_bytes = 4.0 * P * (double)m * n;
+  const double cold = operands > 256e6 ? operands - 256e6 : 0.0;
+  const double sum_us = pick_variant(p, facts).cost * P * k * SUM_UNIT_US * SUM_SCALE * (1.0 + SUM_RS_PART_LINES * part_lines) + SUM_LAUNCH_US + cold * mb * SUM_COLD_US_PER_MB;
+  double chunks_us = pick_variant(chunks, facts).cost * k * SUM_UNIT_US * CHUNK_SCALE + chunk_bytes * mb * CHUNK_US_PER_MB + copied * mb * CHUNK_COPY_US_PER_MB + CHUNK_LAUNCHES_US;
+  const double host_us = CHUNK_HOST_US + P * (CHUNK_HOST_PEER_US + CHUNK_HOST_SLICE_US * (S - 1));
+  if (host_us > chunks_us) chunks_us = host_us;
+  return chunks_us < CHUNK_MARGIN * sum_us ? 0 : 1;
+}
+
 MS_API int ms_gemm_ls_sum(const void *const *A, int lda, const void *const *W, int ldw, int P, int m, int n, int k, void *C, int ldc,
                           int in_dtype, int out_dtype, void *workspace, size_t workspace_bytes, void *stream) {
   void *c1[1] = {C};

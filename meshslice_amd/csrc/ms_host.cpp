@@ -227,6 +227,17 @@ PyObject *gemm_sum(PyObject *const *args) {
   return rc == MS_OK ? THPVariable_Wrap(std::move(out)) : nullptr;
 }
 
+// prefers_sum(rs, P, S, m, n, k) -> bool
+PyObject *prefers_sum(PyObject *const *args) {
+  int v[6];
+  for (int i = 0; i < 6; i++) {
+    const long x = PyLong_AsLong(args[i]);
+    if (x < 0 || x > INT32_MAX) return nullptr;
+    v[i] = (int)x;
+  }
+  return PyBool_FromLong(ms_prefers_sum(v[0], v[1], v[2], v[3], v[4], v[5]));
+}
+
 // pack_slices(block, S, B, axis) -> [slices] or None
 PyObject *pack_slices(PyObject *const *args) {
   const at::Tensor *t = matrix(args[0]);
@@ -329,6 +340,7 @@ PyMethodDef g_methods[] = {
     MS_ENTRY("gemm_ls_cyclic", gemm_ls_cyclic, 3),
     MS_ENTRY("gemm_ls_sum", gemm_sum<true>, 3),
     MS_ENTRY("gemm_rs_sum", gemm_sum<false>, 3),
+    MS_ENTRY("prefers_sum", prefers_sum, 6),
     MS_ENTRY("pack_slices", pack_slices, 4),
     MS_ENTRY("unpack_chunks", unpack_chunks, 6),
     {"workspace_set", workspace_set, METH_VARARGS, nullptr},

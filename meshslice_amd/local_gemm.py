@@ -464,6 +464,14 @@ def gemm_rs_sum(X: torch.Tensor, W: torch.Tensor, P: int) -> torch.Tensor:
     return _sum(_lib.load().ms_gemm_rs_sum, X, W, P, k * X.stride(0) * X.element_size(), k * W.stride(0) * W.element_size(), X.shape[1], W.shape[1], k)
 
 
+def prefers_sum(flow: str, P: int, S: int, m: int, n: int, k: int) -> bool:
+    """Whether the sum over a mesh line of P devices, k contraction elements each, is expected sooner from gemm_ls_sum / gemm_rs_sum than from
+    fp32 chunks of S slices added up in memory (``ms_prefers_sum``)."""
+    rs = int(flow == "rs")
+    pays = _lib.host.prefers_sum(rs, P, S, m, n, k)
+    return bool(_lib.load().ms_prefers_sum(rs, P, S, m, n, k)) if pays is None else pays
+
+
 def _sum(entry, X, W, P, x_step, w_step, m, n, k):
     out = torch.empty((m, n), dtype=X.dtype, device=X.device)
     x0, w0 = X.data_ptr(), W.data_ptr()

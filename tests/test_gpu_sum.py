@@ -64,6 +64,25 @@ def test_global_products_have_the_same_bits_through_chunks(R, C, K, u, v, w, alg
     assert torch.equal(got, f(X, W))
 
 
+@pytest.mark.parametrize("algorithm", ["meshflow", "collective"])
+@pytest.mark.parametrize("flow,P,K,m,n,k,in_registers", [
+    ("rs", 16, 2, 256, 640, 6464, False), ("ls", 16, 4, 512, 512, 2816, False), ("rs", 5, 4, 160, 320, 6080, False),      # tiles that leave the device idle, too many devices to split over
+    ("rs", 4, 1, 1024, 4096, 16384, False), ("rs", 4, 2, 1024, 4096, 2048, True), ("ls", 16, 2, 512, 512, 640, True), ("ls", 2, 2, 512, 512, 8192, True)])
+def test_sums_are_carried_in_registers_where_that_is_the_cheaper_way(flow, P, K, m, n, k, in_registers, algorithm, monkeypatch):
+    """Either way has the other's bits; both host paths make the same choice."""
+    if algorithm == "meshflow" and K == 1:
+        K = 2
+    X, W = _operands(flow, m, n, k * P)
+    f = getattr(TP.SPMD(Mesh(create_device_mesh((1, P) if flow == "ls" else (P, 1)), ("row", "col")), algorithm), flow.upper())(K)
+    lib, S = _lib.load(), K if algorithm == "meshflow" else 1
+    got = f(X, W)
+    assert (lib.ms_query(_lib.MS_QUERY_LAST_VARIANT) in (15, 16, 17)) == in_registers
+    assert local_gemm.prefers_sum(flow, P, S, m, n, k) == bool(lib.ms_prefers_sum(int(flow == "rs"), P, S, m, n, k)) == in_registers
+    monkeypatch.setattr(local_gemm, "prefers_sum", lambda *a: not in_registers)
+    assert torch.equal(got, f(X, W))
+    assert (lib.ms_query(_lib.MS_QUERY_LAST_VARIANT) in (15, 16, 17)) != in_registers
+
+
 def test_sums_check_their_arguments():
     x, w = torch.randn(16, 64, device="cuda").bfloat16(), torch.randn(24, 64, device="cuda").bfloat16()
     for bad in (lambda: local_gemm.gemm_ls_sum(x, w, 3), lambda: local_gemm.gemm_ls_sum(x, w.t().contiguous(), 2),
@@ -73,6 +92,8 @@ def test_sums_check_their_arguments():
     with pytest.raises(_lib.MeshSliceError):
         local_gemm.gemm_ls_sum(x.float(), w.float(), 2)
     lib = _lib.load()
+    for odd in ((0, 1, 1, 512, 512, 65536), (1, 64, 2, 512, 512, 65536), (0, 4, 3, 512, 512, 65536), (1, 4, 1, 0, 512, 65536), (0, 4, 1, 512, 512, -1)):
+        assert lib.ms_prefers_sum(*odd) == 1
     assert lib.ms_gemm_ls_sum(None, 64, None, 64, 2, 16, 24, 32, None, 24, 1, 1, None, 0, ctypes.c_void_p(0)) == _lib.MS_ERR_ARG
     assert lib.ms_gemm_rs_sum(None, 64, None, 64, 65, 16, 24, 32, None, 24, 1, 1, None, 0, ctypes.c_void_p(0)) == _lib.MS_ERR_ARG
 
