@@ -213,8 +213,8 @@ int ms_gemm_rs_sum(const void *const *X, int ldx, const void *const *W, int ldw,
                    void *workspace, size_t workspace_bytes, void *stream);
 
 /* Whether the library expects the sum over a mesh line sooner from ms_gemm_ls_sum (rs: ms_gemm_rs_sum) than from ms_gemm_*_peers on S slices and
- * ms_unpack_chunks: 1 or 0, from the extents alone (P devices of k contraction elements each, an output of m x n); 1 too for
- * extents that it cannot price.  The bits are the same either way. */
+ * ms_unpack_chunks: 1 or 0, from the extents (P devices of k contraction elements each, an output of m x n); 1 too for
+ * extents that it cannot price.  Under a forced tile (ms_set_variant) the way that runs it.  The bits are the same either way. */
 int ms_prefers_sum(int rs, int P, int S, int m, int n, int k);
 
 /* ms_gemm_ls_ex / ms_gemm_rs_ex with completion counters, so that the reduce-scatter of chunk s (the psum_scatter that

@@ -458,6 +458,7 @@ Pick pick_variant(const Problem &p, const DevFacts &dev) {
   const bool rs = p.flow == RS, ls = p.flow == LS;
   const long chunks = p.flow == OS || p.sum ? 1 : p.S;
   const double total_k = p.flow == OS || p.sum ? (double)p.K * p.S : (double)p.K;
+  const int forced_splits = p.sum ? 0 : g_splits;      // (a split count is forced on output-stationary products)
   Pick best = {0, 1, 0};
   for (const TileRate &c : TILE_RATES) {
     if (p.sum && !carries_sum(c.v)) continue;
@@ -466,9 +467,9 @@ Pick pick_variant(const Problem &p, const DevFacts &dev) {
     const double rate = rs ? c.rs : ls ? c.ls : c.os;
     const long tiles = (long)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * chunks;
     for (int splits : SPLIT_CHOICES) {
-      if (g_splits != 0 && splits != g_splits) continue;
+      if (forced_splits != 0 && splits != forced_splits) continue;
       if (splits == 1 ? rate == 0.0 : c.split == 0.0) continue;
-      if (splits > 1 && (split_refused(p, dev, c.v, splits) || (g_splits == 0 && total_k / splits < SPLIT_MIN_K))) continue;
+      if (splits > 1 && (split_refused(p, dev, c.v, splits) || (forced_splits == 0 && total_k / splits < SPLIT_MIN_K))) continue;
       // rounds the launch is charged: whole ones, or with the last round partly filled (see balanced_grid) its filled
       // share plus a part of the rest; a launch of less than one round is charged the same way, down to 0.7 of a round (the
       // idle units' power lets the busy ones clock up to 1.4 times higher)
@@ -1170,6 +1171,7 @@ constexpr double CHUNK_MARGIN = 0.93;                                        // 
 
 MS_API int ms_prefers_sum(int rs, int P, int S, int m, int n, int k) {
   if (P < 2 || P > MS_MAX_SLICES || S < 1 || (long)P * S > MS_MAX_SLICES || m < 1 || n < 1 || k < 1 || (rs ? m : n) % S) return 1;
+  if (g_variant >= 1 && g_variant <= VARIANTS) return carries_sum(g_variant);      // (a forced tile is the one that runs)
   if ((long)P * k <= SUM_ALWAYS_K) return 1;
   DevInfo *dev = nullptr;
   if (dev_info(&dev) != MS_OK) return 1;

@@ -83,6 +83,25 @@ def test_sums_are_carried_in_registers_where_that_is_the_cheaper_way(flow, P, K,
     assert (lib.ms_query(_lib.MS_QUERY_LAST_VARIANT) in (15, 16, 17)) != in_registers
 
 
+@pytest.mark.parametrize("flow", ["ls", "rs"])
+@pytest.mark.parametrize("variant", range(1, 15))
+def test_a_forced_tile_runs_global_products(variant, flow):
+    """In registers on the tiles that carry the sum, else in chunks: the same bits; and a split count that is forced on output-stationary
+    products leaves the sums to the library's choice."""
+    X, W = _operands(flow, 528, 784, 2 * 200)
+    f = getattr(TP.SPMD(Mesh(create_device_mesh((1, 2) if flow == "ls" else (2, 1)), ("row", "col")), "collective"), flow.upper())(1)
+    g = local_gemm.gemm_ls_sum if flow == "ls" else local_gemm.gemm_rs_sum
+    want, lib = f(X, W), _lib.load()
+    try:
+        assert lib.ms_set_variant(variant) == 0
+        got, used = f(X, W), lib.ms_query(_lib.MS_QUERY_LAST_VARIANT)
+        assert lib.ms_set_variant(300 + (variant if variant not in (2, 4, 14) else 0)) == 0
+        assert torch.equal(g(X, W, 2), want)
+    finally:
+        lib.ms_set_variant(0)
+    assert torch.equal(got, want) and used == {2: 17, 4: 16, 14: 15}.get(variant, variant)
+
+
 def test_sums_check_their_arguments():
     x, w = torch.randn(16, 64, device="cuda").bfloat16(), torch.randn(24, 64, device="cuda").bfloat16()
     for bad in (lambda: local_gemm.gemm_ls_sum(x, w, 3), lambda: local_gemm.gemm_ls_sum(x, w.t().contiguous(), 2),
