@@ -155,21 +155,27 @@ def load():
 
 
 class _HostMissing:
-    """Stands for the native call path where it has not been built: the first use says so."""
+    """Stands for the native call path where it cannot be loaded: the first use says why."""
+
+    def __init__(self, why: str, cause: ImportError):
+        self._why, self._cause = why, cause
 
     def __getattr__(self, name):
-        if name.startswith("__"):
+        if name.startswith("_"):
             raise AttributeError(name)
-        raise MeshSliceError("meshslice_amd/_host has not been built beside libmeshslice_hip.so (run __graft_entry__.build() or "
-                             "`make -C meshslice_amd/csrc`)")
+        raise MeshSliceError(self._why) from self._cause
 
 
 def _load_host():
     import importlib
     try:
         return importlib.import_module("._host", __package__)
-    except ImportError:
-        return _HostMissing()
+    except ModuleNotFoundError as e:
+        return _HostMissing("meshslice_amd/_host has not been built beside libmeshslice_hip.so (run __graft_entry__.build() or "
+                            "`make -C meshslice_amd/csrc`)", e)
+    except ImportError as e:      # (built against another torch or another libmeshslice_hip.so, say)
+        return _HostMissing(f"meshslice_amd/_host is there and cannot be loaded: {e}; build it anew (__graft_entry__.build() or "
+                            "`make -B -C meshslice_amd/csrc`)", e)
 
 
 host = _load_host()      # (torch is loaded by then: the modules that use it import it first)

@@ -391,3 +391,20 @@ def test_asking_whether_a_matrix_can_be_read_in_place_copies_nothing(monkeypatch
     assert TP._addressable(buf[:512].view(8, 64)) and TP._addressable(buf.view(64, 64)[:, 8:24])
     for t in (buf[1:513].view(8, 64), buf.view(64, 64)[:, 1:25], buf[:8 * 60].view(8, 60), buf[:64].view(8, 8).t(), buf[:64].expand(4, 64)):
         assert not TP._addressable(t)
+
+
+# ---------------------------------------------------------------- the native call path that does not load
+@pytest.mark.parametrize("error,says", [(ModuleNotFoundError("No module named 'meshslice_amd._host'"), "has not been built"),
+                                        (ImportError("undefined symbol: _ZN2at5emptyE"), "cannot be loaded: undefined symbol: _ZN2at5emptyE")])
+def test_a_native_call_path_that_does_not_load_says_why(error, says, monkeypatch):
+    import importlib
+
+    def refused(*a):
+        raise error
+    monkeypatch.setattr(importlib, "import_module", refused)
+    host = _lib._load_host()
+    monkeypatch.undo()
+    assert not hasattr(host, "__wrapped__")
+    with pytest.raises(_lib.MeshSliceError, match=says) as got:
+        host.gemm_os
+    assert got.value.__cause__ is error
