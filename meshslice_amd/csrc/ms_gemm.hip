@@ -257,6 +257,13 @@ bool xcds_take_runs(const msk::GemmArgs &g, int grid, int bm, int bn, bool a_by_
   if (grid % 8 == 0) return true;
   const long k_part = (long)g.K * g.nkslices / g.splits;
   if (grid > 1024 || (g.splits > 1 && k_part < RUNS_MIN_SPLIT_K)) return false;
+  // (the count takes the host 0.8 to 1 us, a fifth of a small product's call: a thread keeps the last answers, by the grid alone)
+  struct Answer { int grid, tiles_m, tiles_n, nchunks, splits, bm, bn, by_chunk; bool runs; };
+  thread_local Answer answers[16] = {};
+  const int by_chunk = a_by_chunk + 2 * b_by_chunk;
+  Answer &kept = answers[(unsigned)(grid + 3 * g.tiles_m + 5 * g.tiles_n + 7 * g.nchunks + g.splits) % 16];
+  if (kept.grid == grid && kept.tiles_m == g.tiles_m && kept.tiles_n == g.tiles_n && kept.nchunks == g.nchunks && kept.splits == g.splits && kept.bm == bm &&
+      kept.bn == bn && kept.by_chunk == by_chunk) return kept.runs;
   // panel numbers of the first round's items, in the order of the kernels' walk
   short a[1024], b[1024];
   int n = 0, na = 0, nb = 0;      // panels of the parts and chunks before this one
@@ -286,7 +293,8 @@ bool xcds_take_runs(const msk::GemmArgs &g, int grid, int bm, int bn, bool a_by_
     }
     fetched[runs] = rows * bm + cols * bn;
   }
-  return (double)fetched[1] < RUNS_MIN_GAIN * (double)fetched[0];
+  kept = {grid, g.tiles_m, g.tiles_n, g.nchunks, g.splits, bm, bn, by_chunk, (double)fetched[1] < RUNS_MIN_GAIN * (double)fetched[0]};
+  return kept.runs;
 }
 constexpr double PARTIAL_ROUND_LOSS = 0.6;
 

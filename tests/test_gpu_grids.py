@@ -35,3 +35,23 @@ def test_every_tile_once(rows, cols, variant):
             assert all(torch.equal(c, want) for c in chunk)
     finally:
         lib.ms_set_variant(0)
+
+
+def test_answers_kept_for_a_grid_are_that_grids():
+    """Grids that share a place in the table of kept answers (19 tiles of 128 x 128 whichever way they lie, as chunks and as one output), in
+    turns and again: the first call's bits each time."""
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(19)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    calls = []
+    for rows, cols in ((19, 1), (1, 19), (3, 7), (7, 3), (9, 13), (13, 9), (17, 13), (13, 17)):
+        A, B = r(rows * 128 - 40, 96), r(96, cols * 128 - 24)
+        W = B.t().contiguous()
+        calls += [lambda A=A, B=B: ms.gemm_os([A], [B]), lambda A=A, W=W: ms.gemm_ls(A, [W, W], out_dtype=torch.bfloat16)[1]]
+    assert lib.ms_set_variant(14) == 0
+    try:
+        first = [f() for f in calls]
+        for f, want in list(zip(calls, first)) * 2 + list(zip(calls, first))[::-1]:
+            assert torch.equal(f(), want) and float((want.float() - first[calls.index(f) // 2 * 2].float()).abs().max()) == 0.0
+    finally:
+        lib.ms_set_variant(0)
