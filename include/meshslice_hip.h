@@ -178,7 +178,8 @@ int ms_gemm_rs_ex(const void *const *X_slices, int ldx, const void *W, int ldw, 
 
 /* ms_gemm_os_ws with B's slices where they lie in the matrix that they are cut from: B_s is the s-th block-cyclic row slice of
  * W [S * k_slice, n] with blocks of eight rows (row r of it is row (r / 8 * S + s) * 8 + r % 8 of W; ms_pack_slices with axis 0
- * and B = 8 copies the same).  k_slice is a multiple of 8; W spans less than 2 GiB.  Same bits as on the copied slices. */
+ * and B = 8 copies the same).  k_slice is a multiple of 8; W spans less than 2 GiB, and 64 * S of its rows (at most: only
+ * slices of fewer than 32 rows meet this) no more than 4 GiB.  Same bits as on the copied slices. */
 int ms_gemm_os_cyclic(const void *const *A_slices, const void *W, int S,
                       int m, int n, int k_slice, int lda, int ldw,
                       void *C, int ldc, int in_dtype, int out_dtype,

@@ -194,6 +194,12 @@ def _gathered(parts: Sequence[torch.Tensor], axis: int) -> torch.Tensor:
     return _gather(parts, axis) if whole is None else whole
 
 
+def _steps_addressable(row_bytes: int, K: int) -> bool:
+    """Whether a K step of a product whose contraction runs through K row slices in place (eight blocks of a slice's rows, 8 * K rows apart)
+    stays within the kernels' 32-bit offsets: always, but for slices of a few rows of hundreds of megabytes."""
+    return 64 * K * row_bytes <= 1 << 32
+
+
 def _uncut(peers: Sequence[torch.Tensor], K: int, B: int):
     """The gathered rows of which _gather_row_slices makes slices, where the kernels can read the slices inside them (blocks of eight rows
     of one matrix), else None.  The peers' slices one below the other are the slices of the whole, as in _gather_col_slices; the copy
@@ -233,7 +239,7 @@ def MeshFlow_OS(X, W, i, j, R, C, K, B):
                          "use algorithm='collective' for the unsliced product")
     A_slices, peers = _gather_col_slices(_row(X, i, C), K, B), _column(W, j, R)
     W_rows = _uncut(peers, K, B)
-    if W_rows is not None:
+    if W_rows is not None and _steps_addressable(W_rows.stride(0) * W_rows.element_size(), K):
         return local_gemm.gemm_os_cyclic(A_slices, W_rows)
     return local_gemm.gemm_os(A_slices, _gather_row_slices(peers, K, B))
 
@@ -660,7 +666,7 @@ class ShardedMatmul:
             try:
                 # (nothing that the kernels can read in place is gathered, cut or interleaved: an OS product's slices decide the order in which it
                 # contracts, the sums over a line are the same whatever the slices)
-                if self.body is MeshFlow_OS and K > 1 and B == 8 and _addressable(W):
+                if self.body is MeshFlow_OS and K > 1 and B == 8 and _addressable(W) and _steps_addressable(W.stride(0) * W.element_size(), K):
                     return local_gemm.gemm_os_cyclic(slice_layout.pack_slices(X, K, B, 1), W)
                 if self.dataflow == "ls" and _sums_on_chip(X, W) and local_gemm.prefers_sum("ls", C, K, X.shape[0], W.shape[0], X.shape[1] // C):
                     return local_gemm.gemm_ls_sum(X, W, C)

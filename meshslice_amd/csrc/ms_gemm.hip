@@ -972,6 +972,9 @@ MS_API int ms_gemm_os_cyclic(const void *const *A_slices, const void *W, int S, 
   const long long es = in_dtype == MS_DTYPE_BF16 ? 2 : 4;
   if (k_slice <= 0 || k_slice % 8) return fail(MS_ERR_ARG, "%s: k_slice = %d is not a number of blocks of eight rows", fn, k_slice);
   if (ldw < 0 || (long long)k_slice * S * ldw * es > 0x7FFFFFFFLL) return fail(MS_ERR_UNSUPPORTED, "%s: W spans 2 GiB or more", fn);
+  // (a K step's loads reach up to eight blocks of rows on, with 32-bit offsets also where the slice has fewer: wrapped around they would
+  // fetch some of its rows a second time, against zeros, which infinities turn into NaN)
+  if ((long long)S * 8 * ldw * es * 8 > 0x100000000LL) return fail(MS_ERR_UNSUPPORTED, "%s: eight blocks of a slice's rows span more than 4 GiB of W", fn);
   const void *b[MS_MAX_SLICES];
   for (int s = 0; s < S; s++) b[s] = W ? static_cast<const char *>(W) + (long long)s * 8 * ldw * es : nullptr;
   void *c1[1] = {C};

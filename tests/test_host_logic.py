@@ -408,3 +408,27 @@ def test_a_native_call_path_that_does_not_load_says_why(error, says, monkeypatch
     with pytest.raises(_lib.MeshSliceError, match=says) as got:
         host.gemm_os
     assert got.value.__cause__ is error
+
+
+# ---------------------------------------------------------------- row slices read in place: 32-bit offsets
+@pytest.mark.parametrize("S,k_slice,ldw,es", [(8, 8, 1 << 23, 2), (64, 8, 1 << 20, 2), (2, 16, (1 << 25) - 8, 2), (4, 8, (1 << 24) - 4, 4)])
+def test_a_k_step_of_slices_in_place_stays_within_32_bits(S, k_slice, ldw, es):
+    """W spans less than 2 GiB, eight blocks of a slice's rows more than 4: the offsets of the rows beyond the slice wrap round to rows of it."""
+    import ctypes
+    row = ldw * es
+    assert S * k_slice * row < 1 << 31
+    offsets = [r // 8 * (8 * S * row) + r % 8 * row for r in range(128 // es)]               # as the kernels' loads form them
+    extent = (k_slice - 1) // 8 * (8 * S * row) + (k_slice - 1) % 8 * row + row              # what the resource covers
+    assert any(o % (1 << 32) < extent for o in offsets[k_slice:]) and not TP._steps_addressable(row, S)
+    buf = np.zeros(64, np.float32)
+    table, _keep = _lib.ptr_array([buf.ctypes.data] * S)
+    rc = _lib.load().ms_gemm_os_cyclic(table, ctypes.c_void_p(buf.ctypes.data), S, 8, ldw, k_slice, k_slice, ldw, ctypes.c_void_p(buf.ctypes.data), ldw,
+                                       int(es == 2), int(es == 2), None, 0, None)
+    assert rc == _lib.MS_ERR_UNSUPPORTED
+
+
+def test_slices_of_32_rows_and_more_always_fit():
+    for S in range(2, 65):
+        for es in (2, 4):
+            ldw = ((1 << 31) - 1) // (S * 32 * es)          # the widest W of S slices of 32 rows
+            assert TP._steps_addressable(ldw * es, S)
