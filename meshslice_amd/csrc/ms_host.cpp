@@ -4,8 +4,10 @@
 // Every function here takes the ordinary case only (plain dense GPU tensors on the current device, lists or tuples of equal
 // slices, no tracing, no capture where a workspace would have to come from the graph's pool) and returns None for everything
 // else, invalid arguments among it: the caller then takes the Python path, which says what is wrong or handles the rest.
-// Nothing is kept between calls but the addresses of the workspaces that local_gemm.workspace() owns and announces
-// (workspace_set / workspace_drop); the interpreter lock is held from looking one up until its launch has been queued.
+// Nothing is kept between calls but the workspaces that local_gemm.workspace() announces (workspace_set / workspace_drop).  The interpreter
+// lock is released while an output is allocated and a product launched: either may wait for the device (a full queue, an allocator that has
+// to free), and another Python thread may be the one that raises the flag that the device waits for.  So everything that is needed of the
+// Python objects is read before, and a call holds the storage of its workspace until its launch has been queued.
 #include <Python.h>
 
 #include <ATen/Functions.h>
@@ -25,12 +27,13 @@ namespace {
 struct Workspace {
   int device = -1;
   void *stream = nullptr;
+  c10::Storage hold;
   void *ptr = nullptr;
   size_t bytes = 0;
   unsigned long long used = 0;      // when the last call took it
 };
 constexpr int MAX_WORKSPACES = 256;
-Workspace g_ws[MAX_WORKSPACES];
+Workspace *const g_ws = new Workspace[MAX_WORKSPACES];      // (never destroyed: the allocator may be gone by then)
 int g_ws_count = 0;
 unsigned long long g_clock = 0;
 
@@ -40,9 +43,27 @@ Workspace *find_workspace(int device, void *stream) {
   return nullptr;
 }
 
+// the interpreter lock is released for the life of one of these
+struct Unlocked {
+  PyThreadState *state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+  Unlocked() = default;
+  Unlocked(const Unlocked &) = delete;
+};
+
 int code_of(const at::Tensor &t) {
   return t.scalar_type() == at::kBFloat16 ? MS_DTYPE_BF16 : t.scalar_type() == at::kFloat ? MS_DTYPE_F32 : -1;
 }
+
+// what a call needs of a matrix once the lock is released
+struct Mat {
+  char *ptr;
+  int64_t rows, cols;
+  int ld, code;
+  at::TensorOptions options;
+  explicit Mat(const at::Tensor &t)
+      : ptr(static_cast<char *>(t.data_ptr())), rows(t.size(0)), cols(t.size(1)), ld((int)t.stride(0)), code(code_of(t)), options(t.options().requires_grad(false)) {}
+};
 
 // a row-major matrix in plain GPU memory, or null
 const at::Tensor *matrix(PyObject *o) {
@@ -91,17 +112,18 @@ Place place_of(const at::Tensor &t) {
   p.ok = true;
   return p;
 }
-// the workspace of that place, or null: none yet, or a capture is under way (its workspaces come from the graph's pool)
-Workspace *workspace_of(const Place &p) {
+// the workspace of that place, or one without storage: none yet, or a capture is under way (its workspaces come from the graph's pool)
+Workspace workspace_of(const Place &p) {
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(p.stream, &capturing) != hipSuccess) {
     (void)hipGetLastError();      // (not for the next launch to find)
-    return nullptr;
+    return Workspace();
   }
-  if (capturing != hipStreamCaptureStatusNone) return nullptr;
+  if (capturing != hipStreamCaptureStatusNone) return Workspace();
   Workspace *w = find_workspace(p.device, p.stream);
-  if (w) w->used = ++g_clock;
-  return w;
+  if (!w) return Workspace();
+  w->used = ++g_clock;
+  return *w;
 }
 
 // the dtype named by `o` (None: `otherwise`), or -1 for one that the kernels do not write
@@ -134,19 +156,27 @@ PyObject *gemm_os(PyObject *const *args) {
   if (!b0 || na != nb || a0->size(1) != b0->size(0) || a0->scalar_type() != b0->scalar_type() || a0->device() != b0->device()) return nullptr;
   const int in = code_of(*a0), outc = wanted_dtype(args[2], in);
   if (outc < 0) return nullptr;
-  const int64_t m = a0->size(0), n = b0->size(1);
-  const at::Tensor *res = nullptr;
+  const Mat A(*a0), B(*b0);
+  const int64_t m = A.rows, n = B.cols;
+  const void *res = nullptr;
+  int ldr = 0;
   if (args[4] != Py_None) {
-    res = matrix(args[4]);
-    if (!res || res->size(0) != m || res->size(1) != n || code_of(*res) != outc || res->device() != a0->device()) return nullptr;
+    const at::Tensor *r = matrix(args[4]);
+    if (!r || r->size(0) != m || r->size(1) != n || code_of(*r) != outc || r->device() != a0->device()) return nullptr;
+    res = r->data_ptr();
+    ldr = (int)r->stride(0);
   }
   const Place p = place_of(*a0);
-  const Workspace *ws = p.ok ? workspace_of(p) : nullptr;
-  if (!ws) return nullptr;
-  at::Tensor out = at::empty({m, n}, a0->options().dtype(type_of(outc)).requires_grad(false));
-  const int rc = ms_gemm_os_ws(a, b, na, (int)m, (int)n, (int)a0->size(1), (int)a0->stride(0), (int)b0->stride(0), out.data_ptr(), (int)n, in, outc,
-                               args[3] == Py_True ? MS_ACT_GELU : MS_ACT_NONE, res ? res->data_ptr() : nullptr, res ? (int)res->stride(0) : 0,
-                               nullptr, nullptr, ws->ptr, ws->bytes, p.stream);
+  const Workspace ws = p.ok ? workspace_of(p) : Workspace();
+  if (!ws.ptr) return nullptr;
+  at::Tensor out;
+  int rc;
+  {
+    Unlocked u;
+    out = at::empty({m, n}, A.options.dtype(type_of(outc)));
+    rc = ms_gemm_os_ws(a, b, na, (int)m, (int)n, (int)A.cols, A.ld, B.ld, out.data_ptr(), (int)n, in, outc, args[3] == Py_True ? MS_ACT_GELU : MS_ACT_NONE,
+                       res, ldr, nullptr, nullptr, ws.ptr, ws.bytes, p.stream);
+  }
   return rc == MS_OK ? THPVariable_Wrap(std::move(out)) : nullptr;
 }
 
@@ -157,13 +187,16 @@ PyObject *gemm_os_cyclic(PyObject *const *args) {
   const at::Tensor *a0 = matrices(args[0], const_cast<void **>(a), &S), *w = a0 ? matrix(args[1]) : nullptr;
   if (!w || a0->size(1) * S != w->size(0) || a0->scalar_type() != w->scalar_type() || a0->device() != w->device()) return nullptr;
   const Place p = place_of(*a0);
-  const Workspace *ws = p.ok ? workspace_of(p) : nullptr;
-  if (!ws) return nullptr;
-  const int64_t m = a0->size(0), n = w->size(1);
-  const int code = code_of(*w);
-  at::Tensor out = at::empty({m, n}, w->options().requires_grad(false));
-  const int rc = ms_gemm_os_cyclic(a, w->data_ptr(), S, (int)m, (int)n, (int)a0->size(1), (int)a0->stride(0), (int)w->stride(0), out.data_ptr(), (int)n,
-                                   code, code, ws->ptr, ws->bytes, p.stream);
+  const Workspace ws = p.ok ? workspace_of(p) : Workspace();
+  if (!ws.ptr) return nullptr;
+  const Mat A(*a0), W(*w);
+  at::Tensor out;
+  int rc;
+  {
+    Unlocked u;
+    out = at::empty({A.rows, W.cols}, W.options);
+    rc = ms_gemm_os_cyclic(a, W.ptr, S, (int)A.rows, (int)W.cols, (int)A.cols, A.ld, W.ld, out.data_ptr(), (int)W.cols, W.code, W.code, ws.ptr, ws.bytes, p.stream);
+  }
   return rc == MS_OK ? THPVariable_Wrap(std::move(out)) : nullptr;
 }
 
@@ -179,11 +212,17 @@ PyObject *gemm_chunks(PyObject *const *args) {
   if (outc < 0) return nullptr;
   const Place p = place_of(*own);
   if (!p.ok) return nullptr;
-  const int64_t m = LS ? own->size(0) : c0->size(1), n = LS ? c0->size(0) : own->size(1), k = own->size(LS ? 1 : 0);
-  at::Tensor buf = at::empty({S, m, n}, own->options().dtype(type_of(outc)).requires_grad(false));
-  chunk_pointers(buf, y);
-  const int rc = LS ? ms_gemm_ls_ex(own->data_ptr(), (int)own->stride(0), cut, (int)c0->stride(0), S, (int)m, (int)n, (int)k, y, (int)n, in, outc, p.stream)
-                    : ms_gemm_rs_ex(cut, (int)c0->stride(0), own->data_ptr(), (int)own->stride(0), S, (int)m, (int)n, (int)k, y, (int)n, in, outc, p.stream);
+  const Mat O(*own), C(*c0);
+  const int64_t m = LS ? O.rows : C.cols, n = LS ? C.rows : O.cols, k = LS ? O.cols : O.rows;
+  at::Tensor buf;
+  int rc;
+  {
+    Unlocked u;
+    buf = at::empty({S, m, n}, O.options.dtype(type_of(outc)));
+    chunk_pointers(buf, y);
+    rc = LS ? ms_gemm_ls_ex(O.ptr, O.ld, cut, C.ld, S, (int)m, (int)n, (int)k, y, (int)n, in, outc, p.stream)
+            : ms_gemm_rs_ex(cut, C.ld, O.ptr, O.ld, S, (int)m, (int)n, (int)k, y, (int)n, in, outc, p.stream);
+  }
   return rc == MS_OK ? chunk_list(buf) : nullptr;
 }
 
@@ -195,11 +234,16 @@ PyObject *gemm_ls_cyclic(PyObject *const *args) {
   if (!w || S < 1 || S > MS_MAX_SLICES || w->size(0) % S || a->size(1) != w->size(1) || a->scalar_type() != w->scalar_type() || a->device() != w->device()) return nullptr;
   const Place p = place_of(*a);
   if (!p.ok) return nullptr;
-  const int64_t m = a->size(0), n = w->size(0) / S;
-  at::Tensor buf = at::empty({S, m, n}, a->options().dtype(type_of(MS_DTYPE_F32)).requires_grad(false));
-  chunk_pointers(buf, y);
-  const int rc = ms_gemm_ls_cyclic(a->data_ptr(), (int)a->stride(0), w->data_ptr(), (int)w->stride(0), (int)S, (int)m, (int)n, (int)a->size(1), y, (int)n,
-                                   code_of(*a), MS_DTYPE_F32, p.stream);
+  const Mat A(*a), W(*w);
+  const int64_t n = W.rows / S;
+  at::Tensor buf;
+  int rc;
+  {
+    Unlocked u;
+    buf = at::empty({S, A.rows, n}, A.options.dtype(type_of(MS_DTYPE_F32)));
+    chunk_pointers(buf, y);
+    rc = ms_gemm_ls_cyclic(A.ptr, A.ld, W.ptr, W.ld, (int)S, (int)A.rows, (int)n, (int)A.cols, y, (int)n, A.code, MS_DTYPE_F32, p.stream);
+  }
   return rc == MS_OK ? chunk_list(buf) : nullptr;
 }
 
@@ -212,18 +256,22 @@ PyObject *gemm_sum(PyObject *const *args) {
   if (!w || P < 1 || P > MS_MAX_SLICES || x->size(C) != w->size(C) || x->size(C) % P || x->scalar_type() != w->scalar_type() || x->device() != w->device())
     return nullptr;
   const Place p = place_of(*x);
-  const Workspace *ws = p.ok ? workspace_of(p) : nullptr;
-  if (!ws) return nullptr;
+  const Workspace ws = p.ok ? workspace_of(p) : Workspace();
+  if (!ws.ptr) return nullptr;
+  const Mat X(*x), W(*w);
   const int64_t k = x->size(C) / P, m = x->size(1 - C), n = w->size(1 - C), es = x->element_size();
   const void *xs[MS_MAX_SLICES], *wsh[MS_MAX_SLICES];
   for (long i = 0; i < P; i++) {
-    xs[i] = static_cast<const char *>(x->data_ptr()) + i * k * es * (LS ? 1 : x->stride(0));
-    wsh[i] = static_cast<const char *>(w->data_ptr()) + i * k * es * (LS ? 1 : w->stride(0));
+    xs[i] = X.ptr + i * k * es * (LS ? 1 : X.ld);
+    wsh[i] = W.ptr + i * k * es * (LS ? 1 : W.ld);
   }
-  at::Tensor out = at::empty({m, n}, x->options().requires_grad(false));
-  const int code = code_of(*x);
-  const int rc = (LS ? ms_gemm_ls_sum : ms_gemm_rs_sum)(xs, (int)x->stride(0), wsh, (int)w->stride(0), (int)P, (int)m, (int)n, (int)k, out.data_ptr(), (int)n,
-                                                        code, code, ws->ptr, ws->bytes, p.stream);
+  at::Tensor out;
+  int rc;
+  {
+    Unlocked u;
+    out = at::empty({m, n}, X.options);
+    rc = (LS ? ms_gemm_ls_sum : ms_gemm_rs_sum)(xs, X.ld, wsh, W.ld, (int)P, (int)m, (int)n, (int)k, out.data_ptr(), (int)n, X.code, X.code, ws.ptr, ws.bytes, p.stream);
+  }
   return rc == MS_OK ? THPVariable_Wrap(std::move(out)) : nullptr;
 }
 
@@ -247,10 +295,16 @@ PyObject *pack_slices(PyObject *const *args) {
   if (r < 1 || c < 1 || cut % (S * B)) return nullptr;
   const Place p = place_of(*t);
   if (!p.ok) return nullptr;
-  at::Tensor buf = at::empty({S, axis == 1 ? r : r / S, axis == 1 ? c / S : c}, t->options().requires_grad(false));
+  const Mat T(*t);
   void *d[MS_MAX_SLICES];
-  chunk_pointers(buf, d);
-  const int rc = ms_pack_slices(t->data_ptr(), (int)t->stride(0), (int)r, (int)c, (int)axis, (int)S, (int)B, d, (int)buf.size(2), code_of(*t), p.stream);
+  at::Tensor buf;
+  int rc;
+  {
+    Unlocked u;
+    buf = at::empty({S, axis == 1 ? r : r / S, axis == 1 ? c / S : c}, T.options);
+    chunk_pointers(buf, d);
+    rc = ms_pack_slices(T.ptr, T.ld, (int)r, (int)c, (int)axis, (int)S, (int)B, d, (int)buf.size(2), T.code, p.stream);
+  }
   return rc == MS_OK ? chunk_list(buf) : nullptr;
 }
 
@@ -279,9 +333,15 @@ PyObject *unpack_chunks(PyObject *const *args) {
   if (rows > INT32_MAX || cols > INT32_MAX || rows < 1 || cols < 1) return nullptr;
   const Place p = place_of(*c0);
   if (!p.ok) return nullptr;
-  at::Tensor out = at::empty({rows, cols}, c0->options().dtype(type_of(outc)).requires_grad(false));
-  const int rc = ms_unpack_chunks(src, (int)P, S, (int)c0->stride(0), axis == 1 ? 0 : (int)(window * keep), axis == 1 ? (int)(window * keep) : 0,
-                                  (int)rows, (int)cols, (int)axis, (int)B, out.data_ptr(), (int)cols, in, outc, p.stream);
+  const Mat C(*c0);
+  at::Tensor out;
+  int rc;
+  {
+    Unlocked u;
+    out = at::empty({rows, cols}, C.options.dtype(type_of(outc)));
+    rc = ms_unpack_chunks(src, (int)P, S, C.ld, axis == 1 ? 0 : (int)(window * keep), axis == 1 ? (int)(window * keep) : 0, (int)rows, (int)cols, (int)axis, (int)B,
+                          out.data_ptr(), (int)cols, in, outc, p.stream);
+  }
   return rc == MS_OK ? THPVariable_Wrap(std::move(out)) : nullptr;
 }
 
@@ -305,21 +365,30 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
   Py_RETURN_NONE;
 }
 
-// workspace_set(device, stream, ptr, bytes); workspace_drop(device, stream); workspace_touch(device, stream, touch = True) -> when it was used last
+// workspace_set(device, stream, tensor); workspace_drop(device, stream); workspace_touch(device, stream, touch = True) -> when it was used last
 PyObject *workspace_set(PyObject *, PyObject *args) {
   int device;
-  unsigned long long stream, ptr, bytes;
-  if (!PyArg_ParseTuple(args, "iKKK", &device, &stream, &ptr, &bytes)) return nullptr;
+  unsigned long long stream;
+  PyObject *o;
+  if (!PyArg_ParseTuple(args, "iKO", &device, &stream, &o)) return nullptr;
+  if (!THPVariable_Check(o)) {
+    PyErr_SetString(PyExc_TypeError, "a workspace is a tensor");
+    return nullptr;
+  }
+  const at::Tensor &t = THPVariable_Unpack(o);
   Workspace *w = find_workspace(device, reinterpret_cast<void *>(stream));
   if (!w && g_ws_count < MAX_WORKSPACES) w = &g_ws[g_ws_count++];
-  if (w) *w = Workspace{device, reinterpret_cast<void *>(stream), reinterpret_cast<void *>(ptr), (size_t)bytes, ++g_clock};
+  if (w) *w = Workspace{device, reinterpret_cast<void *>(stream), t.storage(), t.data_ptr(), (size_t)t.nbytes(), ++g_clock};
   Py_RETURN_NONE;
 }
 PyObject *workspace_drop(PyObject *, PyObject *args) {
   int device;
   unsigned long long stream;
   if (!PyArg_ParseTuple(args, "iK", &device, &stream)) return nullptr;
-  if (Workspace *w = find_workspace(device, reinterpret_cast<void *>(stream))) *w = g_ws[--g_ws_count];
+  if (Workspace *w = find_workspace(device, reinterpret_cast<void *>(stream))) {
+    *w = g_ws[--g_ws_count];
+    g_ws[g_ws_count] = Workspace();
+  }
   Py_RETURN_NONE;
 }
 PyObject *workspace_touch(PyObject *, PyObject *args) {

@@ -61,7 +61,7 @@ def _on(device: torch.device):
     return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
-_workspaces = {}            # (device index, stream handle) -> uint8 tensor; the native call path knows their addresses and when each was used last
+_workspaces = {}            # (device index, stream handle) -> uint8 tensor; the native call path holds them too and knows when each was used last
 _workspaces_lock = threading.Lock()
 _WORKSPACE_CACHE_MAX = 8      # streams per device that keep a workspace of their own (about 100 MB each)
 
@@ -109,7 +109,7 @@ def workspace(device, stream=None) -> torch.Tensor:
         for k in drop:      # (the native call path must not hand one out that is about to go)
             _lib.host.workspace_drop(*k)
         evicted = [_workspaces.pop(k) for k in drop]
-        _lib.host.workspace_set(*key, have.data_ptr(), have.numel())
+        _lib.host.workspace_set(*key, have)
     if evicted:
         torch.cuda.synchronize(idx)     # their streams may still be running products that use them
         del evicted

@@ -1,11 +1,12 @@
 """The native call path (csrc/ms_host.cpp) against the Python path that takes what it declines: same results, same refusals."""
 import threading
+import time
 
 import pytest
 import torch
 
 import meshslice_amd as ms
-from meshslice_amd import _lib, local_gemm
+from meshslice_amd import TensorParallel as TP, _lib, local_gemm
 from meshslice_amd.slice_layout import pack_slices, unpack_chunks
 
 pytestmark = pytest.mark.gpu
@@ -147,3 +148,65 @@ def test_threads_on_streams_of_their_own():
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert not bad
+
+
+@pytest.mark.parametrize("name", ["gemm_os", "gemm_ls", "pack_slices", "gemm_ls_sum"])
+def test_a_call_that_waits_for_a_full_queue_does_not_stop_other_threads(name):
+    """One thread queues calls behind a product that waits for its slice until the queue takes no more; the flag comes from another thread.
+    The wait is bounded: a thread that could not run raises its flag too late, and the product says so."""
+    dev, cur = torch.device("cuda", torch.cuda.current_device()), torch.cuda.current_stream()
+    other = TP._gather_stream(dev, cur)
+    if other is None:
+        pytest.skip("no stream runs beside a waiting product")
+    a, b = torch.randn(8, 512, device="cuda").bfloat16(), torch.randn(512, 8, device="cuda").bfloat16()
+    call = {"gemm_os": lambda: ms.gemm_os([a], [b]), "gemm_ls": lambda: ms.gemm_ls(a, [a]), "pack_slices": lambda: pack_slices(a, 2, 8, 1),
+            "gemm_ls_sum": lambda: local_gemm.gemm_ls_sum(a, a, 2)}[name]
+    call()
+    ready = torch.zeros(2, dtype=torch.int32, device="cuda")
+    queued = []
+
+    def fill():
+        with torch.cuda.stream(cur):
+            for i in range(40000):
+                call()
+                queued.append(i)
+    torch.cuda.synchronize()
+    local_gemm.gemm_os_gated([a], [b], ready, timeout_ms=4000)
+    t = threading.Thread(target=fill)
+    t.start()
+    time.sleep(1.0)
+    with torch.cuda.stream(other):
+        local_gemm.signal_set(ready, 0)
+    blocked = len(queued)
+    t.join()
+    torch.cuda.synchronize()
+    assert not local_gemm.gate_timed_out(ready), f"{blocked} calls were queued"
+
+
+def test_a_workspace_taken_away_during_a_call_lives_until_its_launch():
+    """Evicted from the table while another thread's calls use it: no result changes and the counters it comes back with are zero."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    A, B = [torch.randn(256, 4096, generator=g, device="cuda").bfloat16()], [torch.randn(4096, 256, generator=g, device="cuda").bfloat16()]
+    want = ms.gemm_os(A, B)
+    assert _lib.load().ms_query(_lib.MS_QUERY_LAST_SPLITS) > 1
+    stream, bad, stop = torch.cuda.Stream(), [], threading.Event()
+    torch.cuda.synchronize()
+
+    def work():
+        with torch.cuda.stream(stream):
+            for _ in range(400):
+                y = ms.gemm_os(A, B)
+                if not torch.equal(y, want):
+                    bad.append(1)
+        stop.set()
+    t = threading.Thread(target=work)
+    t.start()
+    while not stop.is_set():
+        for _ in range(12):      # (more streams than keep a workspace)
+            with torch.cuda.stream(torch.cuda.Stream()):
+                ms.gemm_os([A[0][:8]], B)
+        time.sleep(0.001)
+    t.join()
+    torch.cuda.synchronize()
+    assert not bad and len([k for k in local_gemm._workspaces if k[0] == torch.cuda.current_device()]) <= local_gemm._WORKSPACE_CACHE_MAX
+    assert torch.equal(ms.gemm_os(A, B), want)
