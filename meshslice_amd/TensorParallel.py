@@ -177,9 +177,18 @@ def _gather_row_slices(peers: Sequence[torch.Tensor], K: int, B: int) -> List[to
     return [buf[k] for k in range(K)]
 
 
-def _addressable(t: torch.Tensor) -> bool:
-    """Whether the kernels can read a matrix as it stands."""
-    return _aligned(t) and t.stride(0) >= t.shape[1] and t.shape[0] * t.stride(0) * t.element_size() < 1 << 31
+def _steps_addressable(row_bytes: int, K: int) -> bool:
+    """Whether a K step of a product whose contraction runs through K row slices in place (eight blocks of a slice's rows, 8 * K rows apart)
+    stays within the kernels' 32-bit offsets: always, but for slices of a few rows of hundreds of megabytes."""
+    return 64 * K * row_bytes <= 1 << 32
+
+
+def _addressable(t: torch.Tensor, K: int = 0) -> bool:
+    """Whether the kernels can read a matrix as it stands, with K row slices in place as the slices of a contraction."""
+    rows, cols = t.shape
+    ld, step = t.stride()
+    row = ld * t.element_size()
+    return step == 1 and t.data_ptr() % 16 == 0 and row % 16 == 0 and ld >= cols and rows * row < 1 << 31 and _steps_addressable(row, K)
 
 
 def _readable(parts: Sequence[torch.Tensor], axis: int):
@@ -192,12 +201,6 @@ def _gathered(parts: Sequence[torch.Tensor], axis: int) -> torch.Tensor:
     """_gather's matrix; shards that lie side by side in one matrix are that already and are not copied."""
     whole = _readable(parts, axis)
     return _gather(parts, axis) if whole is None else whole
-
-
-def _steps_addressable(row_bytes: int, K: int) -> bool:
-    """Whether a K step of a product whose contraction runs through K row slices in place (eight blocks of a slice's rows, 8 * K rows apart)
-    stays within the kernels' 32-bit offsets: always, but for slices of a few rows of hundreds of megabytes."""
-    return 64 * K * row_bytes <= 1 << 32
 
 
 def _uncut(peers: Sequence[torch.Tensor], K: int, B: int):
@@ -239,7 +242,7 @@ def MeshFlow_OS(X, W, i, j, R, C, K, B):
                          "use algorithm='collective' for the unsliced product")
     A_slices, peers = _gather_col_slices(_row(X, i, C), K, B), _column(W, j, R)
     W_rows = _uncut(peers, K, B)
-    if W_rows is not None and _steps_addressable(W_rows.stride(0) * W_rows.element_size(), K):
+    if W_rows is not None and _addressable(W_rows, K):
         return local_gemm.gemm_os_cyclic(A_slices, W_rows)
     return local_gemm.gemm_os(A_slices, _gather_row_slices(peers, K, B))
 
@@ -596,7 +599,10 @@ def _sums_on_chip(X, W) -> bool:
     in memory: bf16 operands that the kernel can address in place.  That writes a tenth of the bytes: LS 2048 x 3072 x 12288 of four devices
     172 -> 128 us, RS 3072 x 12288 x 2048 of two 251 -> 131, small ones a quarter of the launches (512 x 256 x 1024 on 4x2 97 -> 23 us).
     Where the contraction is long it can be the slower way: local_gemm.prefers_sum prices both."""
-    return X.dtype == torch.bfloat16 and all(t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0 and t.stride(0) >= t.shape[1] for t in (X, W))
+    if X.dtype != torch.bfloat16:
+        return False
+    x, w = X.stride(0), W.stride(0)
+    return (X.data_ptr() | W.data_ptr()) % 16 == 0 and (x | w) % 8 == 0 and x >= X.shape[1] and w >= W.shape[1]
 
 
 # (the bodies launched ahead of their gathers keep a product per device where that produces chunks; the ring bodies' slices
@@ -666,12 +672,16 @@ class ShardedMatmul:
             try:
                 # (nothing that the kernels can read in place is gathered, cut or interleaved: an OS product's slices decide the order in which it
                 # contracts, the sums over a line are the same whatever the slices)
-                if self.body is MeshFlow_OS and K > 1 and B == 8 and _addressable(W) and _steps_addressable(W.stride(0) * W.element_size(), K):
+                if self.body is MeshFlow_OS and K > 1 and B == 8 and _addressable(W, K):
                     return local_gemm.gemm_os_cyclic(slice_layout.pack_slices(X, K, B, 1), W)
-                if self.dataflow == "ls" and _sums_on_chip(X, W) and local_gemm.prefers_sum("ls", C, K, X.shape[0], W.shape[0], X.shape[1] // C):
-                    return local_gemm.gemm_ls_sum(X, W, C)
-                if self.dataflow == "rs" and _sums_on_chip(X, W) and local_gemm.prefers_sum("rs", R, K, X.shape[1], W.shape[1], X.shape[0] // R):
-                    return local_gemm.gemm_rs_sum(X, W, R)
+                if self.dataflow == "ls" and _sums_on_chip(X, W):
+                    m, k = X.shape
+                    if local_gemm.prefers_sum("ls", C, K, m, W.shape[0], k // C):
+                        return local_gemm.gemm_ls_sum(X, W, C)
+                elif self.dataflow == "rs" and _sums_on_chip(X, W):
+                    k, m = X.shape
+                    if local_gemm.prefers_sum("rs", R, K, m, W.shape[1], k // R):
+                        return local_gemm.gemm_rs_sum(X, W, R)
                 return self._whole_mesh(X, W, K, B)
             except torch.OutOfMemoryError:
                 pass       # what all mesh lines need at once (slices of all of X, gathered operands, chunks) does not fit beside the caller's tensors: one line's may

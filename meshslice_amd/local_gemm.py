@@ -467,9 +467,8 @@ def gemm_rs_sum(X: torch.Tensor, W: torch.Tensor, P: int) -> torch.Tensor:
 def prefers_sum(flow: str, P: int, S: int, m: int, n: int, k: int) -> bool:
     """Whether the sum over a mesh line of P devices, k contraction elements each, is expected sooner from gemm_ls_sum / gemm_rs_sum than from
     fp32 chunks of S slices added up in memory (``ms_prefers_sum``)."""
-    rs = int(flow == "rs")
-    pays = _lib.host.prefers_sum(rs, P, S, m, n, k)
-    return bool(_lib.load().ms_prefers_sum(rs, P, S, m, n, k)) if pays is None else pays
+    pays = _lib.host.prefers_sum(flow == "rs", P, S, m, n, k)
+    return bool(_lib.load().ms_prefers_sum(flow == "rs", P, S, m, n, k)) if pays is None else pays
 
 
 def _sum(entry, X, W, P, x_step, w_step, m, n, k):
