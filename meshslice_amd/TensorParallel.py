@@ -93,6 +93,10 @@ def _column(grid, j, R):
     return _Line(grid.G.narrow(1, j * grid.w, grid.w), R, 0) if isinstance(grid, _Grid) else [grid[i][j] for i in range(R)]
 
 
+def _shard(grid, i, j):
+    return grid.G.narrow(0, i * grid.h, grid.h).narrow(1, j * grid.w, grid.w) if isinstance(grid, _Grid) else grid[i][j]
+
+
 def _need(v: int, d: int, what: str) -> None:
     if d <= 0 or v % d:
         raise ValueError(f"{what} = {v} is not a multiple of {d}")
@@ -226,13 +230,13 @@ def Collective_OS(X, W, i, j, R, C, K, B):
 def Collective_LS(X, W, i, j, R, C, K, B):
     """reference :24-27: gather W over row; partial product X_ij @ Wj^T (input of psum_scatter)."""
     Wj = _gathered(_column(W, j, R), 0)
-    return local_gemm.gemm_ls(_own(X[i][j]), [Wj])
+    return local_gemm.gemm_ls(_own(_shard(X, i, j)), [Wj])
 
 
 def Collective_RS(X, W, i, j, R, C, K, B):
     """reference :29-32: gather X over col; partial product Xi^T @ W_ij (input of psum_scatter)."""
     Xi = _gathered(_row(X, i, C), 1)
-    return local_gemm.gemm_rs([Xi], _own(W[i][j]))
+    return local_gemm.gemm_rs([Xi], _own(_shard(W, i, j)))
 
 
 def MeshFlow_OS(X, W, i, j, R, C, K, B):
@@ -381,20 +385,20 @@ def MeshFlow_LS_overlap(X, W, i, j, R, C, K, B):
     """MeshFlow_LS with the one launch ahead of the gathers of W's row slices (:176-189; ``gemm_ls_gated``): chunk k is
     multiplied as soon as slice k has arrived.  Same chunks as MeshFlow_LS, bit for bit."""
     bufW, fillW = _row_slice_filler(_column(W, j, R), K, B)
-    own = _own(X[i][j])
+    own = _own(_shard(X, i, j))
     return _launch_ahead_of_gathers(K, bufW.device, lambda ready: local_gemm.gemm_ls_gated(own, [bufW[k] for k in range(K)], ready), (fillW,))
 
 
 def MeshFlow_RS_overlap(X, W, i, j, R, C, K, B):
     """MeshFlow_RS with the one launch ahead of the gathers of X's column slices (:198-212; ``gemm_rs_gated``)."""
     bufX, fillX = _col_slice_filler(_row(X, i, C), K, B)
-    own = _own(W[i][j])
+    own = _own(_shard(W, i, j))
     return _launch_ahead_of_gathers(K, bufX.device, lambda ready: local_gemm.gemm_rs_gated([bufX[k] for k in range(K)], own, ready), (fillX,))
 
 
 def MeshFlow_LS(X, W, i, j, R, C, K, B):
     """reference :174-193: K gathered row slices of W; K fp32 partial chunks X_ij @ W_k^T."""
-    own, peers = _own(X[i][j]), _column(W, j, R)
+    own, peers = _own(_shard(X, i, j)), _column(W, j, R)
     W_rows = _uncut(peers, K, B)
     if W_rows is not None:
         return local_gemm.gemm_ls_cyclic(own, W_rows, K)
@@ -404,7 +408,7 @@ def MeshFlow_LS(X, W, i, j, R, C, K, B):
 def MeshFlow_RS(X, W, i, j, R, C, K, B):
     """reference :195-214: K gathered column slices of X; K fp32 partial chunks X_k^T @ W_ij."""
     X_slices = _gather_col_slices(_row(X, i, C), K, B)
-    return local_gemm.gemm_rs(X_slices, _own(W[i][j]))
+    return local_gemm.gemm_rs(X_slices, _own(_shard(W, i, j)))
 
 
 # ------------------------------------------------------------------------------------------------
@@ -439,38 +443,52 @@ def _usable(views: Sequence[torch.Tensor]) -> List[torch.Tensor]:
     return [v.contiguous() for v in views]
 
 
+def _halves(parts, axis: int) -> Sequence[torch.Tensor]:
+    """The half-blocks of a mesh line's shards, cut across ``axis``: half ``hi`` of block ``b`` is number ``2 * b + hi``.  (One cut of the view
+    that covers the line: a view per access to its shards took one device of 2 x 4 some 20 us of the host.)"""
+    width = parts.step if isinstance(parts, _Line) else parts[0].shape[axis]
+    _need(width, 2, "sliced extent of a shard")
+    return _cut(parts.panel, width // 2, axis) if isinstance(parts, _Line) else [v for p in parts for v in _cut(p, width // 2, axis)]
+
+
+def _cut(t: torch.Tensor, h: int, axis: int) -> Sequence[torch.Tensor]:
+    if h < 1:
+        raise ValueError(f"matrix {tuple(t.shape)} has no half-blocks")
+    return t.split(h, axis)
+
+
 def _ring_os(algorithm, X, W, i, j, R, C):
     Wj = _gathered(_column(W, j, R), 0)                     # [Kd, n/C]
-    _need(X[i][j].shape[1], 2, "columns of an X shard"); _need(Wj.shape[0], 2 * C, "gathered rows of W")
-    h = Wj.shape[0] // C // 2
-    order = _ring_order(algorithm, "os", R, C, i, j)
-    A = _usable([X[i][b][:, hi * h:(hi + 1) * h] for b, hi in order])
-    Bs = [Wj[(2 * b + hi) * h:(2 * b + hi + 1) * h] for b, hi in order]
-    return local_gemm.gemm_os(A, Bs)
+    halves = _halves(_row(X, i, C), 1)
+    _need(Wj.shape[0], 2 * C, "gathered rows of W")
+    order = [2 * b + hi for b, hi in _ring_order(algorithm, "os", R, C, i, j)]
+    rows = _cut(Wj, Wj.shape[0] // C // 2, 0)
+    return local_gemm.gemm_os(_usable([halves[x] for x in order]), [rows[x] for x in order])
 
 
 def _ring_ls(algorithm, X, W, i, j, R, C):
     Wj = _gathered(_column(W, j, R), 0)                     # [O, I/C]
     _need(Wj.shape[0], 2 * C, "gathered rows of W")
     h = Wj.shape[0] // C // 2
-    order = _ring_order(algorithm, "ls", R, C, i, j)
-    Xij = _own(X[i][j])
+    order = [2 * b + hi for b, hi in _ring_order(algorithm, "ls", R, C, i, j)]
+    Xij = _own(_shard(X, i, j))
     part = torch.empty((Xij.shape[0], Wj.shape[0]), dtype=torch.float32, device=Xij.device)
-    outs = [part[:, (2 * b + hi) * h:(2 * b + hi + 1) * h] for b, hi in order]
-    if any(o.data_ptr() % 16 for o in outs):
+    rows, columns = _cut(Wj, h, 0), _cut(part, h, 1)
+    if any(columns[x].data_ptr() % 16 for x in order):
         raise ValueError(f"half-blocks of {h} output columns are not 16-byte aligned")
-    local_gemm.gemm_ls(Xij, [Wj[(2 * b + hi) * h:(2 * b + hi + 1) * h] for b, hi in order], out=outs)
+    local_gemm.gemm_ls(Xij, [rows[x] for x in order], out=[columns[x] for x in order])
     return [part]
 
 
 def _ring_rs(algorithm, X, W, i, j, R, C):
-    _need(X[i][j].shape[1], 2, "columns of an X shard")
-    h = X[i][j].shape[1] // 2
-    order = _ring_order(algorithm, "rs", R, C, i, j)
-    Xs = _usable([X[i][b][:, hi * h:(hi + 1) * h] for b, hi in order])
-    Wij = _own(W[i][j])
+    halves = _halves(_row(X, i, C), 1)
+    h = halves[0].shape[1]
+    order = [2 * b + hi for b, hi in _ring_order(algorithm, "rs", R, C, i, j)]
+    Xs = _usable([halves[x] for x in order])
+    Wij = _own(_shard(W, i, j))
     part = torch.empty((2 * h * C, Wij.shape[1]), dtype=torch.float32, device=Wij.device)
-    local_gemm.gemm_rs(Xs, Wij, out=[part[(2 * b + hi) * h:(2 * b + hi + 1) * h] for b, hi in order])
+    rows = _cut(part, h, 0)
+    local_gemm.gemm_rs(Xs, Wij, out=[rows[x] for x in order])
     return [part]
 
 

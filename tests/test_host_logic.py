@@ -432,3 +432,49 @@ def test_slices_of_32_rows_and_more_always_fit():
         for es in (2, 4):
             ldw = ((1 << 31) - 1) // (S * 32 * es)          # the widest W of S slices of 32 rows
             assert TP._steps_addressable(ldw * es, S)
+
+
+# ---------------------------------------------------------------- the half-blocks of the ring bodies
+@pytest.mark.parametrize("algorithm,R,C", [("wang", 1, 2), ("wang", 2, 4), ("cannon", 3, 3)])
+@pytest.mark.parametrize("flow", ["os", "ls", "rs"])
+def test_ring_bodies_cut_their_half_blocks_at_once_and_in_ring_order(flow, algorithm, R, C, monkeypatch):
+    """On CPU tensors, the product replaced: the blocks that it is given, in order, from shards as a grid of one matrix and as lists; and not
+    a view per access to a shard."""
+    m, n, k = 8 * R * C, 16 * R * C, 16 * R * C
+    X = torch.randn((k, m) if flow == "rs" else (m, k))
+    W = torch.randn((n, k) if flow == "ls" else (k, n))
+    seen = []
+    monkeypatch.setattr(TP.local_gemm, "gemm_" + flow, lambda a, b, out=None: seen.append((a, b, out)))
+    ring = {"os": TP._ring_os, "ls": TP._ring_ls, "rs": TP._ring_rs}[flow]
+    Xs, Ws = TP._shards(X, R, C), TP._shards(W, R, C)
+    cut = lambda t, b, hi, h, axis: t.narrow(axis, (2 * b + hi) * h, h)
+    for i in range(R):
+        for j in range(C):
+            order = TP._ring_order(algorithm, flow, R, C, i, j)
+            column = W[:, j * (W.shape[1] // C):(j + 1) * (W.shape[1] // C)]
+            row = X[i * (X.shape[0] // R):(i + 1) * (X.shape[0] // R)]
+            for grids in ((TP._Grid(X, R, C), TP._Grid(W, R, C)), (Xs, Ws)):
+                views = []
+                with monkeypatch.context() as patched:
+                    patched.setattr(torch.Tensor, "narrow", lambda t, *a, f=torch.Tensor.narrow: views.append(1) or f(t, *a))
+                    y = ring(algorithm, *grids, i, j, R, C)
+                assert len(views) <= 4
+                a, b, out = seen.pop()
+                if flow != "rs":
+                    h = column.shape[0] // C // 2
+                    assert all(torch.equal(v, cut(column, q, hi, h, 0)) for v, (q, hi) in zip(b, order)) and len(b) == 2 * C
+                if flow != "ls":
+                    h = row.shape[1] // C // 2
+                    assert all(torch.equal(v, cut(row, q, hi, h, 1)) for v, (q, hi) in zip(a, order)) and len(a) == 2 * C
+                if flow == "ls":
+                    assert torch.equal(a, Xs[i][j]) and all(v.data_ptr() == cut(y[0], q, hi, y[0].shape[1] // C // 2, 1).data_ptr() for v, (q, hi) in zip(out, order))
+                if flow == "rs":
+                    assert torch.equal(b, Ws[i][j]) and all(v.data_ptr() == cut(y[0], q, hi, y[0].shape[0] // C // 2, 0).data_ptr() for v, (q, hi) in zip(out, order))
+
+
+@pytest.mark.parametrize("flow", ["os", "rs"])
+def test_ring_bodies_refuse_what_has_no_half_blocks(flow):
+    for shape in ((8, 6), (8, 0)):
+        X, W = torch.zeros(shape), torch.zeros((shape[1] if flow == "os" else 8, 8))
+        with pytest.raises(ValueError):
+            (TP._ring_os if flow == "os" else TP._ring_rs)("wang", TP._Grid(X, 1, 2), TP._Grid(W, 1, 2), 0, 0, 1, 2)
