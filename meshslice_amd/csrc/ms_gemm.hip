@@ -382,6 +382,7 @@ int launch_bf16_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, 
 //  12: 256x384, 4 waves, 2 x 64 on the 16x16x32 MFMA (gemm_bf16_x16_kernel)     13: 256x256, the same kernel
 //  14: 128x128, 4 waves, 3 x 64 (one workgroup per unit: for products of at most one round of such tiles, where a third
 //      stage covers the load latency that two 64-deep stages do not: 2048^3 in 20.7 us against 26.3 us, 1536^3 14.7 against 18.8)
+//      (1 is never picked, 13 and 7 are faster: an id that can be forced, as before)
 //      2 and 4 are for outputs of one or two hundred such tiles, where 128x128 pays for more operand bytes per FLOP and
 //      256-wide tiles leave units idle: 2048 x 3072 x 4096 on 128x192 43 us, 128x128 50, 256x192 61; 3072^3 on 192x192 48 us, 256x192
 //      52; 1499 x 4104 x 3096 on 192x192 46 us, 128x128 57.  (128x256, 256x128 and 192x128 as well would give another 0.3 % over drawn products.)
