@@ -410,6 +410,25 @@ def test_a_native_call_path_that_does_not_load_says_why(error, says, monkeypatch
     assert got.value.__cause__ is error
 
 
+def test_importing_the_package_loads_no_native_code():
+    """The libraries come after the GPU runtime's own, which a process loads with its first tensor there."""
+    import subprocess
+    import sys
+    code = ("import meshslice_amd.TensorParallel; from meshslice_amd import _lib; maps = open('/proc/self/maps').read(); "
+            "assert 'libmeshslice_hip' not in maps and 'meshslice_amd/_host' not in maps; assert callable(_lib.host.gemm_os) and callable(_lib.host.gemm_ls); "
+            "assert type(_lib.host).__name__ == 'module' and 'libmeshslice_hip' in open('/proc/self/maps').read()")
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+
+
+def test_the_native_call_path_has_no_thread_local_variables():
+    """One that no call reads would keep the search going that the order of loading ends."""
+    import importlib.util
+    elf = open(importlib.util.find_spec("meshslice_amd._host").origin, "rb").read()
+    start, (size, count) = int.from_bytes(elf[32:40], "little"), (int.from_bytes(elf[o:o + 2], "little") for o in (54, 56))
+    kinds = [int.from_bytes(elf[start + i * size:start + i * size + 4], "little") for i in range(count)]
+    assert elf[:6] == b"\x7fELF\x02\x01" and 1 in kinds and 7 not in kinds      # 1: loaded, 7: thread-local storage
+
+
 # ---------------------------------------------------------------- row slices read in place: 32-bit offsets
 @pytest.mark.parametrize("S,k_slice,ldw,es", [(8, 8, 1 << 23, 2), (64, 8, 1 << 20, 2), (2, 16, (1 << 25) - 8, 2), (4, 8, (1 << 24) - 4, 4)])
 def test_a_k_step_of_slices_in_place_stays_within_32_bits(S, k_slice, ldw, es):
