@@ -54,8 +54,8 @@ class _Line:
     """The shards of one mesh row or column of a global matrix, in axis order: the views, made where they are asked for, and
     the one view that covers them."""
 
-    def __init__(self, panel: torch.Tensor, n: int, axis: int):
-        self.panel, self.n, self.axis, self.step = panel, n, axis, panel.shape[axis] // n
+    def __init__(self, panel: torch.Tensor, n: int, axis: int, step=None):
+        self.panel, self.n, self.axis, self.step = panel, n, axis, panel.shape[axis] // n if step is None else step
 
     def __len__(self):
         return self.n
@@ -65,6 +65,10 @@ class _Line:
             raise IndexError(p)
         return self.panel.narrow(self.axis, p % self.n * self.step, self.step)
 
+    def blocks(self):
+        """All of them, in one cut."""
+        return self.panel.chunk(self.n, self.axis) if self.step else list(self)
+
 
 class _Grid:
     """_shards without the R * C views: ``grid[i]`` is mesh row i's shards, ``_column(grid, j)`` mesh column j's."""
@@ -72,9 +76,10 @@ class _Grid:
     def __init__(self, G: torch.Tensor, R: int, C: int):
         if G.dim() != 2:
             raise ValueError("operands must be 2-D")
-        if G.shape[0] % R or G.shape[1] % C:
+        h, w = G.shape
+        if h % R or w % C:
             raise ValueError(f"matrix {tuple(G.shape)} does not shard evenly over a {R}x{C} mesh")
-        self.G, self.R, self.C, self.h, self.w = G, R, C, G.shape[0] // R, G.shape[1] // C
+        self.G, self.R, self.C, self.h, self.w = G, R, C, h // R, w // C
 
     def __len__(self):
         return self.R
@@ -82,7 +87,7 @@ class _Grid:
     def __getitem__(self, i):
         if not -self.R <= i < self.R:
             raise IndexError(i)
-        return _Line(self.G.narrow(0, i % self.R * self.h, self.h), self.C, 1)
+        return _Line(self.G.narrow(0, i % self.R * self.h, self.h), self.C, 1, self.w)
 
 
 def _row(grid, i, C):
@@ -90,11 +95,17 @@ def _row(grid, i, C):
 
 
 def _column(grid, j, R):
-    return _Line(grid.G.narrow(1, j * grid.w, grid.w), R, 0) if isinstance(grid, _Grid) else [grid[i][j] for i in range(R)]
+    return _Line(grid.G.narrow(1, j * grid.w, grid.w), R, 0, grid.h) if isinstance(grid, _Grid) else [grid[i][j] for i in range(R)]
 
 
 def _shard(grid, i, j):
     return grid.G.narrow(0, i * grid.h, grid.h).narrow(1, j * grid.w, grid.w) if isinstance(grid, _Grid) else grid[i][j]
+
+
+def _blocks(parts) -> Sequence[torch.Tensor]:
+    """The shards of a mesh line as views, for a body that takes each of them more than once: a view per access to them took the overlapped OS body
+    of 2x2 devices in eight slices (2048 x 2048 x 2048, fp32) 697 us, 586 as one cut."""
+    return parts.blocks() if isinstance(parts, _Line) else parts
 
 
 def _need(v: int, d: int, what: str) -> None:
@@ -116,7 +127,7 @@ def _own(block: torch.Tensor) -> torch.Tensor:
 def _gather(parts: Sequence[torch.Tensor], axis: int) -> torch.Tensor:
     """tiled all_gather of whole shards as the receiving device sees it: peers' parts concatenated in axis
     order, materialised contiguous in HBM (what a real all-gather delivers)."""
-    return torch.cat(list(parts), dim=axis).contiguous()
+    return torch.cat(tuple(_blocks(parts)), dim=axis).contiguous()
 
 
 PANEL_MAX_ROWS = 65535 * 8      # rows that one launch of the layout kernels always takes
@@ -262,6 +273,7 @@ OVERLAP_RESERVED_CUS = 32      # compute units left to the emulated gathers' cop
 def _col_slice_filler(peers, K, B):
     """(buffer ``[K, rows, len(peers) * cols / K]`` for the K gathered column slices, ``fill(k)`` that gathers slice k into
     it on the current stream): slice k of a shard is its B-wide column blocks b with b % K == k (reference :155,157,198-199)."""
+    peers = _blocks(peers)
     r, c = peers[0].shape
     _need(c, K * B, "sliced extent")
     w = c // K
@@ -275,6 +287,7 @@ def _col_slice_filler(peers, K, B):
 
 def _row_slice_filler(peers, K, B):
     """The same for the K gathered row slices ``[K, len(peers) * rows / K, cols]`` (reference :156,158,177-178)."""
+    peers = _blocks(peers)
     h, n = peers[0].shape
     _need(h, K * B, "sliced extent")
     hk = h // K
@@ -454,7 +467,7 @@ def _halves(parts, axis: int) -> Sequence[torch.Tensor]:
 def _cut(t: torch.Tensor, h: int, axis: int) -> Sequence[torch.Tensor]:
     if h < 1:
         raise ValueError(f"matrix {tuple(t.shape)} has no half-blocks")
-    return t.split(h, axis)
+    return t.chunk(t.shape[axis] // h, axis)
 
 
 def _ring_os(algorithm, X, W, i, j, R, C):

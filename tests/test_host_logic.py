@@ -491,6 +491,24 @@ def test_ring_bodies_cut_their_half_blocks_at_once_and_in_ring_order(flow, algor
                     assert torch.equal(b, Ws[i][j]) and all(v.data_ptr() == cut(y[0], q, hi, y[0].shape[0] // C // 2, 0).data_ptr() for v, (q, hi) in zip(out, order))
 
 
+@pytest.mark.parametrize("axis", [0, 1])
+def test_fillers_take_a_view_of_each_shard_once(axis, monkeypatch):
+    """The emulated gathers of the overlapped bodies, slice after slice, from the shards of one matrix as a line and as a list."""
+    n, K, B = 3, 4, 8
+    G = torch.randn((n * K * B * 2, 24) if axis == 0 else (24, n * K * B * 2))
+    shards, filler = list(G.chunk(n, axis)), TP._row_slice_filler if axis == 0 else TP._col_slice_filler
+    cut = lambda t, k: torch.cat(list(t.split(B, axis))[k::K], axis)
+    for peers in (TP._Line(G, n, axis), shards):
+        views = []
+        monkeypatch.setattr(TP._Line, "__getitem__", lambda line, p, f=TP._Line.__getitem__: views.append(p) or f(line, p))
+        buf, fill = filler(peers, K, B)
+        for k in range(K):
+            fill(k)
+            assert torch.equal(buf[k], torch.cat([cut(s, k) for s in shards], axis))
+        assert not views
+        monkeypatch.undo()
+
+
 @pytest.mark.parametrize("flow", ["os", "rs"])
 def test_ring_bodies_refuse_what_has_no_half_blocks(flow):
     for shape in ((8, 6), (8, 0)):
