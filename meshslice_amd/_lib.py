@@ -182,8 +182,8 @@ class _Host:
     """Stands for the native call path until its first use loads it, by when the caller's tensors have initialised the GPU.  Where the library that was
     loaded last has thread-local variables and a thread reads none of them, glibc before 2.39 searches for every other library's on each access.  The C
     library's are read on each call, so it has to come after the GPU runtime's own libraries; loaded before them it left the tensor properties that
-    Python reads 25 % slower for the whole process: the checks of gemm_os of two slices 4.5 -> 5.8 us, the call with ``out=`` 13.5 -> 15.9, an
-    overlapped body of 2x2 devices 400 -> 460."""
+    Python reads 25 % slower for the whole process: the checks of gemm_os of two slices 4.5 -> 5.8 us, the call with ``out=`` 13.2 -> 15.9, an
+    overlapped body of 2x2 devices 421 -> 460."""
 
     def __getattr__(self, name):
         global host
