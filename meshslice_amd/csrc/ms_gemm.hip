@@ -529,8 +529,8 @@ double partial_round_loss(int v) { return v == 3 || v == 14 || v == SMALL || v =
 bool carries_sum(int v) { return v == 2 || v == 4 || v == 14; }
 constexpr double FOLD_K = 90.0;
 
-// A 128-deep K step of an operand whose rows lie along the contraction loads up to sixteen blocks of eight rows on, with 32-bit offsets:
-// where those would wrap around (rows of more than 32 MB) they would fetch rows of the slice instead of zeros.
+// Whether sixteen blocks of eight rows, a 128-deep K step of an operand whose rows lie along the contraction, span at most 4 GiB.  Where they span more (rows
+// of more than 32 MB) a slice, of less than 2 GiB, has fewer than 64 rows: more than half of the step would be padding, and the 64-deep tiles are the ones to take.
 bool small_tile_reaches(const Problem &p) {
   const long long es = p.in_dtype == MS_DTYPE_BF16 ? 2 : 4;
   const long long a_blk = p.flow == RS ? 8LL * p.lda * es : 0, b_blk = p.flow == LS ? 0 : p.b_blk ? (long long)p.b_blk : 8LL * p.ldb * es;
