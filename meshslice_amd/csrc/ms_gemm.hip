@@ -72,6 +72,21 @@ MS_INSTANTIATE_SUM(128, 128)
 MS_INSTANTIATE_SUM(128, 192)
 MS_INSTANTIATE_SUM(192, 192)
 #undef MS_INSTANTIATE_SUM
+// operands whose rows along the contraction are too far apart for the other kernels' offsets (Operand's FAR, reaches): one tile of each type
+#define MS_INSTANTIATE_FAR(AK, OBF, EPI, FOLD) \
+  template __global__ void msk::gemm_bf16_ring_kernel<128, 128, 64, 3, 2, 2, AK, false, OBF, EPI, FOLD, false, true>(const msk::GemmArgs);
+MS_INSTANTIATE_FAR(true, true, false, false)
+MS_INSTANTIATE_FAR(true, false, false, false)
+MS_INSTANTIATE_FAR(true, true, true, false)
+MS_INSTANTIATE_FAR(true, false, true, false)
+MS_INSTANTIATE_FAR(false, true, false, false)
+MS_INSTANTIATE_FAR(false, false, false, false)
+MS_INSTANTIATE_FAR(false, true, false, true)
+#undef MS_INSTANTIATE_FAR
+template __global__ void msk::gemm_f32_tile_kernel<2, 2, 1, 1, true, false, true, false, true>(const msk::GemmArgs);
+template __global__ void msk::gemm_f32_tile_kernel<2, 2, 1, 1, true, false, false, false, true>(const msk::GemmArgs);
+template __global__ void msk::gemm_f32_tile_kernel<2, 2, 1, 1, false, false, true, false, true>(const msk::GemmArgs);
+template __global__ void msk::gemm_f32_tile_kernel<2, 2, 1, 1, false, false, false, false, true>(const msk::GemmArgs);
 #define MS_INSTANTIATE_BIG(TM, TN)                                                                             \
   template __global__ void msk::gemm_bf16_big_kernel<TM, TN, true, false, true, false>(const msk::GemmArgs);   \
   template __global__ void msk::gemm_bf16_big_kernel<TM, TN, true, false, false, false>(const msk::GemmArgs);  \
@@ -336,8 +351,16 @@ int workgroups_per_unit(int variant) { return variant == 3 && g_reserved_cus == 
 extern const char *const SPLIT_REFUSALS[];
 int split_refused(const Problem &p, const DevFacts &dev, int variant, int splits);
 
-// tile BM x BN, WGM x WGN waves, NS ring stages of BK_ k-elements; contraction split `splits` ways
-template <int BM, int BN, int WGM, int WGN, int BK_, int NS, int KIND = 0>
+// Whether the 32-bit offsets of a K step of `step` elements reach: they are counted for all of its rows, also for those that a short slice does not have.
+// Beyond 4 GiB they would wrap around to rows that it has.
+bool reaches(const Problem &p, int step) {
+  const long long es = p.in_dtype == MS_DTYPE_BF16 ? 2 : 4;
+  const long long a_blk = p.flow == RS ? 8LL * p.lda * es : 0, b_blk = p.flow == LS ? 0 : p.b_blk ? (long long)p.b_blk : 8LL * p.ldb * es;
+  return step / 8 * (a_blk > b_blk ? a_blk : b_blk) <= 0x100000000LL;
+}
+
+// tile BM x BN, WGM x WGN waves, NS ring stages of BK_ k-elements; contraction split `splits` ways; FAR: for operands that the tile does not reach
+template <int BM, int BN, int WGM, int WGN, int BK_, int NS, int KIND = 0, bool FAR = false>
 int launch_bf16_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, int variant, int splits) {
   msk::GemmArgs g;
   memset(&g, 0, sizeof(g));
@@ -376,7 +399,15 @@ int launch_bf16_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, 
   const bool obf = p.out_dtype == MS_DTYPE_BF16;
   g.act = p.act; g.res = p.res; g.ldr = p.ldr; g.row_sum = p.row_sum; g.row_sumsq = p.row_sumsq;
   const bool epi = p.act != 0 || p.res || p.row_sum || p.row_sumsq;
-  if (p.sum) {
+  if constexpr (FAR) {
+    if (p.sum) msk::gemm_bf16_ring_kernel<BM, BN, BK_, NS, WGM, WGN, false, false, true, false, true, false, true><<<gd, bd, 0, stream>>>(g);
+    else if (p.flow == OS && epi && obf) msk::gemm_bf16_ring_kernel<BM, BN, BK_, NS, WGM, WGN, true, false, true, true, false, false, true><<<gd, bd, 0, stream>>>(g);
+    else if (p.flow == OS && epi) msk::gemm_bf16_ring_kernel<BM, BN, BK_, NS, WGM, WGN, true, false, false, true, false, false, true><<<gd, bd, 0, stream>>>(g);
+    else if (p.flow == OS && obf) msk::gemm_bf16_ring_kernel<BM, BN, BK_, NS, WGM, WGN, true, false, true, false, false, false, true><<<gd, bd, 0, stream>>>(g);
+    else if (p.flow == OS) msk::gemm_bf16_ring_kernel<BM, BN, BK_, NS, WGM, WGN, true, false, false, false, false, false, true><<<gd, bd, 0, stream>>>(g);
+    else if (obf) msk::gemm_bf16_ring_kernel<BM, BN, BK_, NS, WGM, WGN, false, false, true, false, false, false, true><<<gd, bd, 0, stream>>>(g);
+    else msk::gemm_bf16_ring_kernel<BM, BN, BK_, NS, WGM, WGN, false, false, false, false, false, false, true><<<gd, bd, 0, stream>>>(g);
+  } else if (p.sum) {
     if constexpr (KIND == 0 && NS == 3 && BM > 64) {
       if (g.splits > 1) {
         if (p.flow == LS) msk::gemm_bf16_ring_kernel<BM, BN, BK_, NS, WGM, WGN, true, true, true, false, true, true><<<gd, bd, 0, stream>>>(g);
@@ -461,6 +492,7 @@ constexpr int VARIANTS = 14;
 constexpr int SMALL = 18, FLAT = 19;              // the 64x64 and 64x128 tiles (15 to 17: the sums over devices on 14, 4, 2)
 constexpr int F32_FIRST = 21, F32_LAST = 25;      // ids of the fp32 kernel's tiles (ms_set_variant, MS_QUERY_LAST_VARIANT)
 constexpr int F32_WAVES = 28;                     // gemm_f32_waves_kernel
+constexpr int F32_STEP = 32, F32_FAR = 24;        // its K step, and the tile of operands that this does not reach
 constexpr int F32_NARROW = 26;                    // and of the two that only the chooser takes (64 x 192, 64 x 128; not ms_set_variant)
 struct TileShape { int bm, bn; };
 constexpr TileShape TILE_OF[FLAT + 1] = {{0, 0},     {256, 256}, {192, 192}, {128, 128}, {128, 192}, {256, 192},
@@ -529,14 +561,6 @@ double partial_round_loss(int v) { return v == 3 || v == 14 || v == SMALL || v =
 bool carries_sum(int v) { return v == 2 || v == 4 || v == 14; }
 constexpr double FOLD_K = 90.0;
 
-// Whether sixteen blocks of eight rows, a 128-deep K step of an operand whose rows lie along the contraction, span at most 4 GiB.  Where they span more (rows
-// of more than 32 MB) a slice, of less than 2 GiB, has fewer than 64 rows: more than half of the step would be padding, and the 64-deep tiles are the ones to take.
-bool small_tile_reaches(const Problem &p) {
-  const long long es = p.in_dtype == MS_DTYPE_BF16 ? 2 : 4;
-  const long long a_blk = p.flow == RS ? 8LL * p.lda * es : 0, b_blk = p.flow == LS ? 0 : p.b_blk ? (long long)p.b_blk : 8LL * p.ldb * es;
-  return 16 * (a_blk > b_blk ? a_blk : b_blk) <= 0x100000000LL;
-}
-
 // Unsplit output-stationary products of more than half a round of 64x64 tiles take them below this many contraction elements: from there on 128x128
 // in three or four parts is ahead on ten of twelve drawn products (483 x 1944 x 9472: 30.1 against 44.2 us, 1406 x 472 x 4488 20.4 against
 // 22.1; 1024 x 768 x 4096 is one that loses, 17.6 against 15.0).
@@ -557,7 +581,7 @@ Pick pick_variant(const Problem &p, const DevFacts &dev, bool small = true) {
   Pick best = {0, 1, 0};
   for (const TileRate &c : TILE_RATES) {
     if (p.sum && !carries_sum(c.v)) continue;
-    if ((c.v == SMALL && !(small && small_tile_reaches(p))) || (c.v == FLAT && !small)) continue;
+    if ((c.v == SMALL && (!small || !reaches(p, k_step(SMALL)))) || (c.v == FLAT && !small)) continue;
     const int bm = TILE_OF[c.v].bm, bn = TILE_OF[c.v].bn;
     const bool pairs = workgroups_per_unit(c.v) == 2;
     const double rate = rs ? c.rs : ls ? c.ls : c.os;
@@ -605,7 +629,7 @@ Pick pick_variant(const Problem &p, const DevFacts &dev, bool small = true) {
 
 int launch_variant(int v, int splits, const Problem &p, const DevFacts &dev, hipStream_t stream) {
   if (p.slice_ready && v == 1) return fail(MS_ERR_UNSUPPORTED, "tile variant %d has no input gate (256x256 on four waves of the ring kernel)", v);
-  if (v == SMALL && !small_tile_reaches(p)) return fail(MS_ERR_UNSUPPORTED, "tile variant %d does not reach rows of more than 32 MB", v);
+  if (!reaches(p, k_step(v))) return fail(MS_ERR_UNSUPPORTED, "tile variant %d does not reach rows of more than %d MB", v, 4096 / k_step(v));
   // (the kernels that add up devices' sums go by ids of their own: 15 to 17 for the tiles 14, 4 and 2)
   if (g_launches == 0) { g_last_variant = !p.sum ? v : v == 14 ? 15 : v == 4 ? 16 : 17; g_last_splits = splits; }
   switch (v) {
@@ -637,7 +661,14 @@ int launch_variant(int v, int splits, const Problem &p, const DevFacts &dev, hip
 // their chunks are promised in slice order.
 int launch_bf16(const Problem &p, const DevFacts &dev, hipStream_t stream) {
   if (!dev.gfx950) return fail(MS_ERR_UNSUPPORTED, "the bf16 kernels need a gfx950 device");
-  if (is_bf16_tile(g_variant) && (!p.sum || carries_sum(g_variant))) return launch_variant(g_variant, g_splits > 1 ? g_splits : 1, p, dev, stream);
+  const bool forced = is_bf16_tile(g_variant) && (!p.sum || carries_sum(g_variant));
+  if (!reaches(p, k_step(14))) {
+    if ((forced && g_variant != 14) || (g_splits > 1 && !p.sum))
+      return fail(MS_ERR_UNSUPPORTED, "tile variant %d in %d parts does not reach rows of more than %d MB", g_variant, g_splits > 1 ? g_splits : 1, 4096 / k_step(14));
+    if (g_launches == 0) { g_last_variant = p.sum ? 15 : 14; g_last_splits = 1; }
+    return launch_bf16_tile<128, 128, 2, 2, 64, 3, 0, true>(p, dev, stream, 14, 1);
+  }
+  if (forced) return launch_variant(g_variant, g_splits > 1 ? g_splits : 1, p, dev, stream);
   const Pick single = pick_variant(p, dev);
   // (a gated product stays one launch: a second one would stand in the stream behind the first while that waits for slices)
   if (p.flow == OS && single.splits == 1 && g_splits == 0 && !p.slice_ready) {
@@ -703,7 +734,7 @@ int fill_f32_args(const Problem &p, int bm, int bn, msk::GemmArgs &g, long &tota
   return MS_OK;
 }
 
-template <int WGM, int WGN, int TM, int TN>
+template <int WGM, int WGN, int TM, int TN, bool FAR = false>
 int launch_f32_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, int id, bool share, int splits) {
   constexpr int BM = 32 * TM * WGM, BN = 32 * TN * WGN;
   msk::GemmArgs g;
@@ -723,7 +754,12 @@ int launch_f32_tile(const Problem &p, const DevFacts &dev, hipStream_t stream, i
   msk::set_walk(g, grid);
   dim3 gd(grid), bd(WGM * WGN * 64);
   const bool obf = p.out_dtype == MS_DTYPE_BF16;
-  if (p.flow == OS) {
+  if constexpr (FAR) {
+    if (p.flow == OS && obf) msk::gemm_f32_tile_kernel<WGM, WGN, TM, TN, true, false, true, false, true><<<gd, bd, 0, stream>>>(g);
+    else if (p.flow == OS) msk::gemm_f32_tile_kernel<WGM, WGN, TM, TN, true, false, false, false, true><<<gd, bd, 0, stream>>>(g);
+    else if (obf) msk::gemm_f32_tile_kernel<WGM, WGN, TM, TN, false, false, true, false, true><<<gd, bd, 0, stream>>>(g);
+    else msk::gemm_f32_tile_kernel<WGM, WGN, TM, TN, false, false, false, false, true><<<gd, bd, 0, stream>>>(g);
+  } else if (p.flow == OS) {
     if (g.splits > 1) {
       if (obf) msk::gemm_f32_tile_kernel<WGM, WGN, TM, TN, true, false, true, true><<<gd, bd, 0, stream>>>(g);
       else msk::gemm_f32_tile_kernel<WGM, WGN, TM, TN, true, false, false, true><<<gd, bd, 0, stream>>>(g);
@@ -871,6 +907,10 @@ F32Pick pick_f32(const Problem &p, const DevFacts &dev) {
 }
 
 int launch_f32(const Problem &p, const DevFacts &dev, hipStream_t stream) {
+  if (!reaches(p, F32_STEP)) {
+    if (g_splits > 1 || (g_variant >= F32_FIRST && g_variant != F32_FAR)) return fail(MS_ERR_UNSUPPORTED, "fp32 tile variant %d does not reach rows of more than %d MB", g_variant, 4096 / F32_STEP);
+    return launch_f32_tile<2, 2, 1, 1, true>(p, dev, stream, F32_FAR, false, 1);
+  }
   if (g_variant == F32_WAVES) return launch_f32_waves(p, dev, stream);
   const F32Pick best = pick_f32(p, dev);
   if (best.id == 0) return fail(MS_ERR_ARG, "contraction cannot be split %d ways on fp32 tile %d here", g_splits, g_variant);
