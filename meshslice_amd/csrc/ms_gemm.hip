@@ -511,6 +511,10 @@ constexpr int SPLIT_CHOICES[] = {1, 2, 3, 4, 6, 8};
 constexpr int SPLIT_MAX = 8;
 constexpr long SPLIT_MIN_K = 256;            // contraction elements per split item, at least
 constexpr double SPLIT_FIX = 4e6;            // fixed cost of an exchange (about 1.4 us),
+// a sum over devices has more to gain from staying whole: its parts are the devices, however short each one's share is.  On 300 drawn sums of 2 to 8 devices
+// (m and n 64 to 12288) the choice takes 1.0047 of the best tile's and way's time with this, 1.0075 with SPLIT_FIX, 1.0049 with 1.0e7, 1.0069 with 1.7e7: RS 384 x 3712
+// x 736 of four devices 23.0 us whole, 29.5 in four parts, LS 411 x 1280 x 280 of four 16.6 and 20.2
+constexpr double SUM_SPLIT_FIX = 1.3e7;
 constexpr double SPLIT_PER_PART = 1.3e6;     // per part (half a microsecond: a block's last arriver reads the parts one after the other),
 constexpr double SPLIT_PER_ELEMENT = 7.9;    // per part and output element (8 bytes through memory)
 
@@ -605,7 +609,7 @@ Pick pick_variant(const Problem &p, const DevFacts &dev, bool small = true) {
       const double loss = partial_round_loss(c.v);
       const double part = exact + loss * (1.0 - exact);
       const double rounds = exact <= 1.0 ? (part > 0.7 ? part : 0.7) : exact + loss * (whole - exact);
-      const double exchange = splits == 1 ? 0.0 : SPLIT_FIX + splits * (SPLIT_PER_PART + (double)p.M * p.N * SPLIT_PER_ELEMENT);
+      const double exchange = splits == 1 ? 0.0 : (p.sum ? SUM_SPLIT_FIX : SPLIT_FIX) + splits * (SPLIT_PER_PART + (double)p.M * p.N * SPLIT_PER_ELEMENT);
       // (two 128x128 workgroups share a unit only where there are more tiles than units)
       const double shared = !pairs || tiles * splits <= dev.cus ? 0.0 : tiles * splits >= 2L * dev.cus ? 1.0 : (double)(tiles * splits - dev.cus) / dev.cus;
       const double eff = splits > 1 ? c.split : rate - (pairs ? (rate - (rs ? PAIRED_RS : ls ? PAIRED_LS : PAIRED_OS)) * shared : 0.0);
@@ -1341,7 +1345,7 @@ MS_API int ms_prefers_sum(int rs, int P, int S, int m, int n, int k) {
   const double mb = 1e-6, part_lines = rs ? 0.5 * ((m % 64 != 0) + (n % 64 != 0)) : 0.0;
   const double operands = 2.0 * ((double)m + n) * P * k, copied = 2.0 * (rs ? m : n) * (double)P * k, chunk_bytes = 4.0 * P * (double)m * n;
   const double cold = operands > 256e6 ? operands - 256e6 : 0.0;
-  // (chunks are priced without the 64-row tiles, as the constants were fitted: no sum runs on them)
+  // (chunks run on the 64-row tiles as well where those are faster, but the constants were fitted to their price without: the choice errs to the side of registers)
   const double sum_us = pick_variant(p, facts).cost * P * k * SUM_UNIT_US * SUM_SCALE * (1.0 + SUM_RS_PART_LINES * part_lines) + SUM_LAUNCH_US + cold * mb * SUM_COLD_US_PER_MB;
   double chunks_us = pick_variant(chunks, facts, false).cost * k * SUM_UNIT_US * CHUNK_SCALE + chunk_bytes * mb * CHUNK_US_PER_MB + copied * mb * CHUNK_COPY_US_PER_MB + CHUNK_LAUNCHES_US;
   const double host_us = CHUNK_HOST_US + P * (CHUNK_HOST_PEER_US + CHUNK_HOST_SLICE_US * (S - 1));
