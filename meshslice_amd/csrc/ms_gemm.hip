@@ -573,13 +573,14 @@ constexpr double SMALL_OS_MAX_K = 4096.0;
 // 10.0 us against 8.9 on 96 of 128x128), and their rate where the whole device runs them for more than one (LS 1871 x 24 x 10016 in sixteen chunks, 480
 // tiles, 85 us against 71 on 240 of 128x128)
 constexpr double SMALL_ROUND = 2.5e6, SMALL_CROWDED = 1.1;
+constexpr double L2S_BYTES = 28e6;      // what of an operand the eight XCDs' L2s (32 MB) hold beside the rest
 
 // the tile shape and split count with the lowest estimated cost for the whole problem (`small`: the 64-row tiles among them)
 Pick pick_variant(const Problem &p, const DevFacts &dev, bool small = true) {
   const bool rs = p.flow == RS, ls = p.flow == LS;
   const long chunks = p.flow == OS || p.sum ? 1 : p.S;
   const double total_k = p.flow == OS || p.sum ? (double)p.K * p.S : (double)p.K;
-  const double whole_k = (double)((p.K + 63) / 64 * 64) * (p.flow == OS || p.sum ? p.S : 1);      // (the 64x64 tile feels the tails of short slices)
+  const double whole_k = (double)((p.K + 63) / 64 * 64) * (p.flow == OS || p.sum ? p.S : 1);      // (the 64x64 tile feels the tails of short slices: 500 drawn OS products take 1.016 of the best tile's time with tails rounded up to 64, 1.018 to its step of 128, or not at all)
   const long small_tiles = (long)((p.M + 63) / 64) * ((p.N + 63) / 64) * chunks;
   const int forced_splits = p.sum ? 0 : g_splits;      // (a split count is forced on output-stationary products)
   Pick best = {0, 1, 0};
@@ -596,8 +597,13 @@ Pick pick_variant(const Problem &p, const DevFacts &dev, bool small = true) {
       // (64x128 is for where 64x64 makes more than half a round: below, the smaller tile is ahead, 365 x 368 x 432 in six slices 6.8 against 8.2 us)
       if (c.v == FLAT && splits == 1 && 2 * small_tiles <= dev.cus) continue;
       // (chunks of one 64-row tile leave it no more tiles than 128x128 and half the bytes in flight: RS 48 x 5432 x 4393 in four chunks 39 us against 32; up to
-      // 2048 contraction elements its shorter steps win, RS 40 x 1496 x 1361 in sixteen 10.7 against 12.2)
-      if (c.v == FLAT && splits == 1 && p.M <= 64 && total_k >= 2048.0) continue;
+      // 2048 contraction elements its shorter steps win, RS 40 x 1496 x 1361 in sixteen 10.7 against 12.2, but less of it where 128x128 makes one round of two
+      // workgroups a unit and it makes two: RS 256 x 4048 x 642 in sixteen, 512 tiles, 15.4 against 17.5, 512 x 3904 x 889 15.3 against 20.0; 384 x 3520 x 292, 448 tiles, 8.6 against 8.3)
+      if (c.v == FLAT && splits == 1 && p.M <= 64 && (total_k >= 2048.0 || (tiles > dev.cus && tiles <= 2L * dev.cus && tiles * total_k >= 1200.0 * dev.cus))) continue;
+      // (RS chunks of one 64-row tile do nothing but stream W, and of a W whose rows are no whole lines 64 columns fetch two lines for one.  With most of the units at that,
+      // and W beyond what the L2s hold, the fabric is what they wait for: RS 72 x 5256 x 9701 in three chunks 82.8 us, 64.4 on 126 tiles of 128x128, 112 x 7024 x 7648 in two
+      // 54.4 and 45.9, 48 x 2632 x 6867 in six 43.1 and 40.3; of ten such products in 1200 drawn ones two lose, 0.92 and 0.94)
+      if (c.v == SMALL && splits == 1 && rs && p.M <= 64 && p.N % 64 != 0 && tiles <= dev.cus && 4 * tiles > 3L * dev.cus && 2.0 * p.N * total_k > L2S_BYTES) continue;
       if (c.v == SMALL && splits == 1 && forced_splits == 0 && 2 * tiles > dev.cus && total_k >= SMALL_OS_MAX_K && !split_refused(p, dev, 14, 3)) continue;
       if (splits > 1 && (split_refused(p, dev, c.v, splits) || (forced_splits == 0 && total_k / splits < SPLIT_MIN_K))) continue;
       // rounds the launch is charged: whole ones, or with the last round partly filled (see balanced_grid) its filled
