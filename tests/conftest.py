@@ -21,6 +21,29 @@ def _gpu_available():
         return False
 
 
+@pytest.fixture
+def stream_beside():
+    """``f(*streams)``: a stream whose work has been seen to run while a launch on each of ``streams`` waits.  The streams of a process share a few hardware
+    queues, and two that share one run in order: whether a fresh stream shares another's depends on how many there were before it."""
+    import torch
+    from meshslice_amd import TensorParallel as TP
+
+    def find(*streams):
+        dev = streams[0].device
+        torch.cuda.synchronize(dev)
+        for _ in range(12):
+            other = torch.cuda.Stream(dev)
+            for cur in streams:
+                with torch.cuda.stream(cur):
+                    if not TP._runs_beside(cur, other, dev):
+                        break
+            else:
+                torch.cuda.synchronize(dev)
+                return other
+        pytest.skip("no stream runs beside a waiting launch on this machine")
+    return find
+
+
 def pytest_collection_modifyitems(config, items):
     if _gpu_available():
         return

@@ -55,7 +55,7 @@ def test_with_every_flag_set_the_gated_call_equals_the_plain_one(variant, dtype)
     assert orc.rel_frobenius(got.float().cpu().numpy(), orc.oracle_os_block([a.float().cpu().numpy() for a in A], [b.float().cpu().numpy() for b in B])) <= tol
 
 
-def test_slices_filled_and_flagged_by_another_stream_after_the_launch():
+def test_slices_filled_and_flagged_by_another_stream_after_the_launch(stream_beside):
     """The operand buffers hold zeros when the product is launched; a second stream then fills slice after slice and
     raises its flag.  A kernel that read a slice before its flag would add zeros for it."""
     S, m, n, k = 4, 2048, 3072, 1024
@@ -65,7 +65,7 @@ def test_slices_filled_and_flagged_by_another_stream_after_the_launch():
     ready = torch.zeros(S + 1, dtype=torch.int32, device="cuda")
     torch.cuda.synchronize()
     lib = _lib.load()
-    producer = torch.cuda.Stream()
+    producer = stream_beside(torch.cuda.current_stream())
     try:
         assert lib.ms_set_reserved_cus(16) == 0      # the producer's copies need compute units beside the waiting product
         got = ms.gemm_os_gated(A, B, ready, timeout_ms=1500)
@@ -181,7 +181,7 @@ def test_with_every_flag_set_the_gated_chunk_calls_equal_the_plain_ones(variant,
 
 
 @pytest.mark.parametrize("flow", ["ls", "rs"])
-def test_chunk_slices_flagged_in_reverse_order_by_another_stream_after_the_launch(flow):
+def test_chunk_slices_flagged_in_reverse_order_by_another_stream_after_the_launch(flow, stream_beside):
     """The gathered operand's buffers hold zeros at the launch; a second stream fills them LAST SLICE FIRST and raises
     each flag, and the completion counters are watched: every chunk is the product of the filled data, so each
     workgroup waited for its own chunk's flag and for no other."""
@@ -192,7 +192,7 @@ def test_chunk_slices_flagged_in_reverse_order_by_another_stream_after_the_launc
     ops[which] = [torch.zeros_like(t) for t in src[which]]
     ready = torch.zeros(S + 1, dtype=torch.int32, device="cuda")
     done = torch.zeros(S, dtype=torch.int32, device="cuda")
-    producer = torch.cuda.Stream()
+    producer = stream_beside(torch.cuda.current_stream())
     try:
         assert lib.ms_set_reserved_cus(32) == 0      # the producer's copies need compute units beside the waiting product
         want = _plain(flow, src)

@@ -109,7 +109,7 @@ def test_a_watcher_sees_chunks_complete_before_the_kernel_ends(flow):
 
 
 @pytest.mark.parametrize("flow", ["ls", "rs"])
-def test_one_launch_with_both_ends_open_hands_on_chunk_0_before_the_last_slice_has_arrived(flow):
+def test_one_launch_with_both_ends_open_hands_on_chunk_0_before_the_last_slice_has_arrived(flow, stream_beside):
     """ms_gemm_ls_gated / ms_gemm_rs_gated with completion counters: the product is enqueued first, a producer stream
     then delivers slice after slice about 150 us apart (a copy, a delay, the flag), and a watcher polls flags and
     counters from the host.  Chunk 0 must be seen complete while the last flag is still down: the launch multiplies what
@@ -126,7 +126,9 @@ def test_one_launch_with_both_ends_open_hands_on_chunk_0_before_the_last_slice_h
     done = torch.zeros(S, dtype=torch.int32, device="cuda")
     seen_ready = torch.zeros(S + 1, dtype=torch.int32).pin_memory()
     seen_done = torch.zeros(S, dtype=torch.int32).pin_memory()
-    compute, producer, watch = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.Stream()
+    compute = torch.cuda.Stream()
+    producer = stream_beside(compute)
+    watch = stream_beside(compute, producer)
     try:
         assert lib.ms_set_reserved_cus(32) == 0        # the producer's copies and the watcher's need compute units beside the product
         want = signal_tests._plain(flow, src, torch.bfloat16)
