@@ -32,7 +32,7 @@ LARGE = [(1024,) * 3, (2048,) * 3, (3072,) * 3, (4096,) * 3, (5120,) * 3, (6144,
          (8192, 8192, 2048), (2048, 8192, 8192), (4096, 11008, 4096), (16384, 4096, 4096)]
 SMALL = [(1024,) * 3, (1536,) * 3, (2048,) * 3, (2560,) * 3, (3072,) * 3, (2048, 4096, 2048), (2048, 2048, 8192), (1024, 4096, 4096),
          (2048, 1536, 3072), (4096, 1536, 1536)]
-FORCED = (2, 3, 4, 5, 6, 7, 8, 9, 11, 12, 13, 14)
+FORCED = (2, 3, 4, 5, 6, 7, 8, 9, 11, 12, 13, 14, 18, 19)
 SIZES = [512, 768, 1024, 1536, 2048, 2560, 3072, 4096, 5120, 6144, 7168, 8192, 10240, 12288, 16384]
 
 
