@@ -54,8 +54,35 @@ def test_rows_that_overlap_and_odd_bases_are_copied(flow, monkeypatch):
 def test_what_the_ring_bodies_refuse_stays_refused():
     f = TP.SPMD(Mesh(create_device_mesh((1, 2)), ("row", "col")), "wang")
     X, W = _pair("os", 32, 32, 24, torch.bfloat16)       # half-blocks of six contraction elements
-    with pytest.raises(Exception):
+    with pytest.raises(ValueError, match="must be multiples of 8"):
         f.OS()(X, W)
     X, W = _pair("ls", 32, 2 * 2 * 2, 32, torch.bfloat16)      # half-blocks of two output columns
-    with pytest.raises(ValueError):
+    with pytest.raises(ValueError, match="are not 16-byte aligned|must be multiples of"):
         f.LS()(X, W)
+
+
+@pytest.mark.parametrize("flow", ["os", "ls", "rs"])
+@pytest.mark.parametrize("algorithm", ["wang", "cannon"])
+def test_which_products_run_at_once(algorithm, flow, monkeypatch):
+    """All but Cannon's OS do without the bodies of single devices, and operands whose half-blocks do not fit are left to those."""
+    f = getattr(TP.SPMD(Mesh(create_device_mesh((2, 2)), ("row", "col")), algorithm), flow.upper())()
+    X, W = _pair(flow, 64, 64, 64, torch.bfloat16)
+    want = f(X, W)
+
+    class ADevice(Exception):
+        pass
+
+    def body(*a):
+        raise ADevice
+    for name in ("_ring_os", "_ring_ls", "_ring_rs"):
+        monkeypatch.setattr(TP, name, body)
+    if (algorithm, flow) == ("cannon", "os"):
+        with pytest.raises(ADevice):
+            f(X, W)
+    else:
+        assert torch.equal(f(X, W), want)
+    rows = torch.randn(64 * 72, device="cuda").bfloat16().as_strided((64, 64), (40, 1))
+    with pytest.raises(ADevice):
+        f(rows, W)
+    with pytest.raises(ADevice):
+        f(X, rows)
