@@ -388,7 +388,8 @@ int ms_probe_l2_lds_stream(const void *buffer, size_t buffer_bytes, int region_s
  * (256x128, 128x192, 128x128, 64x64, 192x192; split counts as above), 28 the 32x32 tile whose contraction a workgroup's
  * waves share (no split count): fp32 calls then use that tile and bf16 calls the library's choice,
  * as fp32 calls do under 1..14, 18 and 19.  Unknown ids are rejected with MS_ERR_ARG, the others
- * of MS_QUERY_LAST_VARIANT (15 to 17, 26, 27) among them.  The sums over devices have the tiles 2, 4 and 14 and take the library's
+ * of MS_QUERY_LAST_VARIANT (15 to 17, 26, 27) among them.  Operands whose rows lie along the contraction and are more than 64 MB
+ * apart (128 MB in fp32) have one tile of each type, 14 and 24: other forced tiles, and forced splits, are refused for them, and so is 18 beyond 32 MB.  The sums over devices have the tiles 2, 4 and 14 and take the library's
  * choice under every other id. */
 int ms_set_variant(int variant);
 

@@ -17,8 +17,10 @@ by having one GPU and no tracing compiler:
   the running sum in the input dtype, :167);
 * the sliced OS body rejects ``K == 1``: the reference adds slice 0 twice in that case (:163,:172);
   use ``algorithm='collective'`` for the unsliced product;
-* the ring baselines 'wang' and 'cannon' (:34-149, :218-342) drive the same kernels with 2 * size
-  half-block slices in ring order; the hops themselves are host index arithmetic.
+* the ring baselines 'wang' and 'cannon' (:34-149, :218-342): one device's body drives the same kernels with 2 * size
+  half-block slices in ring order, the hops themselves being host index arithmetic.  A global product takes that order only where it
+  shows in the result (OS); the LS and RS bodies hand out Collective's partial sums, and their global products are computed as its are
+  (_RING_BODIES), so timing those does not tell the algorithms apart.
 """
 from __future__ import annotations
 

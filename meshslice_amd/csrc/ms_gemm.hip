@@ -1196,7 +1196,8 @@ MS_API int ms_gemm_os_noalloc(const void *const *A_slices, const void *const *B_
     for (const F32Tile &t : F32_TILES) if (t.id == want.id) { bm = t.bm; bn = t.bn; }
   }
   if (splits <= 1) {
-    // an unsplit product exchanges nothing (without a workspace the library makes the same choice: splits are only ever added)
+    // an unsplit product exchanges nothing (without a workspace the library makes the same choice: splits are only ever added,
+    // and products that SMALL_OS_MAX_K keeps off the 64x64 tile split, all of 200000 drawn ones)
     p.ws = nullptr;
     p.ws_bytes = 0;
     return run(p, stream);

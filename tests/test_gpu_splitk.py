@@ -183,8 +183,8 @@ def test_small_output_long_contraction_is_split_by_default():
 
 
 def test_a_fused_epilogue_keeps_the_product_unsplit():
-    """The fused-epilogue kernels carry no exchange of partial tiles: a product that would split runs unsplit when an
-    epilogue is asked for, and a forced split is refused."""
+    """Of the fused-epilogue kernels only the small tiles' (14 and 18) carry the exchange of partial tiles: a product that would split on a
+    larger tile runs unsplit when an epilogue is asked for, and a forced split there is refused."""
     L = _lib.load()
     A = [_rand((2048, 3072), 1.0, 30 + s) for s in range(4)]
     B = [_rand((3072, 1536), 0.02, 40 + s) for s in range(4)]
