@@ -646,16 +646,26 @@ def _half_blocks_fit(dataflow, X, W, C) -> bool:
     return extent % (2 * C * q) == 0 and C <= 32 and X.stride(0) >= X.shape[1] and W.stride(0) >= W.shape[1]
 
 
+# Bytes of a column's output block from which it is worth 15 us more of the host (a call with ``out=`` is not native) to have it written where it belongs
+# instead of copied there.  2x2 devices, 2048 x 2048 x 2048 69 us with out=, 39 without, 4096 x 4096 x 1024 (32 MB) 69 and 63, 8192 x 8192 x 1024 114 and 212; 1x4, 4096 x 12288 x 512
+# (96 MB) 174 and 138, 8192 x 8192 x 1024 (128 MB) 172 and 225.
+RING_IN_PLACE_BYTES = 20 << 20
+
+
 def _whole_ring_os(X, W, C):
-    """The devices of a mesh column add up the same half-blocks in the same order, so their output blocks are one product: C of them instead of R * C,
-    each written where it belongs.  (The chunks of the ring LS and RS bodies are Collective's partial sums, cut in two.)"""
+    """The devices of a mesh column add up the same half-blocks in the same order, so their output blocks are one product: C of them instead of R * C.
+    (The chunks of the ring LS and RS bodies are Collective's partial sums, cut in two.)"""
     h, n = X.shape[1] // C // 2, W.shape[1] // C
-    halves, rows = X.split(h, 1), W.split(h, 0)
-    Y = torch.empty((X.shape[0], W.shape[1]), dtype=X.dtype, device=X.device)
+    halves, columns = X.split(h, 1), W.split(n, 1)
+    Y = None
+    if C > 1 and X.shape[0] * n * X.element_size() > RING_IN_PLACE_BYTES:
+        Y = torch.empty((X.shape[0], W.shape[1]), dtype=X.dtype, device=X.device)
+    blocks = []
     for j in range(C):
         order = [2 * b + hi for b, hi in _ring_order("wang", "os", 1, C, 0, j)]
-        local_gemm.gemm_os(_usable([halves[x] for x in order]), _usable([rows[x][:, j * n:(j + 1) * n] for x in order]), out=Y[:, j * n:(j + 1) * n])
-    return Y
+        rows = columns[j].split(h, 0)
+        blocks.append(local_gemm.gemm_os(_usable([halves[x] for x in order]), _usable([rows[x] for x in order]), out=None if Y is None else Y[:, j * n:(j + 1) * n]))
+    return Y if Y is not None else torch.cat(blocks, 1) if C > 1 else blocks[0]
 
 
 # (the bodies launched ahead of their gathers keep a product per device where that produces chunks; of the ring bodies only Cannon's OS, whose devices

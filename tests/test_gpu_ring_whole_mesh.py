@@ -86,3 +86,18 @@ def test_which_products_run_at_once(algorithm, flow, monkeypatch):
         f(rows, W)
     with pytest.raises(ADevice):
         f(X, rows)
+
+
+@pytest.mark.parametrize("R,C", [(1, 2), (2, 2), (4, 1), (1, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_column_blocks_are_written_in_place_only_where_they_are_large(R, C, dtype, monkeypatch):
+    """A call with out= costs the host 15 us more: 1x2 devices of small layers took 1.4 of the time device by device with it."""
+    f = TP.SPMD(Mesh(create_device_mesh((R, C)), ("row", "col")), "wang").OS()
+    X, W = _pair("os", 64, 64, 64, dtype)
+    outs, real = [], TP.local_gemm.gemm_os
+    monkeypatch.setattr(TP.local_gemm, "gemm_os", lambda a, b, out=None: (outs.append(out), real(a, b, out=out))[1])
+    copied = f(X, W)
+    assert outs == [None] * C
+    monkeypatch.setattr(TP, "RING_IN_PLACE_BYTES", 0)
+    assert torch.equal(f(X, W), copied) and len(outs) == 2 * C and all((o is None) == (C == 1) for o in outs[C:])
+    assert torch.equal(copied, _device_by_device(f, X, W, monkeypatch))
